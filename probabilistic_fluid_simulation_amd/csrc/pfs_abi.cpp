@@ -6,6 +6,7 @@
 
 #include <atomic>
 #include <climits>
+#include <cmath>
 #include <cstdio>
 #include <deque>
 #include <map>
@@ -120,6 +121,23 @@ int set_error(int code, const std::string &msg) {
 }
 
 void clear_error() { g_last_error.clear(); }
+
+// Proofs are kept per thread for the last few divisors (a step asks for beta
+// and the field's two sides again on every call).
+FixedDiv fixed_div(float d) {
+    struct Entry {
+        float d = 0.0f;
+        FixedDiv f{};
+    };
+    static thread_local Entry memo[8];
+    static thread_local unsigned next = 0;
+    for (const Entry &m : memo)
+        if (m.d == d) return m.f;  // never for NaN; 0 is not asked for
+    Entry &m = memo[next++ & 7u];
+    m.f = prove_fixed_div(d);
+    m.d = d;
+    return m.f;
+}
 
 int check_launch(const char *what) {
     hipError_t e = hipGetLastError();

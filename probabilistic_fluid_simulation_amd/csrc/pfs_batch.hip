@@ -34,6 +34,7 @@
 #include "pfs.h"
 #include "pfs_internal.h"
 #include "pfs_step_kernels.h"
+#include "pfs_wave_kernels.h"
 
 namespace pfs {
 namespace {
@@ -41,12 +42,20 @@ namespace {
 constexpr int kCBX = 64, kCBY = 4;  // dye threads per block: 64 x 4
 constexpr int kCRows = 4;           // pixels per thread, kCBY rows apart: 64 x 16 per block
 
-template <int H, bool LAST, int TS>
-__global__ __launch_bounds__((Geo<H, TS>::NT)) void k_diffuse_batch(
+template <int H, bool LAST>
+__global__ __launch_bounds__((Geo<H, 16>::NT)) void k_diffuse_batch(
     const DiffuseArgs *__restrict__ tab, const int *__restrict__ tile_scene, int ntiles) {
     const int b = xcd_tile(blockIdx.x, ntiles);
     const DiffuseArgs a = tab[tile_scene[b]];
-    diffuse_tile<H, LAST, TS>(a, b - a.tile_base);
+    diffuse_tile<H, LAST, 16>(a, b - a.tile_base);
+}
+
+template <int H, bool FIRST, bool LAST, int S>
+__global__ __launch_bounds__(kWaveMax * 64, S == 2 ? 8 : 6) void k_diffuse_wave_batch(
+    const DiffuseArgs *__restrict__ tab, const int *__restrict__ tile_scene, int ntiles) {
+    const int b = xcd_tile(blockIdx.x, ntiles);
+    const DiffuseArgs a = tab[tile_scene[b]];
+    diffuse_wave<H, FIRST, LAST, S>(a, b - a.tile_base);
 }
 
 template <int H, bool LAST, int TS>
@@ -71,12 +80,27 @@ using PressureBatchFn = void (*)(const PressureArgs *, const int *, int);
 
 #define PFS_H_CASES(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9)
 
-template <int TS>
-DiffuseBatchFn diffuse_batch_for_ts(int H, bool last) {
+DiffuseBatchFn diffuse_small_batch_for(int H, bool last) {
     switch (H) {
 #define PFS_CASE(h) \
     case h:         \
-        return last ? k_diffuse_batch<h, true, TS> : k_diffuse_batch<h, false, TS>;
+        return last ? k_diffuse_batch<h, true> : k_diffuse_batch<h, false>;
+        PFS_H_CASES(PFS_CASE)
+#undef PFS_CASE
+    }
+    return nullptr;
+}
+
+template <int S>
+DiffuseBatchFn diffuse_wave_batch_for(int H, bool first, bool last) {
+    if (!last)
+        return H != kMaxChunk ? nullptr
+                              : first ? k_diffuse_wave_batch<kMaxChunk, true, false, S>
+                                      : k_diffuse_wave_batch<kMaxChunk, false, false, S>;
+    switch (H) {
+#define PFS_CASE(h) \
+    case h:         \
+        return first ? k_diffuse_wave_batch<h, true, true, S> : k_diffuse_wave_batch<h, false, true, S>;
         PFS_H_CASES(PFS_CASE)
 #undef PFS_CASE
     }
@@ -93,11 +117,6 @@ PressureBatchFn pressure_batch_for_ts(int H, bool last) {
 #undef PFS_CASE
     }
     return nullptr;
-}
-
-DiffuseBatchFn diffuse_batch_for(int H, bool last, int ts) {
-    return ts == 16 ? diffuse_batch_for_ts<16>(H, last)
-                    : ts == 32 ? diffuse_batch_for_ts<32>(H, last) : diffuse_batch_for_ts<64>(H, last);
 }
 
 PressureBatchFn pressure_batch_for(int H, bool last, int ts) {
@@ -133,6 +152,11 @@ struct pfs_batch {
         int iters = 0, nchunks = 0, ntiles = 0;
         Chunk plan[kMaxPlan];
         int *tile_scene = nullptr;
+        // The diffusion launches' shapes and tile tables: those of
+        // tile_scene at side 16 (shape {0, 0}), else the chunk's wave tiles.
+        WaveShape shape[kMaxPlan] = {};
+        int dtiles[kMaxPlan] = {};
+        int *dtile_scene[kMaxPlan] = {};
         DiffuseArgs *dtab[kMaxPlan] = {};
         PressureArgs *ptab[2][kMaxPlan] = {};
     };
@@ -249,7 +273,7 @@ struct pfs_batch {
             return off;
         };
         struct Off {
-            size_t tile_scene, dtab[kMaxPlan], ptab[2][kMaxPlan];
+            size_t tile_scene, dtile_scene[kMaxPlan], dtab[kMaxPlan], ptab[2][kMaxPlan];
         };
         std::vector<Off> offs;
         for (auto &kv : by_k) {
@@ -277,6 +301,34 @@ struct pfs_batch {
             o.tile_scene = reserve(tile_scene.size() * sizeof(int));
             std::memcpy(img.data() + o.tile_scene, tile_scene.data(), tile_scene.size() * sizeof(int));
             for (int c = 0; c < g.nchunks; ++c) {
+                const int H = g.plan[c].H;
+                std::vector<int> wave_scene;
+                g.dtiles[c] = g.ntiles;
+                o.dtile_scene[c] = o.tile_scene;
+                if (tile != 16) {
+                    g.shape[c] = wave_shape(H, device_cus(), [&](WaveShape sh) {
+                        long long n = 0;
+                        for (const DiffuseArgs &a : d) n += wave_tiles(a.w, a.h, H, sh);
+                        return n;
+                    });
+                    for (size_t k = 0; k < ids.size(); ++k) {
+                        d[k].tile_base = (int)wave_scene.size();
+                        d[k].tiles_x = wave_tiles_x(d[k].w, H);
+                        d[k].ntiles = (int)wave_tiles(d[k].w, d[k].h, H, g.shape[c]);
+                        wave_scene.insert(wave_scene.end(), d[k].ntiles, (int)k);
+                    }
+                    g.dtiles[c] = (int)wave_scene.size();
+                    // Chunks of one halo share the first one's table.
+                    int same = 0;
+                    while (g.plan[same].H != H) ++same;
+                    if (same == c) {
+                        o.dtile_scene[c] = reserve(wave_scene.size() * sizeof(int));
+                        std::memcpy(img.data() + o.dtile_scene[c], wave_scene.data(),
+                                    wave_scene.size() * sizeof(int));
+                    } else {
+                        o.dtile_scene[c] = o.dtile_scene[same];
+                    }
+                }
                 o.dtab[c] = reserve(d.size() * sizeof(DiffuseArgs));
                 for (size_t k = 0; k < ids.size(); ++k) {
                     DiffuseArgs a = d[k];
@@ -341,6 +393,7 @@ struct pfs_batch {
             Group &g = groups[gi];
             g.tile_scene = reinterpret_cast<int *>(base + offs[gi].tile_scene);
             for (int c = 0; c < g.nchunks; ++c) {
+                g.dtile_scene[c] = reinterpret_cast<int *>(base + offs[gi].dtile_scene[c]);
                 g.dtab[c] = reinterpret_cast<DiffuseArgs *>(base + offs[gi].dtab[c]);
                 for (int q = 0; q < 2; ++q)
                     g.ptab[q][c] = reinterpret_cast<PressureArgs *>(base + offs[gi].ptab[q][c]);
@@ -354,14 +407,24 @@ struct pfs_batch {
         return PFS_OK;
     }
 
+    // Chunk c of the diffusion of group g's scenes.
+    int launch_diffuse(const Group &g, int c) {
+        const Chunk &k = g.plan[c];
+        const WaveShape &sh = g.shape[c];
+        DiffuseBatchFn fn = sh.S == 0   ? diffuse_small_batch_for(k.H, k.last)
+                            : sh.S == 2 ? diffuse_wave_batch_for<2>(k.H, k.first, k.last)
+                                        : diffuse_wave_batch_for<4>(k.H, k.first, k.last);
+        const int threads = sh.S == 0 ? threads_for(k.H, tile) : 64 * sh.nw;
+        hipLaunchKernelGGL(fn, dim3(g.dtiles[c]), dim3(threads), 0, stream, g.dtab[c],
+                           g.dtile_scene[c], g.dtiles[c]);
+        return check_launch("batched diffuse");
+    }
+
     // One timestep of every scene, with the tables of parity q.
     int enqueue_step(int q) {
         for (const Group &g : groups) {
             for (int c = 0; c < g.nchunks; ++c) {
-                hipLaunchKernelGGL(diffuse_batch_for(g.plan[c].H, g.plan[c].last, tile),
-                                   dim3(g.ntiles), dim3(threads_for(g.plan[c].H, tile)), 0, stream,
-                                   g.dtab[c], g.tile_scene, g.ntiles);
-                PFS_TRY(check_launch("batched diffuse"));
+                PFS_TRY(launch_diffuse(g, c));
             }
             for (int c = 0; c < g.nchunks; ++c) {
                 hipLaunchKernelGGL(pressure_batch_for(g.plan[c].H, g.plan[c].last, tile),
@@ -416,10 +479,7 @@ struct pfs_batch {
             bool joined = k == 0 || nblocks == 0;
             for (const Group &g : groups) {
                 for (int c = 0; c < g.nchunks; ++c) {
-                    hipLaunchKernelGGL(diffuse_batch_for(g.plan[c].H, g.plan[c].last, tile),
-                                       dim3(g.ntiles), dim3(threads_for(g.plan[c].H, tile)), 0,
-                                       stream, g.dtab[c], g.tile_scene, g.ntiles);
-                    PFS_TRY(check_launch("batched diffuse"));
+                    PFS_TRY(launch_diffuse(g, c));
                 }
                 if (!joined) {
                     PFS_HIP_TRY(hipStreamWaitEvent(stream, join_ev[k - 1], 0));

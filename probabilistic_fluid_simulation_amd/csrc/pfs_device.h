@@ -8,6 +8,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "pfs_fixed_div.h"
+
 namespace pfs {
 
 // IEEE fmod in the field's precision (fmodf for float, as the reference's
@@ -34,6 +36,17 @@ __device__ __forceinline__ T wrap_coord(T x, T n) {
 template <typename T>
 __device__ __forceinline__ T div_n(T x, T n, T inv_n, bool n_pow2) {
     return n_pow2 ? x * inv_n : x / n;
+}
+
+__device__ __forceinline__ float div_fast2(float x, const FixedDiv &d) {
+    return fmaf(x, d.hi, x * d.lo);
+}
+// A back-trace's displacement x / n.  x needs no range test: below 2^-96,
+// where x*lo may round as a subnormal, the quotient only ever meets a cell
+// coordinate (0 or at least 1) in a subtraction and the wrap's addition of n,
+// neither of which it can change.
+__device__ __forceinline__ float div_const(float x, float n, const FixedDiv &d) {
+    return d.ok ? div_fast2(x, d) : x / n;
 }
 
 // Bilinear blend in the reference's exact order (src/fluid.cpp:62-66).
@@ -91,25 +104,12 @@ __device__ __forceinline__ bool div_fast_ok(float x) {
     const float ax = fabsf(x);
     return ax >= 0x1p-96f && ax < 0x1p96f;  // false for 0, tiny, huge, Inf, NaN
 }
-// Biased exponent of x: div_fast_ok(x) <=> kDivExpLo <= float_exp(x) <= kDivExpHi.
-// Lets a loop track min/max exponents branch-free and test the range once.
-constexpr unsigned kDivExpLo = 127 - 96, kDivExpHi = 127 + 95;
-__device__ __forceinline__ unsigned float_exp(float x) {
-    return (__float_as_uint(x) >> 23) & 0xffu;
-}
 // One Markstein step: q + (x - q*beta)*y, each term rounded once.
 __device__ __forceinline__ float div_step(float q, float x, float beta, float y) {
     return fmaf(fmaf(-q, beta, x), y, q);
 }
 __device__ __forceinline__ float div_fast(float x, float beta, float y) {
     return div_step(div_step(x * y, x, beta, y), x, beta, y);
-}
-// When the host has checked |y*beta - 1| <= 2^-26 (exact in double), then
-// |x*y - x/beta| < ulp(x/beta)/4 for every x, so q0 = RN(x*y) is already
-// faithful and one Markstein step rounds correctly: 3 operations instead
-// of 5 (same range conditions on x).
-__device__ __forceinline__ float div_fast3(float x, float beta, float y) {
-    return div_step(x * y, x, beta, y);
 }
 __device__ __forceinline__ float div_fixed(float x, float beta, float y, bool fast) {
     return (fast && div_fast_ok(x)) ? div_fast(x, beta, y) : x / beta;

@@ -39,6 +39,9 @@ struct Pow2 {
     explicit Pow2(int n) : inv(1.0f / (float)n), is(n > 0 && (n & (n - 1)) == 0) {}
 };
 
+// prove_fixed_div (pfs_fixed_div.h), remembered per thread for a few divisors.
+FixedDiv fixed_div(float d);
+
 // Host-side constants of advect_color, computed in float exactly as
 // src/fluid.cpp:78-83,97-98 computes them.
 ColorArgs color_args(const float *img, float *out, const float *vp, int iw, int ih, int ic, int vw,

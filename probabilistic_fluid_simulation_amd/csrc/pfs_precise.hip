@@ -65,6 +65,7 @@
 #include "pfs.h"
 #include "pfs_internal.h"
 #include "pfs_step_kernels.h"
+#include "pfs_wave_kernels.h"
 
 namespace pfs {
 namespace {
@@ -249,8 +250,6 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// ctl non-null (the step's first launch): workgroup 0 also clears the
-// control block the pressure launches use.
 // x plus the value DPP control CTRL moves into this lane (0 where it moves
 // none), on the two 32-bit halves of a double.
 template <int CTRL, int ROWS>
@@ -274,18 +273,30 @@ __device__ __forceinline__ double wave_scan_dpp(double x) {
     return x;
 }
 
-template <int H, bool LAST, int TS>
-__global__ __launch_bounds__((Geo<H, TS>::NT)) void k_diffuse_precise(DiffuseArgs a, PCtl *ctl) {
-    if (ctl && blockIdx.x == 0) {
-        for (int k = threadIdx.x; k < kMaxLaunch; k += blockDim.x) ctl->count[k] = 0u;
-        for (int k = threadIdx.x; k < kNRows; k += blockDim.x) ctl->total[k] = 0.0;
-        if (threadIdx.x == 0) {
-            ctl->done = 0;
-            ctl->stop = -1;
-            ctl->kp = 0;
-        }
+// ctl non-null (the step's first launch): workgroup 0 also clears the
+// control block the pressure launches use.
+__device__ __forceinline__ void clear_ctl(PCtl *ctl) {
+    if (!ctl || blockIdx.x != 0) return;
+    for (int k = threadIdx.x; k < kMaxLaunch; k += blockDim.x) ctl->count[k] = 0u;
+    for (int k = threadIdx.x; k < kNRows; k += blockDim.x) ctl->total[k] = 0.0;
+    if (threadIdx.x == 0) {
+        ctl->done = 0;
+        ctl->stop = -1;
+        ctl->kp = 0;
     }
-    diffuse_tile<H, LAST, TS, true>(a, xcd_tile(blockIdx.x, a.ntiles));
+}
+
+template <int H, bool LAST>
+__global__ __launch_bounds__((Geo<H, 16>::NT)) void k_diffuse_precise(DiffuseArgs a, PCtl *ctl) {
+    clear_ctl(ctl);
+    diffuse_tile<H, LAST, 16, true>(a, xcd_tile(blockIdx.x, a.ntiles));
+}
+
+template <int H, bool FIRST, bool LAST, int S>
+__global__ __launch_bounds__(kWaveMax * 64, S == 2 ? 8 : 6) void k_diffuse_wave_precise(DiffuseArgs a,
+                                                                                      PCtl *ctl) {
+    clear_ctl(ctl);
+    diffuse_wave<H, FIRST, LAST, S, true>(a, xcd_tile(blockIdx.x, a.ntiles));
 }
 
 // Up to C = H - 1 compensated pressure sweeps of one tile, the residual of
@@ -527,14 +538,12 @@ using PressureFn = void (*)(PreciseArgs);
 
 // Diffusion launches: chunks of C = 4 or 8 sweeps (halo C), the last one
 // of 1..C sweeps (halo 2..C+1).
-template <int TS>
-DiffuseFn diffuse_precise_ts(int H, bool last) {
-    if (!last) return H == 4 ? k_diffuse_precise<4, false, TS>
-                             : H == 8 ? k_diffuse_precise<8, false, TS> : nullptr;
+DiffuseFn diffuse_precise_small(int H, bool last) {
+    if (!last) return H == 4 ? k_diffuse_precise<4, false> : H == 8 ? k_diffuse_precise<8, false> : nullptr;
     switch (H) {
 #define PFS_CASE(h) \
     case h:         \
-        return k_diffuse_precise<h, true, TS>;
+        return k_diffuse_precise<h, true>;
         PFS_CASE(2) PFS_CASE(3) PFS_CASE(4) PFS_CASE(5) PFS_CASE(6) PFS_CASE(7) PFS_CASE(8)
         PFS_CASE(9)
 #undef PFS_CASE
@@ -542,9 +551,22 @@ DiffuseFn diffuse_precise_ts(int H, bool last) {
     return nullptr;
 }
 
-DiffuseFn diffuse_precise_for(int H, bool last, int ts) {
-    return ts == 16 ? diffuse_precise_ts<16>(H, last)
-                    : ts == 32 ? diffuse_precise_ts<32>(H, last) : diffuse_precise_ts<64>(H, last);
+template <int S>
+DiffuseFn diffuse_precise_wave(int H, bool first, bool last) {
+    if (!last) {
+        if (H == 4) return first ? k_diffuse_wave_precise<4, true, false, S> : k_diffuse_wave_precise<4, false, false, S>;
+        if (H == 8) return first ? k_diffuse_wave_precise<8, true, false, S> : k_diffuse_wave_precise<8, false, false, S>;
+        return nullptr;
+    }
+    switch (H) {
+#define PFS_CASE(h) \
+    case h:         \
+        return first ? k_diffuse_wave_precise<h, true, true, S> : k_diffuse_wave_precise<h, false, true, S>;
+        PFS_CASE(2) PFS_CASE(3) PFS_CASE(4) PFS_CASE(5) PFS_CASE(6) PFS_CASE(7) PFS_CASE(8)
+        PFS_CASE(9)
+#undef PFS_CASE
+    }
+    return nullptr;
 }
 
 template <int H>
@@ -618,8 +640,21 @@ int precise_step(float *P, float *Q, int w, int h, float dt, float visc, int K, 
     const int nd = chunk_plan(K, plan, kMaxK, C);
     for (int c = 0; c < nd; ++c) {
         diffuse_chunk(d, c, plan[c], wsf);
-        hipLaunchKernelGGL(diffuse_precise_for(plan[c].H, plan[c].last, ts), dim3(d.ntiles),
-                           dim3(threads_precise(plan[c].H, ts)), 0, s, d, c == 0 ? ctl : nullptr);
+        const Chunk &k = plan[c];
+        PCtl *clear = c == 0 ? ctl : nullptr;
+        if (ts == 16) {
+            hipLaunchKernelGGL(diffuse_precise_small(k.H, k.last), dim3(d.ntiles),
+                               dim3(threads_precise(k.H, ts)), 0, s, d, clear);
+        } else {
+            DiffuseArgs wd = d;
+            const WaveShape sh =
+                wave_shape(k.H, device_cus(), [&](WaveShape x) { return wave_tiles(w, h, k.H, x); });
+            wd.tiles_x = wave_tiles_x(w, k.H);
+            wd.ntiles = (int)wave_tiles(w, h, k.H, sh);
+            hipLaunchKernelGGL(sh.S == 2 ? diffuse_precise_wave<2>(k.H, k.first, k.last)
+                                         : diffuse_precise_wave<4>(k.H, k.first, k.last),
+                               dim3(wd.ntiles), dim3(64 * sh.nw), 0, s, wd, clear);
+        }
         PFS_TRY(check_launch("precise diffuse"));
     }
     PreciseArgs pa{};

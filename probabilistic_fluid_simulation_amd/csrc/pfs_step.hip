@@ -10,20 +10,24 @@
 //      of the same cells (:72-127) when one call runs the whole timestep of
 //      the reference driver (src/main.cpp:222-225).
 //
-// Each workgroup owns a TX x TY tile of cells (64, 32 or 16 square: the
-// caller's choice) and stages the tile plus a
-// halo of H = sweeps (+1 for the final stencil) cells, periodic wrap folded
-// into the staged coordinates.  Thread (x, seg) owns column x of the staged
-// region, rows [seg*S, seg*S + S), in registers.  Every sweep it publishes
-// its cells (alpha-scaled for diffusion) to an LDS plane, waits at one
-// barrier (planes alternate), and updates its cells from the left/right
-// columns in LDS and its own registers above and below.  Cells of the outer
-// ring read clamped neighbours and become garbage; that ring grows by one
-// cell per sweep exactly as the valid region shrinks, so the tile is never
-// touched by it.  Halo cells are recomputed by both neighbouring tiles with
-// the same operations in the same order: every value is bit-identical to the
-// reference's global sweep.  For K > 8 the sweeps run in chunks of 8 with the
-// iterate in workspace planes between chunks.
+// Each workgroup owns a tile of cells and stages it plus a halo of H = sweeps
+// (+1 for the final stencil) cells, periodic wrap folded into the staged
+// coordinates.  Two forms:
+//   - square tiles (64, 32 or 16 wide: kernel P, and kernel D at side 16;
+//     pfs_step_kernels.h): thread (x, seg) owns column x of the staged region,
+//     rows [seg*S, seg*S + S), in registers; every sweep it publishes its cells
+//     (alpha-scaled for diffusion) to an LDS plane, waits at one barrier
+//     (planes alternate), and updates its cells from the left/right columns in
+//     LDS and its own registers above and below;
+//   - wave tiles (kernel D on every field past side 16; pfs_wave_kernels.h):
+//     a wavefront owns whole rows and takes its horizontal neighbours by DPP.
+// Cells of the outer ring read clamped or missing neighbours and become
+// garbage; that ring grows by one cell per sweep exactly as the valid region
+// shrinks, so the tile is never touched by it.  Halo cells are recomputed by
+// both neighbouring tiles with the same operations in the same order: every
+// value is bit-identical to the reference's global sweep.  For K > 8 the
+// sweeps run in chunks of 8 with the iterate in workspace planes between
+// chunks.
 //
 // Buffer contract (equal to fluid.cpp's, derived from its pointer swaps):
 // with P = vp and Q = tmp at entry, E = D^K if K is even else D^(K-1),
@@ -38,14 +42,22 @@
 
 #include "pfs_internal.h"
 #include "pfs_step_kernels.h"
+#include "pfs_wave_kernels.h"
 
 namespace pfs {
 
 namespace {
 
-template <int H, bool LAST, int TS>
-__global__ __launch_bounds__((Geo<H, TS>::NT)) void k_diffuse(DiffuseArgs a) {
-    diffuse_tile<H, LAST, TS>(a, xcd_tile(blockIdx.x, a.ntiles));
+// Side 16 (small fields).
+template <int H, bool LAST>
+__global__ __launch_bounds__((Geo<H, 16>::NT)) void k_diffuse(DiffuseArgs a) {
+    diffuse_tile<H, LAST, 16>(a, xcd_tile(blockIdx.x, a.ntiles));
+}
+
+// Larger fields.
+template <int H, bool FIRST, bool LAST, int S>
+__global__ __launch_bounds__(kWaveMax * 64, S == 2 ? 8 : 6) void k_diffuse_wave(DiffuseArgs a) {
+    diffuse_wave<H, FIRST, LAST, S>(a, xcd_tile(blockIdx.x, a.ntiles));
 }
 
 template <int H, bool LAST, int TS>
@@ -59,12 +71,28 @@ using PressureFn = void (*)(PressureArgs);
 
 #define PFS_H_CASES(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9)
 
-template <int TS>
-DiffuseFn diffuse_for_ts(int H, bool last) {
+DiffuseFn diffuse_small_for(int H, bool last) {
     switch (H) {
 #define PFS_CASE(h) \
     case h:         \
-        return last ? k_diffuse<h, true, TS> : k_diffuse<h, false, TS>;
+        return last ? k_diffuse<h, true> : k_diffuse<h, false>;
+        PFS_H_CASES(PFS_CASE)
+#undef PFS_CASE
+    }
+    return nullptr;
+}
+
+// A chunk that is not the last runs kMaxChunk sweeps.
+template <int S>
+DiffuseFn diffuse_wave_for(int H, bool first, bool last) {
+    if (!last)
+        return H != kMaxChunk ? nullptr
+                              : first ? k_diffuse_wave<kMaxChunk, true, false, S>
+                                      : k_diffuse_wave<kMaxChunk, false, false, S>;
+    switch (H) {
+#define PFS_CASE(h) \
+    case h:         \
+        return first ? k_diffuse_wave<h, true, true, S> : k_diffuse_wave<h, false, true, S>;
         PFS_H_CASES(PFS_CASE)
 #undef PFS_CASE
     }
@@ -83,11 +111,6 @@ PressureFn pressure_for_ts(int H, bool last) {
     return nullptr;
 }
 
-DiffuseFn diffuse_for(int H, bool last, int ts) {
-    return ts == 16 ? diffuse_for_ts<16>(H, last)
-                    : ts == 32 ? diffuse_for_ts<32>(H, last) : diffuse_for_ts<64>(H, last);
-}
-
 PressureFn pressure_for(int H, bool last, int ts) {
     return ts == 16 ? pressure_for_ts<16>(H, last)
                     : ts == 32 ? pressure_for_ts<32>(H, last) : pressure_for_ts<64>(H, last);
@@ -103,6 +126,15 @@ int threads_for_ts(int H) {
 #undef PFS_CASE
     }
     return 0;
+}
+
+// The wave shape of one field's launch with halo H; sets d's tile counts to it.
+WaveShape wave_args(DiffuseArgs &d, int H) {
+    const WaveShape sh =
+        wave_shape(H, device_cus(), [&](WaveShape s) { return wave_tiles(d.w, d.h, H, s); });
+    d.tiles_x = wave_tiles_x(d.w, H);
+    d.ntiles = (int)wave_tiles(d.w, d.h, H, sh);
+    return sh;
 }
 
 }  // namespace
@@ -131,8 +163,17 @@ int fused_step(const StepArgs &s, float *ws, hipStream_t stream, hipEvent_t *ev,
     for (int r = 0; r < reps; ++r)
         for (int c = 0; c < nchunks; ++c) {
             diffuse_chunk(d, c, plan[c], ws);
-            hipLaunchKernelGGL(diffuse_for(plan[c].H, plan[c].last, s.tile), grid,
-                               dim3(threads_for(plan[c].H, s.tile)), 0, stream, d);
+            const Chunk &k = plan[c];
+            if (s.tile == 16) {
+                hipLaunchKernelGGL(diffuse_small_for(k.H, k.last), grid,
+                                   dim3(threads_for(k.H, s.tile)), 0, stream, d);
+            } else {
+                DiffuseArgs w = d;
+                const WaveShape sh = wave_args(w, k.H);
+                hipLaunchKernelGGL(sh.S == 2 ? diffuse_wave_for<2>(k.H, k.first, k.last)
+                                             : diffuse_wave_for<4>(k.H, k.first, k.last),
+                                   dim3(w.ntiles), dim3(64 * sh.nw), 0, stream, w);
+            }
             PFS_TRY(check_launch("fused diffuse"));
         }
     if (ev) PFS_HIP_TRY(hipEventRecord(ev[1], stream));

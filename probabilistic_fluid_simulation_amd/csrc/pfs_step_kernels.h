@@ -4,7 +4,7 @@
 // pfs_step.hip.
 #pragma once
 
-#include "pfs_device.h"
+#include "pfs_internal.h"
 
 namespace pfs {
 
@@ -51,10 +51,10 @@ constexpr int wgs_per_cu(int lds, int threads) {
 
 // Workgroups are dispatched round-robin over the 8 XCDs (workgroup b runs on
 // XCD b % 8).  Remap so that each XCD owns a contiguous band of tiles and the
-// halos its tiles share stay in that XCD's L2.
+// halos its tiles share stay in that XCD's L2.  A bijection on [0, n).
 __device__ __forceinline__ int xcd_tile(int b, int n) {
-    if ((n & 7) != 0) return b;
-    return (b & 7) * (n >> 3) + (b >> 3);
+    const int q = n >> 3, r = n & 7, x = b & 7;
+    return x * q + min(x, r) + (b >> 3);
 }
 
 __device__ __forceinline__ int wrap_index(int g, int n) {
@@ -73,7 +73,8 @@ struct DiffuseArgs {
     float dt, fw, fh, inv_w, inv_h;
     int pow2_w, pow2_h;
     float alpha, beta, rcp_beta, gamma;
-    int fast_div;  // 0: IEEE division; 1: 5-op exact division; 2: 3-op exact division
+    int fast_div;  // division by beta: 0 IEEE, 1 five operations, 2 two (proven for it)
+    FixedDiv db, dw, dh;  // beta, w and h as fixed divisors
     int first, k_even;
     int tile_base;  // first tile of this scene in a batched launch
 };
@@ -91,6 +92,7 @@ struct PressureArgs {
     int w, h, tiles_x, ntiles;
     float dt, fw, fh, inv_w, inv_h;
     int pow2_w, pow2_h;
+    FixedDiv dw, dh;       // w and h as fixed divisors
     float dt_viw, dt_vih;  // dt / (field/image width ratio), as src/fluid.cpp:97-98
     int first;
     int tile_base;  // first tile of this scene in a batched launch
@@ -184,14 +186,63 @@ __device__ __forceinline__ void pressure_sum_comp(float l, float r, float t, flo
     s = u;
 }
 
+// min over the bit patterns read as unsigned: of x and x - n it picks the one
+// in [0, n) for x in [0, 2n), a negative number having the larger pattern.
+__device__ __forceinline__ float min_bits(float a, float b) {
+    return __uint_as_float(min(__float_as_uint(a), __float_as_uint(b)));
+}
+
+// wrap_coord's value for |x| < n (see there): x + n brought into [0, n) by at
+// most two subtractions of n.
+__device__ __forceinline__ float wrap_near(float x, float n) {
+    float s = x + n;
+    s = min_bits(s, s - n);
+    return min_bits(s, s - n);
+}
+
 // Region coordinate of global index g (0 <= g < n) on an axis whose staged
-// region starts at global coordinate o (periodic), or `lim` when g + 1 is
-// not staged right after it.
-__device__ __forceinline__ int staged(int g, int o, int n, int lim) {
-    int r = g - o;  // in (-n, n + H) for o in [-H, n)
-    if (r < 0) r += n;
-    if (r >= n) r -= n;
-    return r < lim - 1 ? r : lim;
+// region starts at global coordinate o in [-n, n) (periodic), if it is staged;
+// else some value past the region.
+__device__ __forceinline__ unsigned region_of(int g, int o, int n) {
+    const int r = g - o;
+    return min(min((unsigned)r, (unsigned)(r + n)), (unsigned)(r - n));
+}
+
+// The back-trace (src/fluid.cpp:36-61) of cell (fi, fj) with velocity c, as
+// staged corners: (rx, ry) the first corner's coordinates in a staged region
+// of nx x ny cells whose cell (0, 0) is global (ox, oy), `on` whether all four
+// corners are staged.  Traces longer than the field, and all of them where
+// the two-operation division by the field's sides is not proven, are not `on`.
+struct Near {
+    float sx, sy;
+    unsigned rx, ry;
+    bool on;
+};
+__device__ __forceinline__ Near near_trace(const DiffuseArgs &a, float fi, float fj, float2 c, int ox,
+                                           int oy, int nx, int ny) {
+    const float xp = fi - div_fast2(a.dt * c.x, a.dw), yp = fj - div_fast2(a.dt * c.y, a.dh);
+    const float xw = wrap_near(xp, a.fw), yw = wrap_near(yp, a.fh);
+    const int i0 = (int)xw, j0 = (int)yw;
+    Near r;
+    r.sx = xw - (float)i0;
+    r.sy = yw - (float)j0;
+    r.rx = region_of(i0, ox, a.w);
+    r.ry = region_of(j0, oy, a.h);
+    r.on = a.dw.ok && a.dh.ok && fabsf(xp) < a.fw && fabsf(yp) < a.fh && r.rx < (unsigned)nx - 1u &&
+           r.ry < (unsigned)ny - 1u;
+    return r;
+}
+
+// The advected velocity of cell (gi, gj) from memory, for any back-trace.
+__device__ __forceinline__ float2 far_advect(const DiffuseArgs &a, int gi, int gj, float2 c) {
+    const float2 *__restrict__ P2 = reinterpret_cast<const float2 *>(a.P);
+    const float xp = (float)gi - div_const(a.dt * c.x, a.fw, a.dw);
+    const float yp = (float)gj - div_const(a.dt * c.y, a.fh, a.dh);
+    const Trace t = trace(xp, yp, a.w, a.h, a.fw, a.fh);
+    const float2 f00 = P2[2 * (t.j0 * a.w + t.i0)], f10 = P2[2 * (t.j0 * a.w + t.i1)];
+    const float2 f01 = P2[2 * (t.j1 * a.w + t.i0)], f11 = P2[2 * (t.j1 * a.w + t.i1)];
+    return make_float2(bilerp(t.sx, t.sy, f00.x, f10.x, f01.x, f11.x),
+                       bilerp(t.sx, t.sy, f00.y, f10.y, f01.y, f11.y));
 }
 
 // COMP (the precision form): the numerators are compensated
@@ -202,7 +253,10 @@ __device__ __forceinline__ void diffuse_tile(const DiffuseArgs &a, int tile) {
     using G = Geo<H, TS>;
     constexpr int S = G::S, RX = G::RX, RY = G::RY, PL = G::RYP * RX;
     constexpr int NS = H - (LAST ? 1 : 0);  // sweeps in this launch
-    __shared__ float2 plane[2 * PL];
+    // The staged velocities lie from plane 1 on: the region and a ring of one
+    // cell around it, so that no back-trace of less than a cell leaves them.
+    constexpr int VP = RX + 2, VN = (G::RYP + 2) * VP;
+    __shared__ float2 plane[PL + (VN > PL ? VN : PL)];
 
     const Strip<G> st(threadIdx.x, tile, a.tiles_x, a.w, a.h);
     const float2 *__restrict__ P2 = reinterpret_cast<const float2 *>(a.P);  // (u,v) at 2*cell
@@ -216,35 +270,39 @@ __device__ __forceinline__ void diffuse_tile(const DiffuseArgs &a, int tile) {
     }
     float u[S], v[S];
     if (a.first) {
-        // Advect every strip cell (src/fluid.cpp:36-67) with its corners
-        // from the staged velocities in LDS plane 1 — or from memory when a
-        // back-trace leaves the staged region.
-        float2 *V = plane + PL;
+        // Advect every strip cell (src/fluid.cpp:36-67) with its corners from
+        // the staged velocities; a trace that near_trace does not take is
+        // redone from memory.
+        float2 *V = plane + PL + VP + 1;  // region cell (0, 0)
+        for (int e = threadIdx.x; e < 2 * (VP + RY); e += blockDim.x) {  // the ring
+            const int m = e - 2 * VP;
+            const int ry = m >= 0 ? (m >> 1) : (e < VP ? -1 : RY);
+            const int rx = m >= 0 ? ((m & 1) ? RX : -1) : (e < VP ? e : e - VP) - 1;
+            V[ry * VP + rx] = P2[2 * (wrap_index(st.y0 + ry, a.h) * a.w + wrap_index(st.x0 + rx, a.w))];
+        }
 #pragma unroll
         for (int k = 0; k < S; ++k)
-            if (st.active) V[(st.r0 + k) * RX + st.x] = c[k];
+            if (st.row_ok(k)) V[(st.r0 + k) * VP + st.x] = c[k];
         __syncthreads();
+        bool off[S], any_off = false;
 #pragma unroll
         for (int k = 0; k < S; ++k) {
-            const float xp = (float)st.gi - div_n(a.dt * c[k].x, a.fw, a.inv_w, a.pow2_w);
-            const float yp = (float)st.gj[k] - div_n(a.dt * c[k].y, a.fh, a.inv_h, a.pow2_h);
-            const Trace t = trace(xp, yp, a.w, a.h, a.fw, a.fh);
-            const int rx = staged(t.i0, st.x0, a.w, RX), ry = staged(t.j0, st.y0, a.h, RY);
-            float2 f00, f10, f01, f11;
-            if (rx < RX && ry < RY) {
-                const int o = ry * RX + rx;
-                f00 = V[o];
-                f10 = V[o + 1];
-                f01 = V[o + RX];
-                f11 = V[o + RX + 1];
-            } else {
-                f00 = P2[2 * (t.j0 * a.w + t.i0)];
-                f10 = P2[2 * (t.j0 * a.w + t.i1)];
-                f01 = P2[2 * (t.j1 * a.w + t.i0)];
-                f11 = P2[2 * (t.j1 * a.w + t.i1)];
-            }
-            u[k] = bilerp(t.sx, t.sy, f00.x, f10.x, f01.x, f11.x);
-            v[k] = bilerp(t.sx, t.sy, f00.y, f10.y, f01.y, f11.y);
+            const Near r = near_trace(a, (float)st.gi, (float)st.gj[k], c[k], st.x0 - 1, st.y0 - 1, VP, RY + 2);
+            off[k] = !r.on;
+            any_off = any_off || off[k];
+            const float2 *F = plane + PL + (r.on ? r.ry * VP + r.rx : 0u);
+            const float2 f00 = F[0], f10 = F[1], f01 = F[VP], f11 = F[VP + 1];
+            u[k] = bilerp(r.sx, r.sy, f00.x, f10.x, f01.x, f11.x);
+            v[k] = bilerp(r.sx, r.sy, f00.y, f10.y, f01.y, f11.y);
+        }
+        if (__any(any_off)) {
+#pragma unroll
+            for (int k = 0; k < S; ++k)
+                if (off[k]) {
+                    const float2 n = far_advect(a, st.gi, st.gj[k], c[k]);
+                    u[k] = n.x;
+                    v[k] = n.y;
+                }
         }
     } else {
 #pragma unroll
@@ -270,7 +328,7 @@ __device__ __forceinline__ void diffuse_tile(const DiffuseArgs &a, int tile) {
     // out = (a*L + a*R + a*T + a*B + 1*C) / beta, left to right.  Sweep s
     // publishes alpha-scaled cells into plane (s+1)&1: sweep 1 uses plane 0
     // while plane 1 may still be read by the advection above.  The division
-    // takes an exactly rounded FMA path (3 or 5 operations); if any numerator
+    // takes an exactly rounded FMA path (2 or 5 operations); if any numerator
     // of the strip is outside that path's range (zero, tiny, huge, Inf) the
     // strip divides per element instead (IEEE division where needed).  Rows
     // past RY are padding: computed, never used.
@@ -292,7 +350,6 @@ __device__ __forceinline__ void diffuse_tile(const DiffuseArgs &a, int tile) {
         const float2 *Bl = B + st.r0 * RX + st.xl, *Br = B + st.r0 * RX + st.xr;
         float nu[S], nv[S];
         float lo = 0x1p127f, hi = 0.0f;  // magnitude range of the numerators
-        const bool short_div = a.fast_div == 2;
 #pragma unroll
         for (int k = 0; k < S; ++k) {
             if (LAST && s == NS) {
@@ -313,23 +370,19 @@ __device__ __forceinline__ void diffuse_tile(const DiffuseArgs &a, int tile) {
             lo = fminf(lo, fminf(fabsf(nu[k]), fabsf(nv[k])));
             hi = fmaxf(hi, fmaxf(fabsf(nu[k]), fabsf(nv[k])));
         }
-        // The range is tested before dividing, in the block that made the
-        // numerators (the compiler then keeps min3/max3 on them).
-        // div_fast is div_fast3 followed by one more Markstein step: the
-        // step is applied in place, so both forms leave the quotients in the
-        // same registers (no copies on the 3-operation path).
-        if (fast && lo >= 0x1p-96f && hi < 0x1p96f) {
+        // The range is tested before dividing.  The two-operation division
+        // has no upper limit.
+        if (a.fast_div == 2 && lo >= 0x1p-96f) {
 #pragma unroll
             for (int k = 0; k < S; ++k) {
-                u[k] = div_fast3(nu[k], a.beta, a.rcp_beta);
-                v[k] = div_fast3(nv[k], a.beta, a.rcp_beta);
+                u[k] = div_fast2(nu[k], a.db);
+                v[k] = div_fast2(nv[k], a.db);
             }
-            if (!short_div) {
+        } else if (fast && lo >= 0x1p-96f && hi < 0x1p96f) {
 #pragma unroll
-                for (int k = 0; k < S; ++k) {
-                    u[k] = div_step(u[k], nu[k], a.beta, a.rcp_beta);
-                    v[k] = div_step(v[k], nv[k], a.beta, a.rcp_beta);
-                }
+            for (int k = 0; k < S; ++k) {
+                u[k] = div_fast(nu[k], a.beta, a.rcp_beta);
+                v[k] = div_fast(nv[k], a.beta, a.rcp_beta);
             }
         } else {
 #pragma unroll
@@ -556,11 +609,15 @@ inline DiffuseArgs diffuse_args(const float *P, const float *Q, int w, int h, fl
     d.alpha = visc * dt;
     d.beta = (float)(1.0 + 4.0 * (double)d.alpha);
     d.rcp_beta = 1.0f / d.beta;
-    d.fast_div = 0;
-    if (d.beta >= 0x1p-20f && d.beta <= 0x1p20f) {  // false for NaN
-        // y*beta is exact in double (24 x 24 bits).
-        const double e = (double)d.rcp_beta * (double)d.beta - 1.0;
-        d.fast_div = (e <= 0x1p-26 && e >= -0x1p-26) ? 2 : 1;
+    d.fast_div = d.beta >= 0x1p-20f && d.beta <= 0x1p20f;  // false for NaN
+    d.dw = fixed_div(d.fw);
+    d.dh = fixed_div(d.fh);
+    d.db = FixedDiv{};
+    if (d.beta >= 1.0f && d.beta <= 64.0f) {
+        // Numerators of at least 2^-96 then keep x*lo and the quotient far
+        // enough above the subnormals.
+        d.db = fixed_div(d.beta);
+        if (d.db.ok) d.fast_div = 2;
     }
     d.gamma = (float)(-1.0 / (double)dt);  // src/fluid.cpp:218
     d.k_even = (iters % 2) == 0;
@@ -599,6 +656,8 @@ inline PressureArgs pressure_args(float *P, float *Q, const float *image, float 
     p.inv_h = 1.0f / (float)h;
     p.pow2_w = (w & (w - 1)) == 0;
     p.pow2_h = (h & (h - 1)) == 0;
+    p.dw = fixed_div(p.fw);
+    p.dh = fixed_div(p.fh);
     // src/fluid.cpp:82-83,97-98 with the image the size of the field.
     const float viw = (float)w / (float)w, vih = (float)h / (float)h;
     p.dt_viw = dt / viw;

@@ -234,6 +234,29 @@ def test_every_tile_side_bitexact(orc, shape, k, tile):
     assert_bitexact(gpu_run(s, 3, combined=True), oracle_run(orc, s, 3))
 
 
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 17, 24])
+@pytest.mark.parametrize("shape", [(1201, 803), (331, 403)])
+def test_wave_tiles_bitexact(orc, shape, k):
+    """The large fields' diffusion kernel in both of its strip heights (4 and
+    2 rows per wavefront), every sweep count of a first, middle and last
+    chunk, on odd fields with partial tiles; back-traces of several cells."""
+    s = scenes.random_scene(*shape, *shape, seed=70 + k, dt=0.5, visc=0.15, iters=k,
+                            vel_scale=30.0 if k % 3 else 4000.0)
+    assert_bitexact(gpu_run(s, 1, combined=True), oracle_run(orc, s, 1))
+
+
+@pytest.mark.parametrize("visc", [0.0, 0.1, 0.113, 2.5, 40.0, 1e9, -0.4])
+def test_wave_tiles_every_division(orc, visc):
+    """Every form of the sweep's division: two operations (proven divisors),
+    five (a divisor of the proof's few exceptions, or past its range), IEEE
+    (past the fast range); and numerators below the fast range (tiny
+    velocities) redone one by one."""
+    s = scenes.random_scene(331, 403, 331, 403, seed=5, dt=1.0, visc=visc, iters=5, vel_scale=3.0)
+    s.vp[100:200, :, :2] *= np.float32(1e-30)
+    s.vp[150:180, 50:90, :2] = 0.0
+    assert_bitexact(gpu_run(s, 1, combined=True), oracle_run(orc, s, 1))
+
+
 def test_autotune_records_side_and_keeps_buffers(orc):
     """autotune_step times every side on scratch copies: the buffers are
     unchanged, the fastest side is recorded for the shape, and steps of the
