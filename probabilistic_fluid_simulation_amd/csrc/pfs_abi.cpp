@@ -28,17 +28,31 @@ std::atomic<int> g_step_path{PFS_PATH_AUTO};  // process-wide settings, read by 
 // One growable workspace per (device, stream): calls on one stream are
 // ordered, so they can share it; calls on different streams must not.
 struct Workspace {
+    std::mutex m;
     float *ptr = nullptr;
     size_t bytes = 0;
 };
-std::mutex g_ws_mutex;
+std::mutex g_ws_mutex;  // of the map
 std::map<std::pair<int, hipStream_t>, Workspace> g_ws;
 
-int get_workspace(size_t bytes, hipStream_t s, float **out) {
+// A stream's workspace, held while the launches that use it are queued: two
+// threads on one stream then queue theirs one after the other, and neither
+// regrows the block between the other's look-up and its launches.
+struct Lease {
+    std::unique_lock<std::mutex> held;
+    float *ptr = nullptr;
+};
+
+int get_workspace(size_t bytes, hipStream_t s, Lease *out) {
     int dev = 0;
     PFS_HIP_TRY(hipGetDevice(&dev));
-    std::lock_guard<std::mutex> lock(g_ws_mutex);
-    Workspace &w = g_ws[{dev, s}];
+    Workspace *entry;
+    {
+        std::lock_guard<std::mutex> lock(g_ws_mutex);
+        entry = &g_ws[{dev, s}];  // entries stay where they are
+    }
+    std::unique_lock<std::mutex> held(entry->m);
+    Workspace &w = *entry;
     if (w.bytes < bytes) {
         if (w.ptr) {
             // Work already queued on this stream may still use the old block.
@@ -56,8 +70,32 @@ int get_workspace(size_t bytes, hipStream_t s, float **out) {
         w.ptr = static_cast<float *>(p);
         w.bytes = bytes;
     }
-    *out = w.ptr;
+    out->held = std::move(held);
+    out->ptr = w.ptr;
     return PFS_OK;
+}
+
+// The workspace of an operator's fused sweeps; false where the one-launch-
+// per-sweep form is to run instead: a stream that is being captured (that form
+// allocates nothing and leaves no address in the graph), no memory, or the
+// per-operator path asked for.  The allocation is made with the thread's
+// capture checks relaxed: a capture on another stream goes on undisturbed.
+bool op_workspace(const pfs_field *a, const pfs_field *b, int iters, hipStream_t s, Lease *out) {
+    if (g_step_path != PFS_PATH_AUTO || iters < kOpMinIters || a->z != 4 ||
+        (uintptr_t)a->data % 16 != 0 || (uintptr_t)b->data % 16 != 0)
+        return false;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (st != hipStreamCaptureStatusNone) return false;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    const bool ok = get_workspace(fused_workspace_bytes(a->x, a->y), s, out) == PFS_OK;
+    if (!ok) clear_error();
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return ok;
 }
 
 bool same_shape(const pfs_field *a, const pfs_field *b) {
@@ -197,6 +235,13 @@ int pfs_diffuse(pfs_field *vp, pfs_field *vp_out, float viscosity, float dt, int
     if (!same_shape(vp, vp_out)) return set_error(PFS_ERR_INVALID, "vp_out shape != vp shape");
     if (vp->data == vp_out->data) return set_error(PFS_ERR_INVALID, "vp and vp_out alias");
     if (iters < 0) return set_error(PFS_ERR_INVALID, "iters < 0");
+    if (Lease ws; op_workspace(vp, vp_out, iters, (hipStream_t)stream, &ws)) {
+        // K - 1 swaps (src/fluid.cpp:188-194) leave the structs exchanged for
+        // even K; the last sweep writes what is then vp_out.
+        if (iters % 2 == 0) std::swap(vp->data, vp_out->data);
+        return diffuse_op(iters % 2 == 0 ? vp_out->data : vp->data, vp_out->data, vp->data, vp->x,
+                          vp->y, dt, viscosity, iters, ws.ptr, (hipStream_t)stream);
+    }
     const float alpha = diffuse_alpha(viscosity, dt);
     const float beta = diffuse_beta(alpha);
     for (int it = 0; it < iters; ++it) {
@@ -229,6 +274,11 @@ int pfs_compute_pressure(pfs_field *vp, pfs_field *vp_out, float dt, int iters, 
     if (vp->data == vp_out->data) return set_error(PFS_ERR_INVALID, "vp and vp_out alias");
     if (iters < 0) return set_error(PFS_ERR_INVALID, "iters < 0");
     hipStream_t s = (hipStream_t)stream;
+    if (Lease ws; op_workspace(vp, vp_out, iters, s, &ws)) {
+        if (iters % 2 == 0) std::swap(vp->data, vp_out->data);  // as in pfs_diffuse
+        return pressure_op(iters % 2 == 0 ? vp_out->data : vp->data, vp_out->data, vp->data, vp->x,
+                           vp->y, dt, iters, ws.ptr, s);
+    }
     PFS_TRY(launch_divergence(vp->data, vp_out->data, vp->x, vp->y, vp->z, pressure_gamma(dt), s));
     for (int it = 0; it < iters; ++it) {
         PFS_TRY(launch_pressure_sweep(vp->data, vp_out->data, vp->x, vp->y, vp->z, s));
@@ -307,6 +357,7 @@ static int timestep(pfs_field *vp, pfs_field *tmp, pfs_field *image, pfs_field *
     // (i, j): same size, 4 channels, float4-aligned.
     const bool dye_fused = image && image->x == vp->x && image->y == vp->y && image->z == 4 &&
                            aligned16(image->data) && aligned16(itmp->data);
+    Lease lease;
     float *ws = ws_given;
     if (ws_given) {
         const size_t need = scene_ws_floats(vp->x, vp->y, iters) * sizeof(float);
@@ -317,7 +368,8 @@ static int timestep(pfs_field *vp, pfs_field *tmp, pfs_field *image, pfs_field *
                                  std::to_string(need) + " bytes of step scratch; the " +
                                  "no-allocation entry point holds " + std::to_string(ws_cap));
     } else {
-        PFS_TRY(get_workspace(fused_workspace_bytes(vp->x, vp->y), (hipStream_t)stream, &ws));
+        PFS_TRY(get_workspace(fused_workspace_bytes(vp->x, vp->y), (hipStream_t)stream, &lease));
+        ws = lease.ptr;
     }
     StepArgs a{vp->data, tmp->data, dye_fused ? image->data : nullptr,
                dye_fused ? itmp->data : nullptr, vp->x, vp->y, dt, viscosity, iters,
@@ -435,7 +487,9 @@ int pfs_fluid_run(pfs_field *vp, pfs_field *tmp, pfs_field *image, pfs_field *it
     hipStream_t s = (hipStream_t)stream;
     RunGraph want{0, {*vp, *tmp, *image, *itmp}, dt, viscosity, iters, 0, 0, nullptr, nullptr};
     PFS_HIP_TRY(hipGetDevice(&want.dev));
-    PFS_TRY(get_workspace(fused_workspace_bytes(vp->x, vp->y), s, &want.ws));  // allocated already
+    Lease lease;
+    PFS_TRY(get_workspace(fused_workspace_bytes(vp->x, vp->y), s, &lease));  // allocated already
+    want.ws = lease.ptr;
     const bool dye_fused = image->x == vp->x && image->y == vp->y && image->z == 4 &&
                            aligned16(image->data) && aligned16(itmp->data);
     want.tile = step_tile(vp->x, vp->y, iters, dye_fused);

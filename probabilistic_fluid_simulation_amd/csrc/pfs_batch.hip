@@ -55,7 +55,7 @@ __global__ __launch_bounds__(kWaveMax * 64, S == 2 ? 8 : 6) void k_diffuse_wave_
     const DiffuseArgs *__restrict__ tab, const int *__restrict__ tile_scene, int ntiles) {
     const int b = xcd_tile(blockIdx.x, ntiles);
     const DiffuseArgs a = tab[tile_scene[b]];
-    diffuse_wave<H, FIRST, LAST, S>(a, b - a.tile_base);
+    diffuse_wave<H, FIRST ? From::Advect : From::Plane, LAST ? To::Step : To::Plane, S>(a, b - a.tile_base);
 }
 
 template <int H, bool LAST, int TS>

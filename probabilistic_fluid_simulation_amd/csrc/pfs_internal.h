@@ -107,6 +107,14 @@ struct StepArgs {
 // idempotent: neither reads what it writes).
 int fused_step(const StepArgs &a, float *ws, hipStream_t s, hipEvent_t *ev, int reps = 1);
 size_t fused_workspace_bytes(int w, int h);
+// The sweeps of the operators diffuse and computePressure on 4-channel,
+// 16-byte aligned fields, kOpMinIters sweeps or more, in a few launches (the
+// same workspace).
+constexpr int kOpMinIters = 5;
+int diffuse_op(const float *a, float *last, float *before, int w, int h, float dt, float visc,
+               int iters, float *ws, hipStream_t s);
+int pressure_op(float *a, float *last, float *before, int w, int h, float dt, int iters, float *ws,
+                hipStream_t s);
 int threads_for(int H, int ts = 64);  // threads of the fused kernels for halo H, tile side ts
 
 // Validation helpers.

@@ -296,7 +296,7 @@ template <int H, bool FIRST, bool LAST, int S>
 __global__ __launch_bounds__(kWaveMax * 64, S == 2 ? 8 : 6) void k_diffuse_wave_precise(DiffuseArgs a,
                                                                                       PCtl *ctl) {
     clear_ctl(ctl);
-    diffuse_wave<H, FIRST, LAST, S, true>(a, xcd_tile(blockIdx.x, a.ntiles));
+    diffuse_wave<H, FIRST ? From::Advect : From::Plane, LAST ? To::Step : To::Plane, S, true>(a, xcd_tile(blockIdx.x, a.ntiles));
 }
 
 // Up to C = H - 1 compensated pressure sweeps of one tile, the residual of

@@ -57,12 +57,29 @@ __global__ __launch_bounds__((Geo<H, 16>::NT)) void k_diffuse(DiffuseArgs a) {
 // Larger fields.
 template <int H, bool FIRST, bool LAST, int S>
 __global__ __launch_bounds__(kWaveMax * 64, S == 2 ? 8 : 6) void k_diffuse_wave(DiffuseArgs a) {
-    diffuse_wave<H, FIRST, LAST, S>(a, xcd_tile(blockIdx.x, a.ntiles));
+    diffuse_wave<H, FIRST ? From::Advect : From::Plane, LAST ? To::Step : To::Plane, S>(
+        a, xcd_tile(blockIdx.x, a.ntiles));
 }
 
 template <int H, bool LAST, int TS>
 __global__ __launch_bounds__((Geo<H, TS>::NT)) void k_pressure(PressureArgs a) {
     pressure_tile<H, LAST, TS>(a, xcd_tile(blockIdx.x, a.ntiles));
+}
+
+// Chunks of the pressure that are not the last, on larger fields.
+__global__ __launch_bounds__(kWaveMax * 64, 8) void k_pressure_wave(PressureArgs a) {
+    pressure_wave<kMaxChunk, From::Plane, To::Plane, 4>(a, xcd_tile(blockIdx.x, a.ntiles));
+}
+
+// The operators diffuse and computePressure.
+template <int H, From FROM, To TO, int S>
+__global__ __launch_bounds__(kWaveMax * 64, S == 2 ? 8 : 6) void k_diffuse_op(DiffuseArgs a) {
+    diffuse_wave<H, FROM, TO, S>(a, xcd_tile(blockIdx.x, a.ntiles));
+}
+
+template <int H, From FROM, To TO, int S>
+__global__ __launch_bounds__(kWaveMax * 64, S == 2 ? 8 : 6) void k_pressure_op(PressureArgs a) {
+    pressure_wave<H, FROM, TO, S>(a, xcd_tile(blockIdx.x, a.ntiles));
 }
 
 // ---- host dispatch over the compile-time halo and tile side ----------------
@@ -128,13 +145,62 @@ int threads_for_ts(int H) {
     return 0;
 }
 
-// The wave shape of one field's launch with halo H; sets d's tile counts to it.
-WaveShape wave_args(DiffuseArgs &d, int H) {
+// The wave shape of one field's launch with halo H; sets the launch's tile
+// counts (of DiffuseArgs or PressureArgs) to it.
+template <typename Args>
+WaveShape wave_args(Args &d, int H) {
     const WaveShape sh =
         wave_shape(H, device_cus(), [&](WaveShape s) { return wave_tiles(d.w, d.h, H, s); });
     d.tiles_x = wave_tiles_x(d.w, H);
     d.ntiles = (int)wave_tiles(d.w, d.h, H, sh);
     return sh;
+}
+
+// An operator's sweeps in launches.  The first reads the field and writes
+// planes, the last reads planes and writes both fields (a launch that read a
+// field and wrote one would race with its own halo reads), so there are at
+// least two: 4 + the rest up to 8 sweeps, else 8 at a time and the rest last.
+struct OpPlan {
+    int first, middles, last;
+};
+OpPlan op_plan(int iters) {
+    if (iters <= kMaxChunk) return {4, 0, iters - 4};
+    const int rest = (iters - 1) % kMaxChunk + 1;
+    return {kMaxChunk, (iters - rest) / kMaxChunk - 1, rest};
+}
+
+template <int S>
+DiffuseFn diffuse_op_for(int ns, From from, To to) {
+    if (to == To::Plane) {
+        if (from == From::Plane) return k_diffuse_wave<kMaxChunk, false, false, S>;
+        return ns == 4 ? k_diffuse_op<4, From::Field, To::Plane, S>
+                       : k_diffuse_op<kMaxChunk, From::Field, To::Plane, S>;
+    }
+    switch (ns) {
+#define PFS_CASE(n) \
+    case n:         \
+        return k_diffuse_op<n, From::Plane, To::Field, S>;
+        PFS_CASE(1) PFS_CASE(2) PFS_CASE(3) PFS_CASE(4) PFS_CASE(5) PFS_CASE(6) PFS_CASE(7) PFS_CASE(8)
+#undef PFS_CASE
+    }
+    return nullptr;
+}
+
+template <int S>
+PressureFn pressure_op_for(int ns, From from, To to) {
+    if (to == To::Plane) {
+        if (from == From::Plane) return k_pressure_op<kMaxChunk, From::Plane, To::Plane, S>;
+        return ns == 4 ? k_pressure_op<4, From::Field, To::Plane, S>
+                       : k_pressure_op<kMaxChunk, From::Field, To::Plane, S>;
+    }
+    switch (ns) {
+#define PFS_CASE(n) \
+    case n:         \
+        return k_pressure_op<n, From::Plane, To::Field, S>;
+        PFS_CASE(1) PFS_CASE(2) PFS_CASE(3) PFS_CASE(4) PFS_CASE(5) PFS_CASE(6) PFS_CASE(7) PFS_CASE(8)
+#undef PFS_CASE
+    }
+    return nullptr;
 }
 
 }  // namespace
@@ -181,11 +247,66 @@ int fused_step(const StepArgs &s, float *ws, hipStream_t stream, hipEvent_t *ev,
     for (int r = 0; r < reps; ++r)
         for (int c = 0; c < nchunks; ++c) {
             pressure_chunk(p, c, plan[c], ws, s.image, s.itmp);
-            hipLaunchKernelGGL(pressure_for(plan[c].H, plan[c].last, s.tile), grid,
-                               dim3(threads_for(plan[c].H, s.tile)), 0, stream, p);
+            const Chunk &k = plan[c];
+            PressureArgs w = p;
+            // Only whole chunks of fields with two workgroups for every CU:
+            // below that the square tiles are as fast (2048^2: 22.5 us against
+            // 24; 1024^2: equal).
+            const WaveShape sh = k.last || s.tile != 64 ? WaveShape{0, 0} : wave_args(w, k.H);
+            if (sh.S == 4 && w.ntiles >= 2 * device_cus())
+                hipLaunchKernelGGL(k_pressure_wave, dim3(w.ntiles), dim3(64 * sh.nw), 0, stream, w);
+            else
+                hipLaunchKernelGGL(pressure_for(k.H, k.last, s.tile), grid,
+                                   dim3(threads_for(k.H, s.tile)), 0, stream, p);
             PFS_TRY(check_launch("fused pressure"));
         }
     if (ev) PFS_HIP_TRY(hipEventRecord(ev[3], stream));
+    return PFS_OK;
+}
+
+// The operators' sweeps (include/fluid.hpp's diffuse and computePressure) in
+// the step's wave tiles.  a holds the input; on return the last iterate is in
+// `last` and the one before it in `before` (the two fields, in the order the
+// reference's pointer swaps leave them).  Other channels keep their values.
+int diffuse_op(const float *a, float *last, float *before, int w, int h, float dt, float visc,
+               int iters, float *ws, hipStream_t stream) {
+    DiffuseArgs d = diffuse_args(a, a, w, h, dt, visc, iters, ws);
+    d.field[0] = last;
+    d.field[1] = before;
+    const OpPlan plan = op_plan(iters);
+    const int n = plan.middles + 2;
+    for (int c = 0; c < n; ++c) {
+        const int ns = c == 0 ? plan.first : c == n - 1 ? plan.last : kMaxChunk;
+        const From from = c == 0 ? From::Field : From::Plane;
+        const To to = c == n - 1 ? To::Field : To::Plane;
+        diffuse_chunk(d, c, Chunk{ns, ns, c == 0, c == n - 1}, ws);
+        const WaveShape sh = wave_args(d, ns);
+        hipLaunchKernelGGL(sh.S == 2 ? diffuse_op_for<2>(ns, from, to) : diffuse_op_for<4>(ns, from, to),
+                           dim3(d.ntiles), dim3(64 * sh.nw), 0, stream, d);
+        PFS_TRY(check_launch("diffuse"));
+    }
+    return PFS_OK;
+}
+
+int pressure_op(float *a, float *last, float *before, int w, int h, float dt, int iters, float *ws,
+                hipStream_t stream) {
+    PressureArgs p = pressure_args(a, a, nullptr, nullptr, w, h, dt, ws);
+    p.gamma = pressure_gamma(dt);
+    p.bdst = ws + (size_t)w * h;  // what bpl reads
+    p.field[0] = last;
+    p.field[1] = before;
+    const OpPlan plan = op_plan(iters);
+    const int n = plan.middles + 2;
+    for (int c = 0; c < n; ++c) {
+        const int ns = c == 0 ? plan.first : c == n - 1 ? plan.last : kMaxChunk;
+        const From from = c == 0 ? From::Field : From::Plane;
+        const To to = c == n - 1 ? To::Field : To::Plane;
+        pressure_chunk(p, c, Chunk{ns, ns, false, c == n - 1}, ws, nullptr, nullptr);
+        const WaveShape sh = wave_args(p, ns);
+        hipLaunchKernelGGL(sh.S == 2 ? pressure_op_for<2>(ns, from, to) : pressure_op_for<4>(ns, from, to),
+                           dim3(p.ntiles), dim3(64 * sh.nw), 0, stream, p);
+        PFS_TRY(check_launch("computePressure"));
+    }
     return PFS_OK;
 }
 

@@ -76,7 +76,8 @@ struct DiffuseArgs {
     int fast_div;  // division by beta: 0 IEEE, 1 five operations, 2 two (proven for it)
     FixedDiv db, dw, dh;  // beta, w and h as fixed divisors
     int first, k_even;
-    int tile_base;  // first tile of this scene in a batched launch
+    int tile_base;    // first tile of this scene in a batched launch
+    float *field[2];  // the operator's fields: of the last iterate, of the one before
 };
 
 struct PressureArgs {
@@ -96,6 +97,9 @@ struct PressureArgs {
     float dt_viw, dt_vih;  // dt / (field/image width ratio), as src/fluid.cpp:97-98
     int first;
     int tile_base;  // first tile of this scene in a batched launch
+    float gamma;      // the operator's own: -1 / dt,
+    float *bdst;      // the divergence plane its first chunk writes,
+    float *field[2];  // its fields: of the last iterate, of the one before
 };
 
 // Thread (x, seg) of a tile: column x of the staged region, rows

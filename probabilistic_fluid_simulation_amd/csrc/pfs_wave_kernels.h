@@ -125,8 +125,21 @@ __device__ __forceinline__ float own_register(float x) {
     return y;
 }
 
-template <int H, bool FIRST, bool LAST, int S, bool COMP = false>
+// Where a launch's cells come from and go to.
+enum class From {
+    Plane,   // the iterate plane of the chunk before
+    Advect,  // the step's first chunk: vp, advected
+    Field    // an operator's first chunk: the field itself
+};
+enum class To {
+    Plane,  // the iterate plane
+    Step,   // the step's last chunk: E, the divergence and the pressure start
+    Field   // an operator's last chunk: the last two iterates into the two fields
+};
+
+template <int H, From FROM, To TO, int S, bool COMP = false>
 __device__ __forceinline__ void diffuse_wave(const DiffuseArgs &a, int tile) {
+    constexpr bool FIRST = FROM == From::Advect, LAST = TO == To::Step;
     constexpr int NS = H - (LAST ? 1 : 0);
     constexpr int NWMAX = kWaveMax;
     constexpr int XB = NWMAX * 2 * 64;  // one exchange buffer: two rows per wave
@@ -207,6 +220,19 @@ __device__ __forceinline__ void diffuse_wave(const DiffuseArgs &a, int tile) {
             }
         }
         __syncthreads();  // the exchange buffers lie over the staged velocities
+    } else if (FROM == From::Field) {
+        const float2 *__restrict__ F2 = reinterpret_cast<const float2 *>(a.P);
+        int gj = t.first_row(a.h);
+#pragma unroll
+        for (int k = 0; k < S; ++k) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const float2 c = F2[2 * (gj * a.w + t.gi[q])];
+                u[k][q] = c.x;
+                v[k][q] = c.y;
+            }
+            gj = t.next_row(gj, a.h);
+        }
     } else {
         int gj = t.first_row(a.h);
 #pragma unroll
@@ -248,6 +274,15 @@ __device__ __forceinline__ void diffuse_wave(const DiffuseArgs &a, int tile) {
                 warm[k][z] = W[4 * (warm_ok(k, z) ? wcell + k * a.w + 64 * z : 0) + 2];
     }
 
+    auto store_field = [&](float *f) {  // channels 0 and 1 of an operator's field
+        float2 *F2 = reinterpret_cast<float2 *>(f);
+#pragma unroll
+        for (int k = 0; k < S; ++k)
+            if (t.row_mine(k, a.h) && col0) {
+                F2[2 * (cell0 + k * a.w)] = make_float2(u[k][0], v[k][0]);
+                if (col1) F2[2 * (cell0 + k * a.w + 1)] = make_float2(u[k][1], v[k][1]);
+            }
+    };
     auto store_uv = [&]() {  // the iterate, or E
 #pragma unroll
         for (int k = 0; k < S; ++k)
@@ -368,9 +403,14 @@ __device__ __forceinline__ void diffuse_wave(const DiffuseArgs &a, int tile) {
 #pragma unroll 1
     for (int s = 1; s < NS; ++s) sweep(s, std::true_type{});
     if (LAST && !a.k_even) store_uv();  // E = D^(K-1)
+    if (TO == To::Field) store_field(a.field[1]);
     sweep(NS, std::false_type{});
     each([](float &x) { x = own_register(x); });
 
+    if (TO == To::Field) {
+        store_field(a.field[0]);
+        return;
+    }
     if (!LAST) {
         store_uv();
         return;
@@ -402,6 +442,134 @@ __device__ __forceinline__ void diffuse_wave(const DiffuseArgs &a, int tile) {
             store_pair(a.bpl + cell, d0, d1, col1);
         }
     }
+}
+
+// H pressure sweeps (src/fluid.cpp:240-257) in the same layout: a chunk of the
+// step that is not its last (Plane to Plane), or of the operator
+// computePressure, whose first chunk also forms the divergence
+// (src/fluid.cpp:221-237) of the field it reads and whose last writes the
+// last two iterates and the divergence into both fields.
+// Bound, like the diffusion's sweeps, by VALU issue; one value a cell and no
+// division.  3840x2160, 8 sweeps: 33 us against 39 us for the square tiles
+// (whose LDS traffic is 7 rows written and 16 read a wave and sweep).
+template <int H, From FROM, To TO, int S>
+__device__ __forceinline__ void pressure_wave(const PressureArgs &a, int tile) {
+    constexpr int NS = H;
+    constexpr int XB = kWaveMax * 2 * 64;
+    __shared__ float2 lds[2 * XB];
+
+    const WaveTile<H, S> t(tile, a.tiles_x, a.w, a.h);
+    const int top_row = max(2 * t.wave - 1, 0) * 64 + t.lane;
+    const int bot_row = min(2 * t.wave + 2, 2 * t.nw - 1) * 64 + t.lane;
+    const bool col0 = t.col_mine(0, a.w), col1 = t.col_mine(1, a.w);
+    const int cell0 = (t.y0 + t.r0) * a.w + t.xc;
+    float2 c[S], rhs[S], lr[S];
+    if (FROM == From::Field) {
+        const float4 *__restrict__ F4 = reinterpret_cast<const float4 *>(a.P);
+        float4 f[S][2];
+        int gj = t.first_row(a.h);
+#pragma unroll
+        for (int k = 0; k < S; ++k) {
+            f[k][0] = F4[gj * a.w + t.gi[0]];
+            f[k][1] = F4[gj * a.w + t.gi[1]];
+            gj = t.next_row(gj, a.h);
+        }
+        lds[2 * t.wave * 64 + t.lane] = make_float2(f[0][0].y, f[0][1].y);
+        lds[(2 * t.wave + 1) * 64 + t.lane] = make_float2(f[S - 1][0].y, f[S - 1][1].y);
+        __syncthreads();
+        const float2 above = lds[top_row], below = lds[bot_row];
+#pragma unroll
+        for (int k = 0; k < S; ++k) {
+            const int up = k > 0 ? k - 1 : 0, down = k + 1 < S ? k + 1 : k;
+            const float2 T = k == 0 ? above : make_float2(f[up][0].y, f[up][1].y);
+            const float2 B = k == S - 1 ? below : make_float2(f[down][0].y, f[down][1].y);
+            c[k] = make_float2(f[k][0].z, f[k][1].z);
+            rhs[k] = make_float2(a.gamma * ((f[k][1].x - from_left(f[k][1].x)) + (B.x - T.x)),
+                                 a.gamma * ((from_right(f[k][0].x) - f[k][0].x) + (B.y - T.y)));
+        }
+    } else {
+        const float *__restrict__ src = a.first ? a.pw : a.psrc;
+        int gj = t.first_row(a.h);
+#pragma unroll
+        for (int k = 0; k < S; ++k) {
+            const float *sr = src + gj * a.w, *br = a.bpl + gj * a.w;
+            if (t.inside) {
+                const Pair<float> x = *reinterpret_cast<const Pair<float> *>(sr + t.xc);
+                const Pair<float> y = *reinterpret_cast<const Pair<float> *>(br + t.xc);
+                c[k] = make_float2(x.a, x.b);
+                rhs[k] = make_float2(y.a, y.b);
+            } else {
+                c[k] = make_float2(sr[t.gi[0]], sr[t.gi[1]]);
+                rhs[k] = make_float2(br[t.gi[0]], br[t.gi[1]]);
+            }
+            gj = t.next_row(gj, a.h);
+        }
+    }
+    const float quarter = own_register(0.25f);
+#pragma unroll
+    for (int k = 0; k < S; ++k) {
+        c[k] = make_float2(own_register(c[k].x), own_register(c[k].y));
+        rhs[k] = make_float2(own_register(rhs[k].x), own_register(rhs[k].y));
+    }
+    // Sweep s reads buffer s & 1 (the divergence's exchange used buffer 0).
+    auto publish = [&](int s) {
+        float2 *X = lds + (s & 1) * XB;
+        X[2 * t.wave * 64 + t.lane] = c[0];
+        X[(2 * t.wave + 1) * 64 + t.lane] = c[S - 1];
+    };
+    auto sides = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < S; ++k)
+            lr[k] = make_float2(from_left(c[k].y) + c[k].y, from_right(c[k].x) + c[k].x);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto cell = [&](int k, const float2 &T, const float2 &B) {  // / 4 as the exact product by a quarter
+        return make_float2((lr[k].x + T.x + B.x + 1.0f * rhs[k].x) * quarter,
+                           (lr[k].y + T.y + B.y + 1.0f * rhs[k].y) * quarter);
+    };
+    auto sweep = [&](int s, auto more) {
+        const float2 *X = lds + (s & 1) * XB;
+        const float2 above = X[top_row], below = X[bot_row];
+        float2 n[S];
+#pragma unroll
+        for (int k = 1; k < S - 1; ++k) n[k] = cell(k, c[k - 1], c[k + 1 < S ? k + 1 : k]);
+        n[0] = cell(0, above, c[1]);
+        n[S - 1] = cell(S - 1, c[S - 2], below);
+#pragma unroll
+        for (int k = 0; k < S; ++k) c[k] = n[k];
+        if (decltype(more)::value) {
+            publish(s + 1);
+            sides();
+            __syncthreads();
+        }
+    };
+    auto store_field = [&](float *f) {  // channels 2 and 3 of an operator's field
+        float2 *F2 = reinterpret_cast<float2 *>(f);
+#pragma unroll
+        for (int k = 0; k < S; ++k)
+            if (t.row_mine(k, a.h) && col0) {
+                F2[2 * (cell0 + k * a.w) + 1] = make_float2(c[k].x, rhs[k].x);
+                if (col1) F2[2 * (cell0 + k * a.w + 1) + 1] = make_float2(c[k].y, rhs[k].y);
+            }
+    };
+    publish(1);
+    sides();
+    __syncthreads();
+#pragma unroll 2
+    for (int s = 1; s < NS; ++s) sweep(s, std::true_type{});
+    if (TO == To::Field) store_field(a.field[1]);
+    sweep(NS, std::false_type{});
+    if (TO == To::Field) {
+        store_field(a.field[0]);
+        return;
+    }
+#pragma unroll
+    for (int k = 0; k < S; ++k)
+        if (t.row_mine(k, a.h) && col0) {
+            store_pair(a.pdst + cell0 + k * a.w, own_register(c[k].x), own_register(c[k].y), col1);
+            if (FROM == From::Field) store_pair(a.bdst + cell0 + k * a.w, rhs[k].x, rhs[k].y, col1);
+        }
 }
 
 // ---- host side: the shape of a launch ---------------------------------------

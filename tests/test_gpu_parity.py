@@ -96,6 +96,96 @@ def test_diffuse_and_pressure_with_swaps(orc, shape, k):
     assert_bitexact([vp.numpy(), tmp.numpy()], [wa, wb], ("vp", "vp_out"))
 
 
+def _both_operators(orc, s, k):
+    """diffuse and computePressure from the same state, with the reference's
+    pointer swaps: the GPU's (vp, vp_out) and the oracle's, four arrays each."""
+    got, want = [], []
+    for name, gpu, cpu in (("diffuse", lambda a, b: fluid.diffuse(a, b, s.visc, s.dt, k),
+                            lambda a, b: orc.diffuse(a, b, s.visc, s.dt, k)),
+                           ("pressure", lambda a, b: fluid.computePressure(a, b, s.dt, k),
+                            lambda a, b: orc.compute_pressure(a, b, s.dt, k))):
+        vp, tmp = VPField.from_numpy(s.vp), VPField.from_numpy(s.tmp)
+        gpu(vp, tmp)
+        got += [vp.numpy(), tmp.numpy()]
+        want += list(cpu(s.vp.copy(), s.tmp.copy()))
+    return got, want
+
+
+@pytest.mark.parametrize("k", [4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 17, 24, 30])
+@pytest.mark.parametrize("shape", [(1, 1), (7, 3), (129, 67), (331, 403), (1201, 803)],
+                         ids=lambda x: "%dx%d" % x)
+def test_operator_sweeps_in_few_launches(orc, shape, k):
+    """From 5 sweeps on, diffuse and computePressure run several sweeps a
+    launch: every split of the sweeps, fields from one cell to several tiles
+    of both strip heights; all channels of both fields."""
+    s = scenes.random_scene(*shape, 1, 1, seed=80 + k, dt=0.7, visc=0.3)
+    got, want = _both_operators(orc, s, k)
+    assert_bitexact(got, want, ("d.vp", "d.out", "p.vp", "p.out"))
+
+
+def test_operator_sweeps_on_general_path():
+    """Five channels, a misaligned field and a stream being captured take one
+    launch per sweep, with the results of the few-launch form; the captured
+    calls replay."""
+    s = scenes.random_scene(70, 41, 1, 1, seed=9, dt=0.7, visc=0.3)
+    k = 7
+
+    def run(vp, tmp):
+        fluid.diffuse(vp, tmp, s.visc, s.dt, k)
+        fluid.computePressure(tmp, vp, s.dt, k)
+        return vp.numpy()[..., :4].tobytes(), tmp.numpy()[..., :4].tobytes()
+
+    def padded(a):
+        return VPField(torch.cat([torch.from_numpy(a).cuda(), torch.zeros(41, 70, 1, device="cuda")], -1).contiguous())
+
+    def shifted(a):
+        buf = torch.empty(a.size + 1, device="cuda")
+        f = VPField(buf[1:].view(a.shape))
+        f.data.copy_(torch.from_numpy(a))
+        return f
+
+    want = run(VPField.from_numpy(s.vp), VPField.from_numpy(s.tmp))
+    assert run(padded(s.vp), padded(s.tmp)) == want
+    assert run(shifted(s.vp), shifted(s.tmp)) == want
+    vp, tmp = VPField.from_numpy(s.vp), VPField.from_numpy(s.tmp)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        fluid.diffuse(vp, tmp, s.visc, s.dt, k)
+        fluid.computePressure(tmp, vp, s.dt, k)
+    for _ in range(3):
+        vp.data.copy_(torch.from_numpy(s.vp))
+        tmp.data.copy_(torch.from_numpy(s.tmp))
+        g.replay()
+        torch.cuda.synchronize()
+        assert (vp.numpy().tobytes(), tmp.numpy().tobytes()) == want
+
+
+def test_operators_from_threads_on_one_stream(orc):
+    """Threads that share a stream share its workspace: their calls' launches
+    do not interleave."""
+    import threading
+    scs = [scenes.random_scene(150 + 40 * i, 90 + 30 * i, 1, 1, seed=i, dt=0.7, visc=0.3) for i in range(4)]
+    bufs = [(VPField.from_numpy(s.vp), VPField.from_numpy(s.tmp)) for s in scs]
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+
+    def work(i):
+        for _ in range(20):
+            fluid.diffuse(*bufs[i], scs[i].visc, scs[i].dt, 9, stream=stream)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for s, (vp, tmp) in zip(scs, bufs):
+        a, b = s.vp.copy(), s.tmp.copy()
+        for _ in range(20):
+            a, b = orc.diffuse(a, b, s.visc, s.dt, 9)
+        assert_bitexact([vp.numpy(), tmp.numpy()], [a, b], ("vp", "out"))
+
+
 @pytest.mark.parametrize("shape", SHAPES, ids=_ids(SHAPES))
 def test_subtract_pressure_gradient(orc, shape):
     s = scenes.random_scene(*shape, seed=5)
