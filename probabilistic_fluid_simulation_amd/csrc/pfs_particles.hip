@@ -29,6 +29,7 @@
 #include <cmath>
 #include <cstdint>
 #include <string>
+#include <type_traits>
 
 #include "pfs.h"
 #include "pfs_device.h"
@@ -375,58 +376,86 @@ struct NArgs {
     __device__ uint32_t id(uint32_t p) const { return order ? order[p] : p; }
 };
 
-// Visits every particle q of the 3x3 cells around p's cell, p included (rows
-// then columns, -1..1, then q ascending): f(q, d2) with d2 the squared
-// periodic distance, for every candidate, so that callers accumulate without
-// branching.  The cells of one row are consecutive keys, so the three are
-// one range of sorted positions, [start of the left cell, end of the right
-// cell), split in two where the row wraps.
-template <typename F>
-__device__ __forceinline__ void for_neighbors(const NArgs &a, int p, F &&f) {
-    const uint32_t c = a.sk[p];
-    if (c >= (uint32_t)a.gx * (uint32_t)a.gy) return;  // a cell by construction: kept as a bound
-    const int cx = (int)(c % (uint32_t)a.gx), cy = (int)(c / (uint32_t)a.gx);
+// ---- four lanes per particle ------------------------------------------------
+// The neighbour passes give a particle a quad of lanes: four candidates (or
+// listed neighbours) are loaded and evaluated side by side, and order-bound
+// sums are then added up one after another, each term broadcast over the quad
+// by a DPP operand of its addition, so that every value equals the serial
+// walk's.  Against one lane per particle the chain of dependent loads is a
+// quarter as long, a wavefront's loads cover consecutive addresses, and a
+// small set fills four times as many wavefronts; the sums cost one addition a
+// term on every lane.  All four lanes of a quad always run together.
+__device__ __forceinline__ int quad_lane() { return (int)(threadIdx.x & 3u); }
+
+template <int J>
+__device__ __forceinline__ uint32_t quad_bcast(uint32_t x) {  // lane J's value
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x55 * J, 0xf, 0xf, true);
+}
+template <int J>
+__device__ __forceinline__ float quad_bcast(float x) {
+    return __uint_as_float(quad_bcast<J>(__float_as_uint(x)));
+}
+// s + the quad's four terms in lane order.
+__device__ __forceinline__ float quad_add(float s, float t) {
+    s += quad_bcast<0>(t);
+    s += quad_bcast<1>(t);
+    s += quad_bcast<2>(t);
+    s += quad_bcast<3>(t);
+    return s;
+}
+__device__ __forceinline__ uint32_t quad_total(uint32_t c) {
+    return quad_bcast<0>(c) + quad_bcast<1>(c) + quad_bcast<2>(c) + quad_bcast<3>(c);
+}
+// The quad's bits of a wave-wide vote.
+__device__ __forceinline__ uint32_t quad_vote(bool b) {
+    return (uint32_t)(__ballot(b) >> (threadIdx.x & 60u)) & 0xfu;
+}
+
+// The sorted positions of one row of the 3x3 cells around cell (cx, cy): [s1,
+// e1) the row's cells in order up to a wrap, [s2, e2) those after it.  The
+// cells of one row are consecutive keys, so without a wrap the three are one
+// range, [start of the left cell, end of the right cell).
+struct RowRanges {
+    uint32_t s1, e1, s2, e2;
+};
+__device__ __forceinline__ RowRanges row_ranges(const NArgs &a, int cx, int cy, int oy) {
+    const int ny = cy + oy < 0 ? cy + oy + a.gy : (cy + oy >= a.gy ? cy + oy - a.gy : cy + oy);
+    const uint32_t row = (uint32_t)(ny * a.gx);
+    RowRanges r{0, 0, 0, 0};
+    if (cx == 0) {  // cells gx-1 | 0, 1
+        r.s1 = a.start[row + a.gx - 1];
+        r.e1 = a.end[row + a.gx - 1];
+        r.s2 = a.start[row];
+        r.e2 = a.end[row + 1];
+    } else if (cx == a.gx - 1) {  // cells gx-2, gx-1 | 0
+        r.s1 = a.start[row + cx - 1];
+        r.e1 = a.end[row + cx];
+        r.s2 = a.start[row];
+        r.e2 = a.end[row];
+    } else {
+        r.s1 = a.start[row + cx - 1];
+        r.e1 = a.end[row + cx + 1];
+    }
+    r.e1 = min(r.e1, (uint32_t)a.n);
+    r.e2 = min(r.e2, (uint32_t)a.n);
+    return r;
+}
+
+// The three rows' ranges (lo, hi: [k][0] up to a wrap, [k][1] after) of p's
+// cell, visited in order: near(q, end, d2_of) for the whole row of a cell away
+// from the domain's edges, else any(q, end, d2_of) for each range; d2_of the
+// squared periodic distance of a candidate at (x, y) from p.
+template <typename Near, typename Any>
+__device__ __forceinline__ void visit_rows(const NArgs &a, int p, int cx, int cy,
+                                           const uint32_t (&lo)[3][2], const uint32_t (&hi)[3][2],
+                                           Near &&near, Any &&any) {
     const float px = a.xs[p], py = a.ys[p];
-    // Candidates are taken four at a time, their loads issued together, and
-    // visited in ascending q as one at a time would.  Away from the domain's
-    // edges no candidate is more than 3 cells away, less than half the
-    // domain when it spans 7 or more cells: there the periodic correction is
-    // the identity and that loop skips it.
-    auto scan = [&](uint32_t q0, uint32_t q1, auto &&d2_of) {
-        q1 = min(q1, (uint32_t)a.n);
-        uint32_t q = q0;
-        const float *xp = a.xs + q0, *yp = a.ys + q0;
-        for (; q + 4 <= q1; q += 4, xp += 4, yp += 4) {
-            const float x0 = xp[0], x1 = xp[1], x2 = xp[2], x3 = xp[3];
-            const float y0 = yp[0], y1 = yp[1], y2 = yp[2], y3 = yp[3];
-            const float e0 = d2_of(x0, y0), e1 = d2_of(x1, y1), e2 = d2_of(x2, y2),
-                        e3 = d2_of(x3, y3);
-            f(q, e0);
-            f(q + 1, e1);
-            f(q + 2, e2);
-            f(q + 3, e3);
-        }
-        for (; q < q1; ++q, ++xp, ++yp) f(q, d2_of(*xp, *yp));
-    };
-    auto rows = [&](auto &&d2_of) {
-        for (int oy = -1; oy <= 1; ++oy) {
-            const int ny = cy + oy < 0 ? cy + oy + a.gy : (cy + oy >= a.gy ? cy + oy - a.gy : cy + oy);
-            const uint32_t row = (uint32_t)(ny * a.gx);
-            if (cx == 0) {  // cells gx-1 | 0, 1
-                scan(a.start[row + a.gx - 1], a.end[row + a.gx - 1], d2_of);
-                scan(a.start[row], a.end[row + 1], d2_of);
-            } else if (cx == a.gx - 1) {  // cells gx-2, gx-1 | 0
-                scan(a.start[row + cx - 1], a.end[row + cx], d2_of);
-                scan(a.start[row], a.end[row], d2_of);
-            } else {
-                scan(a.start[row + cx - 1], a.end[row + cx + 1], d2_of);
-            }
-        }
-    };
     const bool big = a.gx >= 7 && a.gy >= 7;
-    const bool interior = cx >= 1 && cx <= a.gx - 2 && cy >= 1 && cy <= a.gy - 2 && big;
-    if (interior) {
-        rows([&](float ox, float oy) {
+    if (big && cx >= 1 && cx <= a.gx - 2 && cy >= 1 && cy <= a.gy - 2) {
+        // No candidate is more than 3 cells away, less than half the domain
+        // when it spans 7 or more cells: the periodic correction is the
+        // identity.
+        near([&](float ox, float oy) {
             const float dx = ox - px, dy = oy - py;
             return dx * dx + dy * dy;
         });
@@ -439,89 +468,191 @@ __device__ __forceinline__ void for_neighbors(const NArgs &a, int p, F &&f) {
         // every shifted one at least 5W/7 away before the shift, so these
         // are exactly the cases periodic_diff corrects, with its values:
         // (x_q + -W) - x_p and (x_q + -0) - (x_p - W).
-        for (int oy = -1; oy <= 1; ++oy) {
-            const int ny = cy + oy < 0 ? cy + oy + a.gy : (cy + oy >= a.gy ? cy + oy - a.gy : cy + oy);
-            const uint32_t row = (uint32_t)(ny * a.gx);
-            const float qsy = (cy == 0 && oy == -1) ? -a.H : -0.0f;
-            const float pyu = (cy == a.gy - 1 && oy == 1) ? py - a.H : py;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const float qsy = (cy == 0 && k == 0) ? -a.H : -0.0f;
+            const float pyu = (cy == a.gy - 1 && k == 2) ? py - a.H : py;
             auto shifted = [&](float qsx, float pxu) {
                 return [=](float ox, float oy_) {
                     const float dx = (ox + qsx) - pxu, dy = (oy_ + qsy) - pyu;
                     return dx * dx + dy * dy;
                 };
             };
-            if (cx == 0) {  // cells gx-1 | 0, 1
-                scan(a.start[row + a.gx - 1], a.end[row + a.gx - 1], shifted(-a.W, px));
-                scan(a.start[row], a.end[row + 1], shifted(-0.0f, px));
-            } else if (cx == a.gx - 1) {  // cells gx-2, gx-1 | 0
-                scan(a.start[row + cx - 1], a.end[row + cx], shifted(-0.0f, px));
-                scan(a.start[row], a.end[row], shifted(-0.0f, px - a.W));
-            } else {
-                scan(a.start[row + cx - 1], a.end[row + cx + 1], shifted(-0.0f, px));
-            }
+            any(lo[k][0], hi[k][0], shifted(cx == 0 ? -a.W : -0.0f, px));
+            any(lo[k][1], hi[k][1], shifted(-0.0f, cx == a.gx - 1 ? px - a.W : px));
         }
     } else {
-        rows([&](float ox, float oy) {
+        auto d2_of = [&](float ox, float oy) {
             const float dx = periodic_diff(ox, px, a.W, a.half_w);
             const float dy = periodic_diff(oy, py, a.H, a.half_h);
             return dx * dx + dy * dy;
-        });
+        };
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            any(lo[k][0], hi[k][0], d2_of);
+            any(lo[k][1], hi[k][1], d2_of);
+        }
     }
 }
 
-__global__ void k_nbr_count(NArgs a, uint32_t *__restrict__ counts) {
+// Visits every particle q of the 3x3 cells around p's cell, p included (rows
+// then columns, -1..1, then q ascending), four at a time: f(q, ok, d2) on the
+// quad's lanes for consecutive q, ok false past a range's end.
+template <typename F>
+__device__ __forceinline__ void for_neighbors(const NArgs &a, int p, F &&f) {
+    const uint32_t c = a.sk[p];
+    if (c >= (uint32_t)a.gx * (uint32_t)a.gy) return;  // a cell by construction: kept as a bound
+    const int cx = (int)(c % (uint32_t)a.gx), cy = (int)(c / (uint32_t)a.gx);
+    const int l = quad_lane();
+    // Lane j finds row j's ranges (lane 3 repeats row 2), all at once.
+    const RowRanges r = row_ranges(a, cx, cy, (l < 2 ? l : 2) - 1);
+    const uint32_t lo[3][2] = {{quad_bcast<0>(r.s1), quad_bcast<0>(r.s2)},
+                               {quad_bcast<1>(r.s1), quad_bcast<1>(r.s2)},
+                               {quad_bcast<2>(r.s1), quad_bcast<2>(r.s2)}};
+    const uint32_t hi[3][2] = {{quad_bcast<0>(r.e1), quad_bcast<0>(r.e2)},
+                               {quad_bcast<1>(r.e1), quad_bcast<1>(r.e2)},
+                               {quad_bcast<2>(r.e1), quad_bcast<2>(r.e2)}};
+    // Positions of candidate q + l of a range ending at end (p's past it).
+    auto at = [&](uint32_t q, uint32_t end, float &x, float &y) {
+        const uint32_t k = q + l < end ? q + l : (uint32_t)p;
+        x = a.xs[k];
+        y = a.ys[k];
+    };
+    auto scan = [&](uint32_t q, uint32_t end, auto &&d2_of) {
+        for (; q < end; q += 4) {
+            float x, y;
+            at(q, end, x, y);
+            f(q + l, q + l < end, d2_of(x, y));
+        }
+    };
+    visit_rows(
+        a, p, cx, cy, lo, hi,
+        [&](auto &&d2_of) {  // the first candidates of the three rows loaded together
+            float x[3], y[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) at(lo[k][0], hi[k][0], x[k], y[k]);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                if (lo[k][0] < hi[k][0])
+                    f(lo[k][0] + l, lo[k][0] + l < hi[k][0], d2_of(x[k], y[k]));
+                scan(lo[k][0] + 4, hi[k][0], d2_of);
+            }
+        },
+        scan);
+}
+
+// The same visit by one lane per particle, for order-bound sums over sets
+// large enough to fill the GPU that way: f(d2) for every candidate.
+template <typename F>
+__device__ __forceinline__ void for_neighbors_serial(const NArgs &a, int p, F &&f) {
+    const uint32_t c = a.sk[p];
+    if (c >= (uint32_t)a.gx * (uint32_t)a.gy) return;
+    const int cx = (int)(c % (uint32_t)a.gx), cy = (int)(c / (uint32_t)a.gx);
+    uint32_t lo[3][2], hi[3][2];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {  // every row's loads before the first is used
+        const RowRanges r = row_ranges(a, cx, cy, k - 1);
+        lo[k][0] = r.s1;
+        lo[k][1] = r.s2;
+        hi[k][0] = r.e1;
+        hi[k][1] = r.e2;
+    }
+    auto scan = [&](uint32_t q, uint32_t end, auto &&d2_of) {
+        const float *xp = a.xs + q, *yp = a.ys + q;
+        for (; q + 4 <= end; q += 4, xp += 4, yp += 4) {
+            const float x0 = xp[0], x1 = xp[1], x2 = xp[2], x3 = xp[3];
+            const float y0 = yp[0], y1 = yp[1], y2 = yp[2], y3 = yp[3];
+            const float e0 = d2_of(x0, y0), e1 = d2_of(x1, y1), e2 = d2_of(x2, y2),
+                        e3 = d2_of(x3, y3);
+            f(e0);
+            f(e1);
+            f(e2);
+            f(e3);
+        }
+        for (; q < end; ++q, ++xp, ++yp) f(d2_of(*xp, *yp));
+    };
+    visit_rows(
+        a, p, cx, cy, lo, hi,
+        [&](auto &&d2_of) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) scan(lo[k][0], hi[k][0], d2_of);
+        },
+        scan);
+}
+
+// 256 threads: 64 particles.
+__device__ __forceinline__ int quad_particle() {
+    return (int)(blockIdx.x * (blockDim.x >> 2) + (threadIdx.x >> 2));
+}
+
+__global__ __launch_bounds__(256) void k_nbr_count(NArgs a, uint32_t *__restrict__ counts) {
+    const int p = quad_particle();
+    if (p >= a.n) return;
+    uint32_t c = 0;
+    for_neighbors(a, p, [&](uint32_t q, bool ok, float d2) {
+        c += ok && d2 < a.r2 && (int)q != p ? 1u : 0u;
+    });
+    c = quad_total(c);
+    const uint32_t i = a.id((uint32_t)p);
+    if (quad_lane() == 0 && i < (uint32_t)a.n) counts[i] = c;
+}
+
+__global__ __launch_bounds__(256) void k_nbr_count_serial(NArgs a, uint32_t *__restrict__ counts) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= a.n) return;
     uint32_t c = 0;
-    for_neighbors(a, p, [&](uint32_t q, float d2) { c += d2 < a.r2 && (int)q != p ? 1u : 0u; });
+    for_neighbors_serial(a, p, [&](float d2) { c += d2 < a.r2 ? 1u : 0u; });
     const uint32_t i = a.id((uint32_t)p);
-    if (i < (uint32_t)a.n) counts[i] = c;
+    if (i < (uint32_t)a.n) counts[i] = c ? c - 1u : 0u;  // without p itself, as k_density
 }
 
-__global__ void k_nbr_fill(NArgs a, const uint32_t *__restrict__ offsets, uint32_t *__restrict__ nbr,
-                           size_t capacity) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void k_nbr_fill(NArgs a, const uint32_t *__restrict__ offsets,
+                                                  uint32_t *__restrict__ nbr, size_t capacity) {
+    const int p = quad_particle();
     if (p >= a.n) return;
     const uint32_t i = a.id((uint32_t)p);
     if (i >= (uint32_t)a.n) return;
+    const uint32_t below = (1u << quad_lane()) - 1u;
     size_t o = offsets[i];
-    for_neighbors(a, p, [&](uint32_t q, float d2) {
-        if (d2 < a.r2 && (int)q != p) {
-            if (o < capacity) nbr[o] = a.id(q);
-            ++o;
-        }
+    for_neighbors(a, p, [&](uint32_t q, bool ok, float d2) {
+        const bool keep = ok && d2 < a.r2 && (int)q != p;
+        const uint32_t vote = quad_vote(keep);
+        const size_t to = o + __popc(vote & below);
+        if (keep && to < capacity) nbr[to] = a.id(q);
+        o += __popc(vote);
     });
 }
 
 // The same lists by sorted position (order null), written through LDS: the
-// lists of a wave's 64 consecutive particles are one contiguous block of the
+// lists of a wave's 16 consecutive particles are one contiguous block of the
 // output, so each wave gathers its entries in an LDS window of kFillWin
-// slots and then writes the window out with consecutive lanes (a lane's
-// own list would otherwise go out as one scattered word per store).  A
-// block larger than the window takes further traversals, one per window.
-// Waves work independently: the LDS handoff is within one wave, whose LDS
-// accesses complete in order.  3072 slots hold a wave's lists at about 48
-// neighbours per particle in one traversal (48 KB per workgroup).
-constexpr int kFillWin = 3072;
+// slots and then writes the window out with consecutive lanes.  A block larger
+// than the window takes further traversals, one per window.  Waves work
+// independently: the LDS handoff is within one wave, whose LDS accesses
+// complete in order.  1024 slots hold a wave's lists at 64 neighbours per
+// particle in one traversal (16 KB per workgroup).
+constexpr int kFillWin = 1024;
 __global__ __launch_bounds__(256) void k_nbr_fill_lds(NArgs a, const uint32_t *__restrict__ offsets,
                                                       const uint32_t *__restrict__ counts,
                                                       uint32_t *__restrict__ nbr, size_t capacity) {
     __shared__ uint32_t win[4][kFillWin];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    const int pw = blockIdx.x * blockDim.x + wave * 64;  // the wave's first particle
-    if (pw >= a.n) return;                              // the whole wave is past the end
-    const int plast = min(pw + 63, a.n - 1);
+    const int p = quad_particle();
+    const int pw = blockIdx.x * (blockDim.x >> 2) + wave * 16;  // the wave's first particle
+    if (pw >= a.n) return;                                     // the whole wave is past the end
+    const int plast = min(pw + 15, a.n - 1);
+    const uint32_t below = (1u << quad_lane()) - 1u;
     const size_t base = offsets[pw], end = (size_t)offsets[plast] + counts[plast];
     uint32_t *buf = win[wave];
     for (size_t w0 = base; w0 < end; w0 += kFillWin) {
         if (p < a.n) {
             size_t o = offsets[p];
-            for_neighbors(a, p, [&](uint32_t q, float d2) {
-                if (d2 < a.r2 && (int)q != p) {
-                    if (o >= w0 && o < w0 + kFillWin) buf[o - w0] = q;
-                    ++o;
-                }
+            for_neighbors(a, p, [&](uint32_t q, bool ok, float d2) {
+                const bool keep = ok && d2 < a.r2 && (int)q != p;
+                const uint32_t vote = quad_vote(keep);
+                const size_t to = o + __popc(vote & below);
+                if (keep && to >= w0 && to < w0 + kFillWin) buf[to - w0] = q;
+                o += __popc(vote);
             });
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -543,24 +674,43 @@ __global__ __launch_bounds__(256) void k_nbr_fill_lds(NArgs a, const uint32_t *_
 // with d2 < r^2.  A rejected candidate adds +0 (t clamped at 0), which leaves
 // S unchanged, so the loop does not branch.  All terms are positive: S is
 // within (m - 1) u of the exact sum of its m rounded terms.
-__global__ void k_density(NArgs a, float mc, float *__restrict__ rho,
-                          uint32_t *__restrict__ counts) {
+__device__ __forceinline__ void store_density(const NArgs &a, int p, float rho_p, uint32_t cnt,
+                                              float *rho, uint32_t *counts) {
+    const uint32_t i = a.id((uint32_t)p);
+    if (i >= (uint32_t)a.n) return;
+    rho[i] = rho_p;
+    // A finite p met itself (d2 = 0) and counted it; a non-finite p counted
+    // nothing (every d2 it forms is NaN or Inf), as k_nbr_count.
+    if (counts) counts[i] = cnt ? cnt - 1u : 0u;
+}
+
+__global__ __launch_bounds__(256) void k_density(NArgs a, float mc, float *__restrict__ rho,
+                                                 uint32_t *__restrict__ counts) {
+    const int p = quad_particle();
+    if (p >= a.n) return;
+    float sum = 0.0f;
+    uint32_t cnt = 0;
+    for_neighbors(a, p, [&](uint32_t, bool ok, float d2) {
+        const float t = ok ? fmaxf(a.r2 - d2, 0.0f) : 0.0f;
+        sum = quad_add(sum, t * t * t);
+        cnt += ok && d2 < a.r2 ? 1u : 0u;
+    });
+    cnt = quad_total(cnt);
+    if (quad_lane() == 0) store_density(a, p, mc * sum, cnt, rho, counts);
+}
+
+__global__ __launch_bounds__(256) void k_density_serial(NArgs a, float mc, float *__restrict__ rho,
+                                                        uint32_t *__restrict__ counts) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= a.n) return;
     float sum = 0.0f;
     uint32_t cnt = 0;
-    for_neighbors(a, p, [&](uint32_t, float d2) {
+    for_neighbors_serial(a, p, [&](float d2) {
         const float t = fmaxf(a.r2 - d2, 0.0f);
         sum += t * t * t;
         cnt += d2 < a.r2 ? 1u : 0u;
     });
-    const uint32_t i = a.id((uint32_t)p);
-    if (i < (uint32_t)a.n) {
-        rho[i] = mc * sum;
-        // A finite p met itself (d2 = 0) and counted it; a non-finite p
-        // counted nothing (every d2 it forms is NaN or Inf), as k_nbr_count.
-        if (counts) counts[i] = cnt ? cnt - 1u : 0u;
-    }
+    store_density(a, p, mc * sum, cnt, rho, counts);
 }
 
 // A position wrapped into [0, n): unchanged when already inside (the
@@ -640,34 +790,42 @@ struct Staged {
     int on;
 };
 
+// The passes take 256 particles a workgroup, QUAD lanes (1 or 4) each.
+constexpr int kPbfParticles = 256;
+template <int QUAD>
+__device__ __forceinline__ int pbf_particle() {
+    return (int)(blockIdx.x * kPbfParticles + threadIdx.x / QUAD);
+}
+
 template <bool WITH_LAMBDA>
 __device__ __forceinline__ void stage_windows(const PbfArgs &b, Staged &st) {
-    if (threadIdx.x == 0) {
-        const int p0 = blockIdx.x * blockDim.x;
-        const int pl = min(p0 + (int)blockDim.x, b.n) - 1;
+    if (threadIdx.x < 64) {  // one wavefront; lane k finds row k's window (lanes past 2 repeat row 2)
+        const int p0 = blockIdx.x * kPbfParticles;
+        const int pl = min(p0 + kPbfParticles, b.n) - 1;
         const uint32_t c0 = b.sk[p0], c1 = b.sk[pl];
         const int cy = (int)(c0 / (uint32_t)b.gx), cx0 = (int)(c0 % (uint32_t)b.gx),
                   cx1 = (int)(c1 % (uint32_t)b.gx);
-        int on = (int)(c1 / (uint32_t)b.gx) == cy && cy >= 1 && cy <= b.gy - 2 && cx0 >= 1 &&
-                 cx1 <= b.gx - 2 && c0 < (uint32_t)b.gx * (uint32_t)b.gy &&
-                 c1 < (uint32_t)b.gx * (uint32_t)b.gy;
-        uint32_t ws[3] = {0, 0, 0}, len[3] = {0, 0, 0};
+        const bool on = (int)(c1 / (uint32_t)b.gx) == cy && cy >= 1 && cy <= b.gy - 2 && cx0 >= 1 &&
+                        cx1 <= b.gx - 2 && c0 < (uint32_t)b.gx * (uint32_t)b.gy &&
+                        c1 < (uint32_t)b.gx * (uint32_t)b.gy;
+        uint32_t w = 0, len = 0;
         if (on) {
-            for (int k = 0; k < 3; ++k) {
-                const uint32_t row = (uint32_t)((cy - 1 + k) * b.gx);
-                ws[k] = b.cstart[row + cx0 - 1];
-                const uint32_t we = b.cend[row + cx1 + 1];
-                len[k] = we > ws[k] ? we - ws[k] : 0u;
-            }
-            on = len[0] + len[1] + len[2] <= (uint32_t)kStage;
+            const uint32_t row = (uint32_t)((cy - 1 + min((int)threadIdx.x, 2)) * b.gx);
+            w = b.cstart[row + cx0 - 1];
+            const uint32_t we = b.cend[row + cx1 + 1];
+            len = we > w ? we - w : 0u;
         }
-        st.w0 = ws[0];
-        st.w1 = ws[1];
-        st.w2 = ws[2];
-        st.len0 = len[0];
-        st.len01 = len[0] + len[1];
-        st.len012 = len[0] + len[1] + len[2];
-        st.on = on;
+        const uint32_t len0 = quad_bcast<0>(len), len1 = quad_bcast<1>(len), len2 = quad_bcast<2>(len);
+        const uint32_t w1 = quad_bcast<1>(w), w2 = quad_bcast<2>(w);
+        if (threadIdx.x == 0) {
+            st.w0 = w;
+            st.w1 = w1;
+            st.w2 = w2;
+            st.len0 = len0;
+            st.len01 = len0 + len1;
+            st.len012 = len0 + len1 + len2;
+            st.on = on && len0 + len1 + len2 <= (uint32_t)kStage;
+        }
     }
     __syncthreads();
     if (!st.on) return;
@@ -695,42 +853,47 @@ __device__ __forceinline__ uint32_t staged_slot(const Staged &st, uint32_t q) {
     return (uint32_t)kStage;
 }
 
-// Every listed neighbour q of p, in list order: f(q, dx, dy, d2, slot) with
+// Every listed neighbour of p, in list order: f(q, slot, ok, dx, dy, d2) with
 // (dx, dy) = x_q - x_p, periodic (the lists were found at the start; the
-// positions have moved since) and slot q's LDS slot (kStage: not staged).
-// Loads are issued eight at a time.
-template <typename F>
+// positions have moved since), slot q's LDS slot (kStage: not staged), ok false
+// past the list's end (q is then p).  QUAD = 4: four at a time on the quad's
+// lanes, the entries of two steps loaded together.  QUAD = 1: eight loaded
+// together, and the list's last few in fours.
+template <int QUAD, typename F>
 __device__ __forceinline__ void for_listed(const PbfArgs &b, const Staged &st, int p, F &&f) {
     const float px = b.xs[p], py = b.ys[p];
     const uint32_t o = b.noff[p], c = b.ncnt[p];
     const bool on = st.on;
-    auto one = [&](uint32_t q, uint32_t slot, float ox, float oy) {
-        const float dx = periodic_diff(ox, px, b.W, b.half_w);
-        const float dy = periodic_diff(oy, py, b.H, b.half_h);
-        f(q, slot, dx, dy, dx * dx + dy * dy);
-    };
-    constexpr int kB = 8;  // neighbours whose loads are in flight together
-    uint32_t k = 0;
-    for (; k + kB <= c; k += kB) {
-        uint32_t q[kB], sl[kB];
-        float x[kB], y[kB];
+    const uint32_t l = QUAD == 4 ? (uint32_t)quad_lane() : 0u;
+    // n steps from entry k on; all of them listed unless masked.
+    auto batch = [&](uint32_t k, auto n, auto masked) {
+        constexpr int N = decltype(n)::value;
+        uint32_t q[N], sl[N];
+        float x[N], y[N];
+        auto listed = [&](int j) { return !decltype(masked)::value || k + QUAD * j + l < c; };
 #pragma unroll
-        for (int j = 0; j < kB; ++j) q[j] = b.nbr[o + k + j];
+        for (int j = 0; j < N; ++j) q[j] = listed(j) ? b.nbr[o + k + QUAD * j + l] : (uint32_t)p;
 #pragma unroll
-        for (int j = 0; j < kB; ++j) {
+        for (int j = 0; j < N; ++j) {
             sl[j] = on ? staged_slot(st, q[j]) : (uint32_t)kStage;
             const bool lds = sl[j] < (uint32_t)kStage;
             x[j] = lds ? st.x[lds ? sl[j] : 0] : b.xs[q[j]];
             y[j] = lds ? st.y[lds ? sl[j] : 0] : b.ys[q[j]];
         }
 #pragma unroll
-        for (int j = 0; j < kB; ++j) one(q[j], sl[j], x[j], y[j]);
-    }
-    for (; k < c; ++k) {
-        const uint32_t q = b.nbr[o + k];
-        const uint32_t sl = on ? staged_slot(st, q) : (uint32_t)kStage;
-        const bool lds = sl < (uint32_t)kStage;
-        one(q, sl, lds ? st.x[lds ? sl : 0] : b.xs[q], lds ? st.y[lds ? sl : 0] : b.ys[q]);
+        for (int j = 0; j < N; ++j) {
+            const float dx = periodic_diff(x[j], px, b.W, b.half_w);
+            const float dy = periodic_diff(y[j], py, b.H, b.half_h);
+            f(q[j], sl[j], listed(j), dx, dy, dx * dx + dy * dy);
+        }
+    };
+    uint32_t k = 0;
+    if constexpr (QUAD == 4) {
+        for (; k + 4 < c; k += 8) batch(k, std::integral_constant<int, 2>{}, std::true_type{});
+        if (k < c) batch(k, std::integral_constant<int, 1>{}, std::true_type{});
+    } else {
+        for (; k + 8 <= c; k += 8) batch(k, std::integral_constant<int, 8>{}, std::false_type{});
+        for (; k < c; k += 4) batch(k, std::integral_constant<int, 4>{}, std::true_type{});
     }
 }
 
@@ -744,9 +907,15 @@ __device__ __forceinline__ float spiky_w(const PbfArgs &b, float d2) {
     return (d2 > 0.0f && d2 < b.h2) ? w : 0.0f;
 }
 
+// A term of an order-bound sum: the quad's four in lane order, or this lane's.
+template <int QUAD>
+__device__ __forceinline__ float add_terms(float s, float t) {
+    return QUAD == 4 ? quad_add(s, t) : s + t;
+}
+
 // Block-wide FP64 sum (thread 0 gets it): wave shuffles, then the waves in order.
 __device__ __forceinline__ double block_sum(double v) {
-    __shared__ double part[4];
+    __shared__ double part[16];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
@@ -757,49 +926,50 @@ __device__ __forceinline__ double block_sum(double v) {
     return s;
 }
 
-// lambda of iterate b.it and the block sums of C^2 (256 threads).
-__global__ __launch_bounds__(256) void k_pbf_lambda(PbfArgs b) {
+// lambda of iterate b.it and the block sums of C^2.  Per listed neighbour the
+// two passes do about 85 operations, 27 of them the correctly rounded square
+// root and division.
+template <int QUAD>
+__global__ __launch_bounds__(kPbfParticles *QUAD) void k_pbf_lambda(PbfArgs b) {
     if (b.ctl->done) return;  // the same verdict for every thread
     __shared__ Staged st;
     stage_windows<false>(b, st);
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    const int p = pbf_particle<QUAD>();
     double c2 = 0.0;
     if (p < b.n) {
         float S = b.h2 * b.h2 * b.h2;  // p itself
         float gx = 0.0f, gy = 0.0f, g2 = 0.0f;
-        for_listed(b, st, p, [&](uint32_t, uint32_t, float dx, float dy, float d2) {
-            const float t2 = fmaxf(b.h2 - d2, 0.0f);
-            S += t2 * t2 * t2;
-            const float w = spiky_w(b, d2);
+        for_listed<QUAD>(b, st, p, [&](uint32_t, uint32_t, bool ok, float dx, float dy, float d2) {
+            const float t2 = ok ? fmaxf(b.h2 - d2, 0.0f) : 0.0f;
+            S = add_terms<QUAD>(S, t2 * t2 * t2);
+            const float w = spiky_w(b, d2);  // 0 past the list's end, where d2 = 0
             const float vx = w * dx, vy = w * dy;
-            gx += vx;
-            gy += vy;
-            g2 += vx * vx + vy * vy;
+            gx = add_terms<QUAD>(gx, vx);
+            gy = add_terms<QUAD>(gy, vy);
+            g2 = add_terms<QUAD>(g2, vx * vx + vy * vy);
         });
         const float rho = b.mc * S;
         const float C = rho / b.rho0 - 1.0f;
         const float denom = (gx * gx + gy * gy + g2) / b.r0sq + b.eps;
-        b.lambda[p] = -C / denom;
-        c2 = (double)C * (double)C;
+        if (QUAD == 1 || quad_lane() == 0) {
+            b.lambda[p] = -C / denom;
+            c2 = (double)C * (double)C;
+        }
     }
     const double s = block_sum(c2);
     if (threadIdx.x == 0) b.part[(size_t)b.it * b.nblocks + blockIdx.x] = s;
 }
 
 // Folds iterate b.it's block sums (one block of 1024: strided sums in block
-// order, then the waves in order) and decides whether it has converged.
+// order, then the waves in order) and decides whether it has converged.  (A
+// fold by the last workgroup of k_pbf_lambda measured slower: the device-scope
+// fence every workgroup then needs writes its L2 back.)
 __global__ __launch_bounds__(1024) void k_pbf_check(PbfArgs b) {
-    __shared__ double part[16];
     if (b.ctl->done) return;
     double v = 0.0;
     for (int k = threadIdx.x; k < b.nblocks; k += 1024) v += b.part[(size_t)b.it * b.nblocks + k];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
-    __syncthreads();
+    const double s = block_sum(v);
     if (threadIdx.x == 0) {
-        double s = 0.0;
-        for (int k = 0; k < 16; ++k) s += part[k];
         b.res[b.it] = s;
         if (s <= b.tol2n) {
             b.ctl->done = 1;
@@ -809,21 +979,23 @@ __global__ __launch_bounds__(1024) void k_pbf_check(PbfArgs b) {
 }
 
 // The update of iterate b.it into the next iterate (nx, ny).
-__global__ __launch_bounds__(256) void k_pbf_delta(PbfArgs b) {
+template <int QUAD>
+__global__ __launch_bounds__(kPbfParticles *QUAD) void k_pbf_delta(PbfArgs b) {
     if (b.ctl->done) return;
     __shared__ Staged st;
     stage_windows<true>(b, st);
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    const int p = pbf_particle<QUAD>();
     if (p >= b.n) return;
     const float lp = b.lambda[p];
     float ax = 0.0f, ay = 0.0f;
-    for_listed(b, st, p, [&](uint32_t q, uint32_t slot, float dx, float dy, float d2) {
+    for_listed<QUAD>(b, st, p, [&](uint32_t q, uint32_t slot, bool, float dx, float dy, float d2) {
         const float w = spiky_w(b, d2);
         const bool lds = slot < (uint32_t)kStage;
         const float s = lp + (lds ? st.l[lds ? slot : 0] : b.lambda[q]);
-        ax += s * (w * dx);
-        ay += s * (w * dy);
+        ax = add_terms<QUAD>(ax, s * (w * dx));
+        ay = add_terms<QUAD>(ay, s * (w * dy));
     });
+    if (QUAD == 4 && quad_lane() != 0) return;
     b.nx[p] = wrap_pos(b.xs[p] + -(ax / b.rho0), b.W);
     b.ny[p] = wrap_pos(b.ys[p] + -(ay / b.rho0), b.H);
 }
@@ -850,6 +1022,17 @@ __global__ void k_pbf_init(PbfCtl *ctl, double *res, int nres) {
 }
 
 int grid_for(int n) { return (n + 255) / 256; }
+// Particles from which the density and the counts take one lane each instead
+// of four: 4 wavefronts for every SIMD then.  Density with counts, one lane
+// against four, us: 65,536 particles of 20 neighbours 14.2 / 9.9, 131,072
+// 14.9 / 12.0, 262,144 17.8 / 17.9, 1,048,576 41.3 / 60.8.
+constexpr int kSerialFrom = 1 << 18;
+// The same line for the constraint solve's passes.  4 iterations, one lane
+// against four, us: 65,536 particles of 7 / 37 neighbours 135 / 266 against
+// 90 / 155, 262,144 181 / 423 against 168 / 362, 1,048,576 442 / 1119 against
+// 547 / 1148.
+constexpr int kPbfSerialFrom = 3 << 17;
+int quad_grid(int n) { return (n + 63) / 64; }  // 256 threads, four a particle
 
 // The digit plan for keys below ncells: the fewest passes, 8-bit digits
 // where they suffice for that many passes, else 10-bit.
@@ -958,10 +1141,10 @@ int lists_from_counts(const pfs_ngrid *g, const NArgs &a, const uint32_t *counts
                                               std::to_string(nbr_capacity) + " < " +
                                               std::to_string(h_total));
     if (a.order)
-        hipLaunchKernelGGL(k_nbr_fill, dim3(grid_for(g->n)), dim3(256), 0, s, a, offsets, nbr,
+        hipLaunchKernelGGL(k_nbr_fill, dim3(quad_grid(g->n)), dim3(256), 0, s, a, offsets, nbr,
                            nbr_capacity);
     else
-        hipLaunchKernelGGL(k_nbr_fill_lds, dim3(grid_for(g->n)), dim3(256), 0, s, a, offsets,
+        hipLaunchKernelGGL(k_nbr_fill_lds, dim3(quad_grid(g->n)), dim3(256), 0, s, a, offsets,
                            counts, nbr, nbr_capacity);
     return check_launch("neighbour lists");
 }
@@ -1104,7 +1287,10 @@ int pfs_ngrid_neighbors(const pfs_ngrid *g, const float *xs, const float *ys, co
     hipStream_t s = (hipStream_t)stream;
     SortWs w = sort_ws(ws, g->n);
     const NArgs a = nargs(g, xs, ys, order, w.k0, cell_start, cell_end);
-    hipLaunchKernelGGL(k_nbr_count, dim3(grid_for(g->n)), dim3(256), 0, s, a, counts);
+    if (g->n < kSerialFrom)
+        hipLaunchKernelGGL(k_nbr_count, dim3(quad_grid(g->n)), dim3(256), 0, s, a, counts);
+    else
+        hipLaunchKernelGGL(k_nbr_count_serial, dim3(grid_for(g->n)), dim3(256), 0, s, a, counts);
     if (!nbr) return scan_exclusive(counts, offsets, g->n, total, w.sums, s);  // no lists
     return lists_from_counts(g, a, counts, offsets, nbr, nbr_capacity, total, w, s);
 }
@@ -1182,6 +1368,7 @@ int pfs_pbf_solve(const pfs_ngrid *g, float *xs, float *ys, const uint32_t *cell
     b.nblocks = nb;
     b.tol2n = tol * tol * (double)n;
     float *bx[2] = {xs, w.sx}, *by[2] = {ys, w.sy};
+    const bool quad = n < kPbfSerialFrom;
     hipLaunchKernelGGL(k_pbf_init, dim3(1), dim3(256), 0, s, w.ctl, residuals, max_iters + 1);
     for (int it = 0; it <= max_iters; ++it) {
         b.it = it;
@@ -1189,9 +1376,12 @@ int pfs_pbf_solve(const pfs_ngrid *g, float *xs, float *ys, const uint32_t *cell
         b.ys = by[it & 1];
         b.nx = bx[(it + 1) & 1];
         b.ny = by[(it + 1) & 1];
-        hipLaunchKernelGGL(k_pbf_lambda, dim3(nb), dim3(256), 0, s, b);
+        hipLaunchKernelGGL(quad ? k_pbf_lambda<4> : k_pbf_lambda<1>, dim3(nb),
+                           dim3(kPbfParticles * (quad ? 4 : 1)), 0, s, b);
         hipLaunchKernelGGL(k_pbf_check, dim3(1), dim3(1024), 0, s, b);
-        if (it < max_iters) hipLaunchKernelGGL(k_pbf_delta, dim3(nb), dim3(256), 0, s, b);
+        if (it < max_iters)
+            hipLaunchKernelGGL(quad ? k_pbf_delta<4> : k_pbf_delta<1>, dim3(nb),
+                               dim3(kPbfParticles * (quad ? 4 : 1)), 0, s, b);
     }
     hipLaunchKernelGGL(k_pbf_finish, dim3(nb), dim3(256), 0, s, w.ctl, max_iters, w.sx, w.sy, xs, ys,
                        iters_used, n);
@@ -1214,7 +1404,10 @@ int pfs_ngrid_density(const pfs_ngrid *g, const float *xs, const float *ys, cons
     const double r = g->radius;
     const float coef = (float)(4.0 / (3.14159265358979323846 * r * r * r * r * r * r * r * r));
     const float mc = mass * coef;
-    hipLaunchKernelGGL(k_density, dim3(grid_for(g->n)), dim3(256), 0, s, a, mc, rho, counts);
+    if (g->n < kSerialFrom)
+        hipLaunchKernelGGL(k_density, dim3(quad_grid(g->n)), dim3(256), 0, s, a, mc, rho, counts);
+    else
+        hipLaunchKernelGGL(k_density_serial, dim3(grid_for(g->n)), dim3(256), 0, s, a, mc, rho, counts);
     return check_launch("density");
 }
 

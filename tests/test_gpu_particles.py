@@ -87,6 +87,14 @@ def test_lists_and_density_across_the_wrap_at_a_corner():
     assert ng.g.gx >= 7
 
 
+@pytest.mark.parametrize("n", [(1 << 18) - 1, 1 << 18, (1 << 18) + 65])
+def test_either_side_of_the_lane_rule(n):
+    """Four lanes a particle below 2^18 particles, one from there on (counts
+    and density): domain edges on all sides."""
+    x, y = _positions(n, 420.0, 300.0, seed=n)
+    _check_grid(x, y, 420.0, 300.0, 1.4)
+
+
 def test_clustered_particles_and_empty_cells():
     """Many particles in few cells (long equal-key runs across sort tiles)."""
     rng = np.random.default_rng(11)
@@ -198,6 +206,18 @@ def test_pbf_matches_oracle(iters, stop):
     done = ores >= 0
     np.testing.assert_array_equal(r >= 0, done)
     np.testing.assert_allclose(r[done], ores[done], rtol=1e-12)
+
+
+@pytest.mark.parametrize("n", [(3 << 17) - 1, 3 << 17])
+def test_pbf_either_side_of_the_lane_rule(n):
+    ng, og, rho0 = _pbf_setup(n, 1000.0, 1.5, 13, 130.0)
+    ox, oy, olam, ores, _ = og.pbf(1.0, rho0, 5.0, 2)
+    lam, res, _ = ng.pbf(1.0, rho0, 5.0, 2)
+    torch.cuda.synchronize()
+    assert ng.xs.cpu().numpy().tobytes() == ox.tobytes()
+    assert ng.ys.cpu().numpy().tobytes() == oy.tobytes()
+    assert lam.cpu().numpy().tobytes() == olam.tobytes()
+    np.testing.assert_allclose(res.cpu().numpy(), ores, rtol=1e-12)
 
 
 def test_pbf_on_tracers_and_errors():
