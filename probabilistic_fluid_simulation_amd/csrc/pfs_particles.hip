@@ -776,13 +776,18 @@ struct PbfArgs {
     double tol2n;    // convergence: sum C^2 <= tol^2 * n
 };
 
-// The positions a workgroup's 256 particles gather, staged in LDS.  Their
-// lists lie in the three row windows of their cells' 3x3 blocks: when the
-// particles share one cell row away from the domain's edges, row cy + oy
-// contributes the sorted positions [start(cy + oy, cx_first - 1),
-// end(cy + oy, cx_last + 1)), a few hundred in all.  Staged is uniform over
-// the workgroup; otherwise (several rows, an edge, or more than kStage
-// positions) the gathers go to memory.
+// The positions a workgroup's 256 particles gather, staged in LDS (one lane
+// per particle only; with four, the gathers of a quad lie together and memory
+// is as fast: 262,144 particles of 7 / 37 neighbours, 4 iterations 158 / 350 us
+// against 169 / 361 staged).  Their lists lie in the three row windows of their
+// cells' 3x3 blocks: when the particles share one cell row away from the
+// domain's edges, row cy + oy contributes the sorted positions
+// [start(cy + oy, cx_first - 1), end(cy + oy, cx_last + 1)), a few hundred in
+// all.  `on` is uniform over the workgroup; otherwise (several rows, an edge,
+// more than kStage positions, or lists too short to repay the staging) the
+// gathers go to memory.  1,048,576 particles, 4 iterations, staged against not:
+// 7 neighbours 438 / 402 us, 20 731 / 729, 37 1126 / 1269.
+constexpr uint32_t kStageFrom = 20 * 256;  // list entries of the workgroup
 constexpr int kStage = 2048;
 struct Staged {
     float x[kStage], y[kStage], l[kStage];
@@ -805,7 +810,8 @@ __device__ __forceinline__ void stage_windows(const PbfArgs &b, Staged &st) {
         const uint32_t c0 = b.sk[p0], c1 = b.sk[pl];
         const int cy = (int)(c0 / (uint32_t)b.gx), cx0 = (int)(c0 % (uint32_t)b.gx),
                   cx1 = (int)(c1 % (uint32_t)b.gx);
-        const bool on = (int)(c1 / (uint32_t)b.gx) == cy && cy >= 1 && cy <= b.gy - 2 && cx0 >= 1 &&
+        const uint32_t entries = b.noff[pl] + b.ncnt[pl] - b.noff[p0];
+        const bool on = entries >= kStageFrom && (int)(c1 / (uint32_t)b.gx) == cy && cy >= 1 && cy <= b.gy - 2 && cx0 >= 1 &&
                         cx1 <= b.gx - 2 && c0 < (uint32_t)b.gx * (uint32_t)b.gy &&
                         c1 < (uint32_t)b.gx * (uint32_t)b.gy;
         uint32_t w = 0, len = 0;
@@ -860,10 +866,10 @@ __device__ __forceinline__ uint32_t staged_slot(const Staged &st, uint32_t q) {
 // lanes, the entries of two steps loaded together.  QUAD = 1: eight loaded
 // together, and the list's last few in fours.
 template <int QUAD, typename F>
-__device__ __forceinline__ void for_listed(const PbfArgs &b, const Staged &st, int p, F &&f) {
+__device__ __forceinline__ void for_listed(const PbfArgs &b, const Staged *st, int p, F &&f) {
     const float px = b.xs[p], py = b.ys[p];
     const uint32_t o = b.noff[p], c = b.ncnt[p];
-    const bool on = st.on;
+    const bool on = QUAD == 1 && st->on;
     const uint32_t l = QUAD == 4 ? (uint32_t)quad_lane() : 0u;
     // n steps from entry k on; all of them listed unless masked.
     auto batch = [&](uint32_t k, auto n, auto masked) {
@@ -875,10 +881,16 @@ __device__ __forceinline__ void for_listed(const PbfArgs &b, const Staged &st, i
         for (int j = 0; j < N; ++j) q[j] = listed(j) ? b.nbr[o + k + QUAD * j + l] : (uint32_t)p;
 #pragma unroll
         for (int j = 0; j < N; ++j) {
-            sl[j] = on ? staged_slot(st, q[j]) : (uint32_t)kStage;
-            const bool lds = sl[j] < (uint32_t)kStage;
-            x[j] = lds ? st.x[lds ? sl[j] : 0] : b.xs[q[j]];
-            y[j] = lds ? st.y[lds ? sl[j] : 0] : b.ys[q[j]];
+            sl[j] = (uint32_t)kStage;
+            if constexpr (QUAD == 1) {
+                if (on) sl[j] = staged_slot(*st, q[j]);
+                const bool lds = sl[j] < (uint32_t)kStage;
+                x[j] = lds ? st->x[lds ? sl[j] : 0] : b.xs[q[j]];
+                y[j] = lds ? st->y[lds ? sl[j] : 0] : b.ys[q[j]];
+            } else {
+                x[j] = b.xs[q[j]];
+                y[j] = b.ys[q[j]];
+            }
         }
 #pragma unroll
         for (int j = 0; j < N; ++j) {
@@ -932,8 +944,12 @@ __device__ __forceinline__ double block_sum(double v) {
 template <int QUAD>
 __global__ __launch_bounds__(kPbfParticles *QUAD) void k_pbf_lambda(PbfArgs b) {
     if (b.ctl->done) return;  // the same verdict for every thread
-    __shared__ Staged st;
-    stage_windows<false>(b, st);
+    Staged *st = nullptr;
+    if constexpr (QUAD == 1) {
+        __shared__ Staged shared;
+        st = &shared;
+    }
+    if constexpr (QUAD == 1) stage_windows<false>(b, *st);
     const int p = pbf_particle<QUAD>();
     double c2 = 0.0;
     if (p < b.n) {
@@ -982,16 +998,26 @@ __global__ __launch_bounds__(1024) void k_pbf_check(PbfArgs b) {
 template <int QUAD>
 __global__ __launch_bounds__(kPbfParticles *QUAD) void k_pbf_delta(PbfArgs b) {
     if (b.ctl->done) return;
-    __shared__ Staged st;
-    stage_windows<true>(b, st);
+    Staged *st = nullptr;
+    if constexpr (QUAD == 1) {
+        __shared__ Staged shared;
+        st = &shared;
+    }
+    if constexpr (QUAD == 1) stage_windows<true>(b, *st);
     const int p = pbf_particle<QUAD>();
     if (p >= b.n) return;
     const float lp = b.lambda[p];
     float ax = 0.0f, ay = 0.0f;
     for_listed<QUAD>(b, st, p, [&](uint32_t q, uint32_t slot, bool, float dx, float dy, float d2) {
         const float w = spiky_w(b, d2);
-        const bool lds = slot < (uint32_t)kStage;
-        const float s = lp + (lds ? st.l[lds ? slot : 0] : b.lambda[q]);
+        float lq;
+        if constexpr (QUAD == 1) {
+            const bool lds = slot < (uint32_t)kStage;
+            lq = lds ? st->l[lds ? slot : 0] : b.lambda[q];
+        } else {
+            lq = b.lambda[q];
+        }
+        const float s = lp + lq;
         ax = add_terms<QUAD>(ax, s * (w * dx));
         ay = add_terms<QUAD>(ay, s * (w * dy));
     });
