@@ -58,22 +58,24 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
     return x;
 }
 
-// Exclusive scan over the block's kThreads threads; *total gets the sum.
-// Uses `sh` (kWaves + 1 words of LDS).
-__device__ __forceinline__ uint32_t block_excl_scan(uint32_t x, uint32_t *sh, uint32_t *total) {
+// Exclusive scan over a block of NT threads; *total gets the sum.  Uses `sh`
+// (NT / 64 + 1 words of LDS).
+template <int NT>
+__device__ __forceinline__ uint32_t excl_scan(uint32_t x, uint32_t *sh, uint32_t *total) {
+    constexpr int NW = NT / 64;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint32_t inc = wave_incl_scan(x);
     if (lane == 63) sh[wave] = inc;
     __syncthreads();
     if (wave == 0) {
-        const uint32_t w = lane < kWaves ? sh[lane] : 0u;
+        const uint32_t w = lane < NW ? sh[lane] : 0u;
         const uint32_t wi = wave_incl_scan(w);
-        if (lane < kWaves) sh[lane] = wi - w;  // exclusive over waves
-        if (lane == kWaves - 1) sh[kWaves] = wi;
+        if (lane < NW) sh[lane] = wi - w;  // exclusive over waves
+        if (lane == NW - 1) sh[NW] = wi;
     }
     __syncthreads();
     const uint32_t out = sh[wave] + inc - x;
-    *total = sh[kWaves];
+    *total = sh[NW];
     __syncthreads();  // sh may be reused by the caller
     return out;
 }
@@ -88,7 +90,7 @@ __global__ __launch_bounds__(kThreads) void k_scan_reduce(const uint32_t *__rest
     for (int k = 0; k < kItems; ++k)
         if (base + k < (size_t)n) s += in[base + k];
     uint32_t total;
-    (void)block_excl_scan(s, sh, &total);
+    (void)excl_scan<kThreads>(s, sh, &total);
     if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
@@ -102,7 +104,7 @@ __global__ __launch_bounds__(kThreads) void k_scan_down(const uint32_t *__restri
     uint32_t before = 0;
     for (int j = threadIdx.x; j < (int)blockIdx.x; j += kThreads) before += sums[j];
     uint32_t offset;
-    (void)block_excl_scan(before, sh, &offset);
+    (void)excl_scan<kThreads>(before, sh, &offset);
     const size_t base = (size_t)blockIdx.x * kTile + (size_t)threadIdx.x * kItems;
     uint32_t v[kItems], s = 0;
 #pragma unroll
@@ -111,7 +113,7 @@ __global__ __launch_bounds__(kThreads) void k_scan_down(const uint32_t *__restri
         s += v[k];
     }
     uint32_t total;
-    uint32_t run = offset + block_excl_scan(s, sh, &total);
+    uint32_t run = offset + excl_scan<kThreads>(s, sh, &total);
 #pragma unroll
     for (int k = 0; k < kItems; ++k) {
         if (base + k < (size_t)n) out[base + k] = run;
@@ -137,8 +139,9 @@ int scan_exclusive(const uint32_t *in, uint32_t *out, int n, uint32_t *grand, ui
 // ---- stable LSD radix sort of (key, value) pairs ---------------------------
 // Digits of RB bits (8 or 10).  The histogram of block b is stored digit
 // major, hist[d * nb + b]; each digit's row is then scanned on its own
-// (k_digit_rows), and the scatter adds the digit's base, the exclusive scan
-// of the row totals, which every scatter block forms for itself.
+// (k_digit_rows; up to kFewTiles tiles every scatter block adds its columns
+// up itself), and the scatter adds the digit's base, the exclusive scan of the
+// row totals, which every scatter block forms for itself.
 
 // Cell of a position in [0, W): (int)(x * kx) with kx = gx / W (float),
 // clamped into the grid.
@@ -153,22 +156,26 @@ struct CellKeyArgs {  // the first pass computes the keys from the positions
     int gx, gy;
 };
 
+// The sort's tiles: NT threads of kItems keys each.
+template <int NT>
+constexpr int sort_tile() {
+    return NT * kItems;
+}
+
 // Block histograms of one digit.  With FROM_XY the keys are made here from
 // the positions, cy * gx + cx, and written to `keys`.
-template <int RB, bool FROM_XY>
-__global__ __launch_bounds__(kThreads) void k_radix_hist(const uint32_t *__restrict__ kin,
-                                                         CellKeyArgs ck,
-                                                         uint32_t *__restrict__ keys, int n,
-                                                         int shift, uint32_t *__restrict__ hist,
-                                                         int nb) {
+template <int RB, int NT, bool FROM_XY>
+__global__ __launch_bounds__(NT) void k_radix_hist(const uint32_t *__restrict__ kin, CellKeyArgs ck,
+                                                   uint32_t *__restrict__ keys, int n, int shift,
+                                                   uint32_t *__restrict__ hist, int nb) {
     constexpr int R = 1 << RB;
     __shared__ uint32_t h[R];
-    for (int d = threadIdx.x; d < R; d += kThreads) h[d] = 0;
+    for (int d = threadIdx.x; d < R; d += NT) h[d] = 0;
     __syncthreads();
-    const size_t base = (size_t)blockIdx.x * kTile;
+    const size_t base = (size_t)blockIdx.x * sort_tile<NT>();
 #pragma unroll
     for (int r = 0; r < kItems; ++r) {
-        const size_t i = base + (size_t)r * kThreads + threadIdx.x;
+        const size_t i = base + (size_t)r * NT + threadIdx.x;
         if (i < (size_t)n) {
             uint32_t k;
             if (FROM_XY) {
@@ -181,31 +188,30 @@ __global__ __launch_bounds__(kThreads) void k_radix_hist(const uint32_t *__restr
         }
     }
     __syncthreads();
-    for (int d = threadIdx.x; d < R; d += kThreads) hist[(size_t)d * nb + blockIdx.x] = h[d];
+    for (int d = threadIdx.x; d < R; d += NT) hist[(size_t)d * nb + blockIdx.x] = h[d];
 }
 
-// Block d scans row d of the digit-major histogram (nb block counts)
-// exclusively into the same row of `rows`, and writes the row's total to
-// tot[d].
-__global__ __launch_bounds__(kThreads) void k_digit_rows(const uint32_t *__restrict__ hist,
-                                                         uint32_t *__restrict__ rows,
-                                                         uint32_t *__restrict__ tot, int nb) {
-    __shared__ uint32_t sh[kWaves + 1];
-    const size_t row = (size_t)blockIdx.x * nb;
+// Block d scans row d of the digit-major histogram (nb tile counts)
+// exclusively in place, and writes the row's total to tot[d].
+template <int NT>
+__global__ __launch_bounds__(NT) void k_digit_rows(uint32_t *__restrict__ hist,
+                                                   uint32_t *__restrict__ tot, int nb) {
+    __shared__ uint32_t sh[NT / 64 + 1];
+    uint32_t *row = hist + (size_t)blockIdx.x * nb;
     uint32_t carry = 0;
-    for (int b0 = 0; b0 < nb; b0 += kTile) {
+    for (int b0 = 0; b0 < nb; b0 += sort_tile<NT>()) {
         const int j = b0 + threadIdx.x * kItems;
         uint32_t v[kItems], s = 0;
 #pragma unroll
         for (int k = 0; k < kItems; ++k) {
-            v[k] = j + k < nb ? hist[row + j + k] : 0u;
+            v[k] = j + k < nb ? row[j + k] : 0u;
             s += v[k];
         }
         uint32_t total;
-        uint32_t run = carry + block_excl_scan(s, sh, &total);
+        uint32_t run = carry + excl_scan<NT>(s, sh, &total);
 #pragma unroll
         for (int k = 0; k < kItems; ++k) {
-            if (j + k < nb) rows[row + j + k] = run;
+            if (j + k < nb) row[j + k] = run;
             run += v[k];
         }
         carry += total;
@@ -222,38 +228,34 @@ __device__ __forceinline__ int xcd_block(int i, int nb) {
     return x * q + min(x, r) + (i >> 3);
 }
 
-// Scatter of one pass.  Wave w of block b takes the kItems * 64 keys
-// [b * kTile + w * 256, + 256) in kItems rounds of 64, so the tile's order is
-// (wave, round, lane).  The rank of an item among equal digits is: the
-// digit's base (scan of the row totals) plus its row scan at this block, plus
-// the equal digits of earlier waves (per-wave LDS counts, scanned across
-// waves once), plus those of this wave's earlier rounds (the wave's running
-// count) and of the lanes below it (RB ballots, one per digit bit,
-// intersected).  vin null: the values are the key indices.  xs non-null (the
-// last pass): the positions are gathered into sorted order as well.
-template <int RB>
-__global__ __launch_bounds__(kThreads) void k_radix_scatter(
+// Scatter of one pass.  Wave w of a tile takes its kItems * 64 keys from w *
+// 256 on in kItems rounds of 64, so the tile's order is (wave, round, lane).
+// The rank of an item among equal digits is: the digit's base (scan of the
+// digit totals) plus the earlier tiles' count, plus the equal digits of earlier
+// waves (per-wave LDS counts, scanned across waves once), plus those of this
+// wave's earlier rounds (the wave's running count) and of the lanes below it
+// (RB ballots, one per digit bit, intersected).  vin null: the values are the
+// key indices.  xs non-null (the last pass): the positions are gathered into
+// sorted order as well.  FEW: `rows` is the histogram itself, and each tile
+// adds up its few columns (one launch less).
+constexpr int kFewTiles = 16;
+template <int RB, int NT, bool FEW>
+__global__ __launch_bounds__(NT) void k_radix_scatter(
     const uint32_t *__restrict__ kin, const uint32_t *__restrict__ vin, uint32_t *__restrict__ kout,
     uint32_t *__restrict__ vout, int n, int shift, const uint32_t *__restrict__ rows,
     const uint32_t *__restrict__ tot, int nb, const float *__restrict__ x,
     const float *__restrict__ y, float *__restrict__ xs, float *__restrict__ ys) {
-    constexpr int R = 1 << RB;
-    static_assert(R <= kThreads, "one digit per thread");
-    __shared__ uint32_t wcount[kWaves][R];
+    constexpr int R = 1 << RB, NW = NT / 64, TILE = sort_tile<NT>();
+    constexpr int DPT = R > NT ? R / NT : 1;  // digits per thread, consecutive
+    __shared__ uint32_t wcount[NW][R];
     __shared__ uint32_t gofs[R], loff[R];
-    __shared__ uint32_t lkey[kTile], lval[kTile];
-    __shared__ uint32_t sh[kWaves + 1];
+    __shared__ uint32_t lkey[TILE], lval[TILE];
+    __shared__ uint32_t sh[NW + 1];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int tb = xcd_block(blockIdx.x, nb);  // the tile of this workgroup
-    for (int e = threadIdx.x; e < kWaves * R; e += kThreads) (&wcount[0][0])[e] = 0;
-    {
-        const uint32_t t = threadIdx.x < R ? tot[threadIdx.x] : 0u;
-        uint32_t all;
-        const uint32_t dbase = block_excl_scan(t, sh, &all);  // its barriers also order the clear
-        if (threadIdx.x < R) gofs[threadIdx.x] = dbase + rows[(size_t)threadIdx.x * nb + tb];
-    }
+    const int d0 = (int)threadIdx.x * DPT;     // this thread's digits (none: d0 >= R)
     const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    const size_t base = (size_t)tb * kTile + (size_t)wave * (kItems * 64) + lane;
+    const size_t base = (size_t)tb * TILE + (size_t)wave * (kItems * 64) + lane;
     uint32_t key[kItems], val[kItems], dig[kItems], local[kItems];
 #pragma unroll
     for (int r = 0; r < kItems; ++r) {
@@ -261,6 +263,37 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(
         const bool valid = i < (size_t)n;
         key[r] = valid ? kin[i] : 0u;
         val[r] = valid ? (vin ? vin[i] : (uint32_t)i) : 0u;
+    }
+    for (int e = threadIdx.x; e < NW * R; e += NT) (&wcount[0][0])[e] = 0;
+    {
+        uint32_t t[DPT], before[DPT], s = 0;
+#pragma unroll
+        for (int m = 0; m < DPT; ++m) {
+            t[m] = before[m] = 0;
+            if (d0 + m < R) {
+                const size_t row = (size_t)(d0 + m) * nb;
+                if (FEW) {
+#pragma unroll
+                    for (int b = 0; b < kFewTiles; ++b) {
+                        const uint32_t c = b < nb ? rows[row + b] : 0u;
+                        t[m] += c;
+                        before[m] += b < tb ? c : 0u;
+                    }
+                } else {
+                    t[m] = tot[d0 + m];
+                    before[m] = rows[row + tb];
+                }
+            }
+            s += t[m];
+        }
+        uint32_t all;
+        uint32_t dbase = excl_scan<NT>(s, sh, &all);  // its barriers also order the clear
+#pragma unroll
+        for (int m = 0; m < DPT; ++m)
+            if (d0 + m < R) {
+                gofs[d0 + m] = dbase + before[m];
+                dbase += t[m];
+            }
     }
 #pragma unroll
     for (int r = 0; r < kItems; ++r) {
@@ -286,35 +319,45 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(
         __builtin_amdgcn_wave_barrier();
     }
     __syncthreads();
-    uint32_t dtotal = 0;
-    if (threadIdx.x < R) {  // digit counts of the waves -> exclusive across waves
-        for (int w = 0; w < kWaves; ++w) {
-            const uint32_t c = wcount[w][threadIdx.x];
-            wcount[w][threadIdx.x] = dtotal;
-            dtotal += c;
-        }
-    }
-    // The tile is first put in digit order in LDS (loff[d]: the tile's first
-    // slot of digit d), then written out by consecutive threads, so that each
-    // store instruction covers a few runs of consecutive positions.
+    // Digit counts of the waves -> exclusive across waves; then the tile's
+    // first slot of each digit (loff).  The tile is put in digit order in LDS
+    // and written out by consecutive threads, so that each store instruction
+    // covers a few runs of consecutive positions.
     {
+        uint32_t dt[DPT], s = 0;
+#pragma unroll
+        for (int m = 0; m < DPT; ++m) {
+            dt[m] = 0;
+            if (d0 + m < R)
+                for (int w = 0; w < NW; ++w) {
+                    const uint32_t c = wcount[w][d0 + m];
+                    wcount[w][d0 + m] = dt[m];
+                    dt[m] += c;
+                }
+            s += dt[m];
+        }
         uint32_t all;
-        const uint32_t lo = block_excl_scan(dtotal, sh, &all);
-        if (threadIdx.x < R) loff[threadIdx.x] = lo;
+        uint32_t lo = excl_scan<NT>(s, sh, &all);
+#pragma unroll
+        for (int m = 0; m < DPT; ++m)
+            if (d0 + m < R) {
+                loff[d0 + m] = lo;
+                lo += dt[m];
+            }
         __syncthreads();
     }
 #pragma unroll
     for (int r = 0; r < kItems; ++r) {
         if (base + (size_t)r * 64 >= (size_t)n) continue;
         const uint32_t li = loff[dig[r]] + wcount[wave][dig[r]] + local[r];
-        if (li < (uint32_t)kTile) {  // always: kept as a bound
+        if (li < (uint32_t)TILE) {  // always: kept as a bound
             lkey[li] = key[r];
             lval[li] = val[r];
         }
     }
     __syncthreads();
-    const int count = (int)min((size_t)kTile, (size_t)n - (size_t)tb * kTile);
-    for (int j = threadIdx.x; j < count; j += kThreads) {
+    const int count = (int)min((size_t)TILE, (size_t)n - (size_t)tb * TILE);
+    for (int j = threadIdx.x; j < count; j += NT) {
         const uint32_t k = lkey[j], v = lval[j];
         const uint32_t d = (k >> shift) & (R - 1);
         const uint32_t pos = gofs[d] + ((uint32_t)j - loff[d]);
@@ -330,14 +373,33 @@ __global__ __launch_bounds__(kThreads) void k_radix_scatter(
 }
 
 // ---- grid ------------------------------------------------------------------
-// start[c] = the lower bound of cell c in the sorted keys (binary search;
-// the top levels of every search hit the same few cache lines), which is
-// also end[c - 1]; the last cell ends at n.
-__global__ void k_cell_tables(const uint32_t *__restrict__ sk, int n, uint32_t *__restrict__ start,
-                              uint32_t *__restrict__ end, uint32_t ncells) {
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
+// start[c] = the lower bound of cell c in the sorted keys, which is also
+// end[c - 1]; the last cell ends at n.  Chains of dependent loads bound this,
+// 20 for a binary search of 2^20 keys: two waves of a block of cells find the
+// bounds of its first cell and of the next block's, 64 probes at a time (4
+// loads), and each cell is then searched between them, in L1.  1,000,000 cells
+// and particles: 8.3 -> 6.8 us.
+__global__ __launch_bounds__(256) void k_cell_tables(const uint32_t *__restrict__ sk, int n,
+                                                     uint32_t *__restrict__ start,
+                                                     uint32_t *__restrict__ end, uint32_t ncells) {
+    __shared__ uint32_t bracket[2];
+    const uint32_t c0 = blockIdx.x * 256, c = c0 + threadIdx.x;
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (wave < 2) {
+        const uint32_t want = c0 + wave * 256;
+        uint32_t lo = 0, hi = (uint32_t)n;
+        while (lo < hi) {  // the answer stays in [lo, hi]; hi - lo falls below a 64th
+            const uint32_t step = (hi - lo + 63) >> 6, p = lo + lane * step;
+            const uint32_t less = (uint32_t)__popcll(__ballot(p < hi && sk[p] < want));
+            const uint32_t top = lo + less * step;  // the first probe not below, if in range
+            if (less) lo = top - step + 1;
+            hi = less ? min(hi, top) : lo;
+        }
+        if (lane == 0) bracket[wave] = lo;
+    }
+    __syncthreads();
     if (c >= ncells) return;
-    uint32_t lo = 0, hi = (uint32_t)n;
+    uint32_t lo = bracket[0], hi = bracket[1];
     while (lo < hi) {
         const uint32_t mid = (lo + hi) >> 1;
         if (sk[mid] < c) lo = mid + 1;
@@ -1055,7 +1117,7 @@ int grid_for(int n) { return (n + 255) / 256; }
 constexpr int kSerialFrom = 1 << 18;
 // The same line for the constraint solve's passes.  4 iterations, one lane
 // against four, us: 65,536 particles of 7 / 37 neighbours 135 / 266 against
-// 90 / 155, 262,144 181 / 423 against 168 / 362, 1,048,576 442 / 1119 against
+// 81 / 130, 262,144 181 / 423 against 145 / 327, 1,048,576 438 / 1126 against
 // 547 / 1148.
 constexpr int kPbfSerialFrom = 3 << 17;
 int quad_grid(int n) { return (n + 63) / 64; }  // 256 threads, four a particle
@@ -1076,20 +1138,21 @@ RadixPlan radix_plan(uint32_t ncells) {
 }
 
 // Workspace layout (words): sorted keys (2 buffers), values spare buffer,
-// digit histogram and its row scans (2^10 * nblocks each), digit row totals
-// (2^10), scan block sums.
+// digit histogram (2^11 words for each 4096 keys: four 8-bit rows of 1024-key
+// tiles, or two 10-bit rows of 2048-key ones), digit row totals (2^10), scan
+// block sums.
 struct SortWs {
-    uint32_t *k0, *k1, *v1, *hist, *hscan, *tot, *sums;
+    uint32_t *k0, *k1, *v1, *hist, *tot, *sums;
 };
 size_t hist_words(int n) {
     const size_t nb = (size_t)nblocks_for((size_t)n);
-    return ((size_t)1 << kMaxRadixBits) * (nb ? nb : 1);
+    return ((size_t)2 << kMaxRadixBits) * (nb ? nb : 1);
 }
 size_t sort_ws_words(int n, size_t ncells) {
     const size_t hist = hist_words(n);
-    size_t sums = std::max<size_t>(nblocks_for(hist), nblocks_for((size_t)n));
+    size_t sums = std::max<size_t>(nblocks_for(hist / 2), nblocks_for((size_t)n));
     sums = std::max<size_t>(sums, nblocks_for(ncells));
-    return 3 * (size_t)n + 2 * hist + ((size_t)1 << kMaxRadixBits) + sums + 64;
+    return 3 * (size_t)n + hist + ((size_t)1 << kMaxRadixBits) + sums + 64;
 }
 SortWs sort_ws(void *ws, int n) {  // ws: 4-byte aligned
     uint32_t *p = static_cast<uint32_t *>(ws);
@@ -1098,8 +1161,7 @@ SortWs sort_ws(void *ws, int n) {  // ws: 4-byte aligned
     s.k1 = p + n;
     s.v1 = p + 2 * (size_t)n;
     s.hist = p + 3 * (size_t)n;
-    s.hscan = s.hist + hist_words(n);
-    s.tot = s.hscan + hist_words(n);
+    s.tot = s.hist + hist_words(n);
     s.sums = s.tot + ((size_t)1 << kMaxRadixBits);
     return s;
 }
@@ -1108,6 +1170,60 @@ bool valid_grid(const pfs_ngrid *g) {
     return g && g->n >= 1 && g->gx >= 3 && g->gy >= 3 && g->domain_w > 0 && g->domain_h > 0 &&
            g->radius > 0 && (int64_t)g->gx * g->gy <= ((int64_t)1 << 30) &&
            g->radius <= g->domain_w / g->gx && g->radius <= g->domain_h / g->gy;
+}
+
+// Up to kSmallSort particles the sort's tiles are 1024 keys (8-bit digits)
+// or 2048 (10-bit): 4096-key tiles leave most CUs idle there, and a tile is one
+// long chain.  Both kinds' counts fit the same workspace.  Building the grid
+// of 10,000 / 60,000 / 1,000,000 cells, large -> small tiles: 16,384 particles
+// 29.7 / 31.9 / 41.5 -> 25.5 / 26.2 / 41.3 us; 131,072: 37.7 / 39.3 / 55.2 ->
+// 28.9 / 29.8 / 46.9; 524,288: 46.9 / 47.6 / 65.5 -> 39.8 / 41.2 / 59.4;
+// 786,432: 50.9 / 50.9 / 70.2 -> 50.5 / 52.6 / 77.2, where the large ones stay.
+constexpr int kSmallSort = 1 << 19;
+
+struct SortArgs {
+    int n;
+    const float *x, *y;
+    uint32_t *keys;
+    float *xs, *ys;
+    uint32_t *const *kb, *const *vb;
+    SortWs w;
+    CellKeyArgs ck;
+    hipStream_t s;
+};
+
+template <int RB, int NT>
+void sort_passes(const SortArgs &a, int passes) {
+    const int nb = (a.n + sort_tile<NT>() - 1) / sort_tile<NT>();
+    const uint32_t *kin = a.keys;
+    for (int p = 0; p < passes; ++p) {
+        const int shift = RB * p;
+        const bool last = p + 1 == passes;
+        const uint32_t *vin = p == 0 ? nullptr : a.vb[p & 1];
+        float *oxs = last ? a.xs : nullptr, *oys = last ? a.ys : nullptr;
+        if (p == 0)
+            hipLaunchKernelGGL((k_radix_hist<RB, NT, true>), dim3(nb), dim3(NT), 0, a.s, nullptr, a.ck,
+                               a.keys, a.n, shift, a.w.hist, nb);
+        else
+            hipLaunchKernelGGL((k_radix_hist<RB, NT, false>), dim3(nb), dim3(NT), 0, a.s, kin, a.ck,
+                               nullptr, a.n, shift, a.w.hist, nb);
+        if (nb <= kFewTiles) {
+            hipLaunchKernelGGL((k_radix_scatter<RB, NT, true>), dim3(nb), dim3(NT), 0, a.s, kin, vin,
+                               a.kb[(p + 1) & 1], a.vb[(p + 1) & 1], a.n, shift, a.w.hist, a.w.tot, nb,
+                               a.x, a.y, oxs, oys);
+        } else {
+            if (nb <= sort_tile<256>())
+                hipLaunchKernelGGL(k_digit_rows<256>, dim3(1 << RB), dim3(256), 0, a.s, a.w.hist,
+                                   a.w.tot, nb);
+            else
+                hipLaunchKernelGGL(k_digit_rows<kThreads>, dim3(1 << RB), dim3(kThreads), 0, a.s,
+                                   a.w.hist, a.w.tot, nb);
+            hipLaunchKernelGGL((k_radix_scatter<RB, NT, false>), dim3(nb), dim3(NT), 0, a.s, kin, vin,
+                               a.kb[(p + 1) & 1], a.vb[(p + 1) & 1], a.n, shift, a.w.hist, a.w.tot, nb,
+                               a.x, a.y, oxs, oys);
+        }
+        kin = a.kb[(p + 1) & 1];
+    }
 }
 
 NArgs nargs(const pfs_ngrid *g, const float *xs, const float *ys,
@@ -1246,7 +1362,7 @@ int pfs_ngrid_build(const pfs_ngrid *g, const float *x, const float *y, uint32_t
         return set_error(PFS_ERR_INVALID,
                          "ngrid: workspace not 4-byte aligned or smaller than pfs_ngrid_workspace_bytes()");
     hipStream_t s = (hipStream_t)stream;
-    const int n = g->n, nb = nblocks_for((size_t)n);
+    const int n = g->n;
     const uint32_t ncells = (uint32_t)g->gx * (uint32_t)g->gy;
     SortWs w = sort_ws(ws, n);
 
@@ -1259,39 +1375,11 @@ int pfs_ngrid_build(const pfs_ngrid *g, const float *x, const float *y, uint32_t
     uint32_t *kb[2] = {passes % 2 == 0 ? w.k0 : w.k1, passes % 2 == 0 ? w.k1 : w.k0};
     uint32_t *vb[2] = {passes % 2 == 0 ? order : w.v1, passes % 2 == 0 ? w.v1 : order};
     const CellKeyArgs ck{x, y, g->kx, g->ky, g->gx, g->gy};
-    const uint32_t *kin = keys;
-    for (int p = 0; p < passes; ++p) {
-        const int shift = plan.bits * p;
-        const bool last = p + 1 == passes;
-        const uint32_t *vin = p == 0 ? nullptr : vb[p & 1];
-        float *oxs = last ? xs : nullptr, *oys = last ? ys : nullptr;
-        if (plan.bits == 8) {
-            if (p == 0)
-                hipLaunchKernelGGL((k_radix_hist<8, true>), dim3(nb), dim3(kThreads), 0, s, nullptr,
-                                   ck, keys, n, shift, w.hist, nb);
-            else
-                hipLaunchKernelGGL((k_radix_hist<8, false>), dim3(nb), dim3(kThreads), 0, s, kin,
-                                   ck, nullptr, n, shift, w.hist, nb);
-            hipLaunchKernelGGL(k_digit_rows, dim3(1 << 8), dim3(kThreads), 0, s, w.hist, w.hscan,
-                               w.tot, nb);
-            hipLaunchKernelGGL(k_radix_scatter<8>, dim3(nb), dim3(kThreads), 0, s, kin, vin,
-                               kb[(p + 1) & 1], vb[(p + 1) & 1], n, shift, w.hscan, w.tot, nb, x, y,
-                               oxs, oys);
-        } else {
-            if (p == 0)
-                hipLaunchKernelGGL((k_radix_hist<10, true>), dim3(nb), dim3(kThreads), 0, s, nullptr,
-                                   ck, keys, n, shift, w.hist, nb);
-            else
-                hipLaunchKernelGGL((k_radix_hist<10, false>), dim3(nb), dim3(kThreads), 0, s, kin,
-                                   ck, nullptr, n, shift, w.hist, nb);
-            hipLaunchKernelGGL(k_digit_rows, dim3(1 << 10), dim3(kThreads), 0, s, w.hist, w.hscan,
-                               w.tot, nb);
-            hipLaunchKernelGGL(k_radix_scatter<10>, dim3(nb), dim3(kThreads), 0, s, kin, vin,
-                               kb[(p + 1) & 1], vb[(p + 1) & 1], n, shift, w.hscan, w.tot, nb, x, y,
-                               oxs, oys);
-        }
-        kin = kb[(p + 1) & 1];
-    }
+    const SortArgs sa{n, x, y, keys, xs, ys, kb, vb, w, ck, s};
+    if (plan.bits == 8)
+        n <= kSmallSort ? sort_passes<8, 256>(sa, passes) : sort_passes<8, 1024>(sa, passes);
+    else
+        n <= kSmallSort ? sort_passes<10, 512>(sa, passes) : sort_passes<10, 1024>(sa, passes);
     // Cell tables: the lower bound of every cell (empty ones included) in the
     // sorted keys, left in k0 by the last pass.
     const unsigned cblocks = (unsigned)(((size_t)ncells + 255) / 256);

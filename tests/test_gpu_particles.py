@@ -95,6 +95,33 @@ def test_either_side_of_the_lane_rule(n):
     _check_grid(x, y, 420.0, 300.0, 1.4)
 
 
+@pytest.mark.parametrize("n,W,H", [
+    (16 << 10, 90.0, 70.0), ((16 << 10) + 1, 90.0, 70.0),    # 8-bit digits, 16 / 17 tiles
+    (16 << 11, 500.0, 300.0), ((16 << 11) + 1, 500.0, 300.0),  # 10-bit
+    (1 << 19, 90.0, 70.0), ((1 << 19) + 1, 90.0, 70.0),      # small and large tiles
+    (1 << 19, 500.0, 300.0), ((1 << 19) + 1, 500.0, 300.0),
+    ((1 << 22) + 1, 500.0, 300.0)])                          # 1025 tiles a row
+def test_grid_at_the_edges_of_the_sorts_tiles(n, W, H):
+    """Keys, order and cell tables against a stable argsort; a third of the
+    particles lie in one cell, so that its table's neighbours are far apart."""
+    x, y = _positions(n, W, H, seed=n)
+    x[::3], y[::3] = 40.25, 50.75
+    ng = particles.NeighborGrid(n, W, H, 1.0)
+    ng.build(torch.from_numpy(x).cuda(), torch.from_numpy(y).cuda())
+    g = ng.g
+    cx = np.minimum((x * np.float32(g.kx)).astype(np.int64), g.gx - 1)
+    cy = np.minimum((y * np.float32(g.ky)).astype(np.int64), g.gy - 1)
+    key = cy * g.gx + cx
+    order = np.argsort(key, kind="stable")
+    np.testing.assert_array_equal(_u32(ng.keys), key)
+    np.testing.assert_array_equal(_u32(ng.order), order)
+    cells = np.arange(g.gx * g.gy)
+    np.testing.assert_array_equal(_u32(ng.cell_start), np.searchsorted(key[order], cells))
+    np.testing.assert_array_equal(_u32(ng.cell_end), np.searchsorted(key[order], cells, "right"))
+    np.testing.assert_array_equal(ng.xs.cpu().numpy(), x[order])
+    np.testing.assert_array_equal(ng.ys.cpu().numpy(), y[order])
+
+
 def test_clustered_particles_and_empty_cells():
     """Many particles in few cells (long equal-key runs across sort tiles)."""
     rng = np.random.default_rng(11)
