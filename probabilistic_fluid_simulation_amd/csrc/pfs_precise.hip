@@ -50,8 +50,8 @@
 // which is exactly the reference's step when Kp = Kd (the plain step's
 // contract, see pfs_step.hip).
 //
-// The FP64 twin runs the same contract in double with plain arithmetic, one
-// launch per sweep and given (Kd, Kp): the yardstick the precision form's
+// The FP64 twin runs the same contract in double with plain arithmetic, up to
+// 8 sweeps per launch and given (Kd, Kp): the yardstick the precision form's
 // error is reported against.  With Kd = Kp = K it reproduces the
 // reference's algorithm in double exactly.
 
@@ -61,6 +61,7 @@
 #include <cmath>
 #include <cstring>
 #include <string>
+#include <utility>
 
 #include "pfs.h"
 #include "pfs_internal.h"
@@ -74,7 +75,7 @@ constexpr int kMaxK = PFS_PRECISE_MAX_ITERS;
 
 // ============================ FP64 twin ======================================
 constexpr int kBX = 64, kBY = 4;
-constexpr int kRows = 8;  // rows per thread: a block covers kBX x (kBY * kRows) cells
+constexpr int kRows = 2;  // rows per thread: a block covers kBX x (kBY * kRows) cells
 
 struct Cell {
     int i, j, im, ip, jm, jp;
@@ -100,117 +101,312 @@ __device__ __forceinline__ void for_cells(int w, int h, F &&f) {
     }
 }
 
-// Advection of vp[0,1] (src/fluid.cpp:24-70) into the iterate plane d.
+// Advection of vp[0,1] (src/fluid.cpp:24-70) into the iterate planes u, v.
 __global__ __launch_bounds__(kBX *kBY) void k_t_advect(const double *__restrict__ P,
-                                                      double2 *__restrict__ d, int w, int h,
+                                                      double *__restrict__ u,
+                                                      double *__restrict__ v, int w, int h,
                                                       double dt, double fw, double fh,
                                                       double inv_w, double inv_h, int pow2_w,
                                                       int pow2_h) {
     for_cells(w, h, [&](const Cell &c) {
         const int cell = c.j * w + c.i;
-        const double xp = (double)c.i - div_n(dt * P[4 * cell], fw, inv_w, pow2_w);
-        const double yp = (double)c.j - div_n(dt * P[4 * cell + 1], fh, inv_h, pow2_h);
+        auto at = [&](int k) { return *reinterpret_cast<const Pair<double> *>(P + 4 * k); };
+        const Pair<double> here = at(cell);
+        const double xp = (double)c.i - div_n(dt * here.a, fw, inv_w, pow2_w);
+        const double yp = (double)c.j - div_n(dt * here.b, fh, inv_h, pow2_h);
         const TraceT<double> t = trace(xp, yp, w, h, fw, fh);
-        const int a00 = 4 * (t.j0 * w + t.i0), a10 = 4 * (t.j0 * w + t.i1);
-        const int a01 = 4 * (t.j1 * w + t.i0), a11 = 4 * (t.j1 * w + t.i1);
-        d[cell] = {bilerp(t.sx, t.sy, P[a00], P[a10], P[a01], P[a11]),
-                   bilerp(t.sx, t.sy, P[a00 + 1], P[a10 + 1], P[a01 + 1], P[a11 + 1])};
-    });
-}
-
-// One diffusion sweep (src/fluid.cpp:154-185) on the iterate planes.
-__global__ __launch_bounds__(kBX *kBY) void k_t_diffuse(const double2 *__restrict__ in,
-                                                       double2 *__restrict__ out, int w, int h,
-                                                       double alpha, double beta) {
-    for_cells(w, h, [&](const Cell &c) {
-        const double2 L = in[c.j * w + c.im], R = in[c.j * w + c.ip], T = in[c.jm * w + c.i],
-                      B = in[c.jp * w + c.i], C = in[c.j * w + c.i];
-        out[c.j * w + c.i] = {diffuse_cell(L.x, R.x, T.x, B.x, C.x, alpha, beta),
-                              diffuse_cell(L.y, R.y, T.y, B.y, C.y, alpha, beta)};
+        const Pair<double> f00 = at(t.j0 * w + t.i0), f10 = at(t.j0 * w + t.i1);
+        const Pair<double> f01 = at(t.j1 * w + t.i0), f11 = at(t.j1 * w + t.i1);
+        u[cell] = bilerp(t.sx, t.sy, f00.a, f10.a, f01.a, f11.a);
+        v[cell] = bilerp(t.sx, t.sy, f00.b, f10.b, f01.b, f11.b);
     });
 }
 
 // Divergence of D^Kd (src/fluid.cpp:221-237) into b, and the pressure start
 // (tmp[2] for even Kd, vp[2] for odd) into iterate plane 0.
-__global__ __launch_bounds__(kBX *kBY) void k_t_divergence(const double2 *__restrict__ dk,
-                                                          const double *__restrict__ P,
-                                                          const double *__restrict__ Q,
+__global__ __launch_bounds__(kBX *kBY) void k_t_divergence(const double *__restrict__ u,
+                                                          const double *__restrict__ v,
+                                                          const double *__restrict__ start,
                                                           double *__restrict__ b,
                                                           double *__restrict__ p0, int w, int h,
-                                                          double gamma, int kd_even) {
+                                                          double gamma) {
     for_cells(w, h, [&](const Cell &c) {
         const int cell = c.j * w + c.i;
-        const double uR = dk[c.j * w + c.ip].x - dk[c.j * w + c.im].x;
-        const double vT = dk[c.jp * w + c.i].y - dk[c.jm * w + c.i].y;
+        const double uR = u[c.j * w + c.ip] - u[c.j * w + c.im];
+        const double vT = v[c.jp * w + c.i] - v[c.jm * w + c.i];
         b[cell] = gamma * (uR + vT);
-        p0[cell] = kd_even ? Q[4 * cell + 2] : P[4 * cell + 2];
-    });
-}
-
-// Pressure sweep (src/fluid.cpp:240-257): p^s from p^(s-1).
-__global__ __launch_bounds__(kBX *kBY) void k_t_pressure(const double *__restrict__ in,
-                                                        double *__restrict__ out,
-                                                        const double *__restrict__ b, int w,
-                                                        int h) {
-    for_cells(w, h, [&](const Cell &c) {
-        out[c.j * w + c.i] = pressure_cell(in[c.j * w + c.im], in[c.j * w + c.ip],
-                                           in[c.jm * w + c.i], in[c.jp * w + c.i],
-                                           b[c.j * w + c.i]);
+        p0[cell] = start[4 * cell + 2];
     });
 }
 
 // Gradient subtraction with p^Kp (src/fluid.cpp:269-296) and the output
-// contract; iterate k lives in plane k % 3.
+// contract.
 __global__ __launch_bounds__(kBX *kBY) void k_t_finalize(
-    double *__restrict__ P, double *__restrict__ Q, const double2 *__restrict__ dk,
-    const double2 *__restrict__ dkm1, const double *p0, const double *p1, const double *p2,
-    const double *__restrict__ b, int w, int h, double dt, int kd, int kp) {
-    const double *pk = kp % 3 == 0 ? p0 : kp % 3 == 1 ? p1 : p2;
-    const double *pkm1 = kp % 3 == 1 ? p0 : kp % 3 == 2 ? p1 : p2;
+    double *__restrict__ P, double *__restrict__ Q, const double *__restrict__ eu,
+    const double *__restrict__ ev, const double *__restrict__ pk, const double *__restrict__ pkm1,
+    const double *__restrict__ b, int w, int h, double dt) {
     for_cells(w, h, [&](const Cell &c) {
         const int cell = c.j * w + c.i;
         const double pL = pk[c.j * w + c.im], pR = pk[c.j * w + c.ip];
         const double pT = pk[c.jm * w + c.i], pB = pk[c.jp * w + c.i];
         const double gradX = (pR - pL) * dt / 2.0;
         const double gradY = (pB - pT) * dt / 2.0;
-        const double2 e = (kd % 2 == 0) ? dk[cell] : dkm1[cell];
-        const double bb = b[cell];
-        P[4 * cell] = e.x - gradX;
-        P[4 * cell + 1] = e.y - gradY;
+        const double ex = eu[cell], ey = ev[cell], bb = b[cell];
+        P[4 * cell] = ex - gradX;
+        P[4 * cell + 1] = ey - gradY;
         P[4 * cell + 2] = pkm1[cell];
         P[4 * cell + 3] = bb;
-        Q[4 * cell] = e.x;
-        Q[4 * cell + 1] = e.y;
+        Q[4 * cell] = ex;
+        Q[4 * cell + 1] = ey;
         Q[4 * cell + 2] = pk[cell];
         Q[4 * cell + 3] = bb;
     });
 }
 
-// Workspace of the twin: two iterate planes of double2, b and three pressure
-// planes of double.
-size_t twin_ws_bytes(int w, int h) { return (size_t)w * h * (2 * sizeof(double2) + 4 * sizeof(double)); }
+__device__ __forceinline__ double from_left(double x) {
+    return __hiloint2double(
+        __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x138, 0xf, 0xf, true),
+        __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double from_right(double x) {
+    return __hiloint2double(
+        __builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x130, 0xf, 0xf, true),
+        __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x130, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double own_register(double x) {
+    double y;
+    asm("v_mov_b64 %0, %1" : "=v"(y) : "v"(x));
+    return y;
+}
+
+constexpr int kTwinSweeps = 8;  // sweeps per launch, at most
+
+// A launch of ns Jacobi sweeps over planes of doubles; blockIdx.y picks the
+// plane (u or v for the diffusion).
+struct TwinArgs {
+    int w, h, tiles_x, ns;
+    const double *src[2];
+    double *dst[2];   // the last sweep's iterate
+    double *prev[2];  // the one before it, if not null
+    const double *rhs;                 // pressure: the divergence
+    double alpha, beta, rcp_beta;      // diffusion
+    int fast_div;
+};
+
+// ns sweeps in the wave layout of pfs_wave_kernels.h: a wavefront owns S whole
+// rows of a 128-cell region, two cells a lane, DPP to the sides, the outer
+// rows exchanged through LDS.  u and v don't meet in a sweep, so each has its
+// own workgroups and a sweep of either kind is one value a cell; the halo is
+// ns cells (columns: rounded up to even).  DIFF: src/fluid.cpp:154-185, else
+// src/fluid.cpp:240-257, operations and their order as there.  The division
+// by beta is Markstein's (see div_fast) where the host allows it and a
+// wavefront's numerators lie in [2^-900, 2^900), else IEEE division.
+// One launch per sweep was bound by memory and the launches' ends (7.3 and 6.5
+// us a sweep at 1001x751, 16 sweeps: 117 and 104 us);
+// 8 sweeps a launch are bound by VALU issue and the exchange: 17.9 and 10.1 us a
+// launch, 36 and 20 us.
+template <int S, bool DIFF>
+__global__ __launch_bounds__(kWaveMax * 64) void k_t_sweeps(TwinArgs a) {
+    constexpr int XB = kWaveMax * 2 * 64;
+    __shared__ double2 lds[2 * XB];
+    const int H = a.ns, hx = H + (H & 1), w = a.w, h = a.h;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nw = blockDim.x >> 6, ry = nw * S, r0 = wave * S;
+    const int tile = xcd_tile(blockIdx.x, gridDim.x);
+    const int x0 = (tile % a.tiles_x) * (kWaveRX - 2 * hx) - hx;
+    const int y0 = (tile / a.tiles_x) * (ry - 2 * H) - H;
+    const int xc = x0 + 2 * lane;
+    const bool inside = x0 >= 0 && x0 + kWaveRX <= w;
+    const int g0 = wrap_index(xc, w), g1 = wrap_index(xc + 1, w);
+    const bool z = blockIdx.y != 0;
+    const double *__restrict__ src = z ? a.src[1] : a.src[0];
+    double *dst = z ? a.dst[1] : a.dst[0], *prev = z ? a.prev[1] : a.prev[0];
+
+    auto load = [&](const double *row, double (&f)[2]) {
+        Pair<double> c;
+        if (inside) {
+            c = *reinterpret_cast<const Pair<double> *>(row + xc);
+        } else {
+            c.a = row[g0];
+            c.b = row[g1];
+        }
+        f[0] = c.a;
+        f[1] = c.b;
+    };
+    double x[S][2], rhs[S][2];
+    int gj = wrap_index(y0 + r0, h);
+#pragma unroll
+    for (int k = 0; k < S; ++k) {
+        load(src + gj * w, x[k]);
+        if (!DIFF) load(a.rhs + gj * w, rhs[k]);
+        gj = gj + 1 == h ? 0 : gj + 1;
+    }
+#pragma unroll
+    for (int k = 0; k < S; ++k)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            x[k][q] = own_register(x[k][q]);
+            if (!DIFF) rhs[k][q] = own_register(rhs[k][q]);
+        }
+
+    const bool col = lane >= hx / 2 && lane < (kWaveRX - hx) / 2;
+    auto store = [&](double *f) {
+#pragma unroll
+        for (int k = 0; k < S; ++k) {
+            const int r = r0 + k, j = y0 + r;
+            if (r < H || r >= ry - H || j >= h || !col || xc >= w) continue;
+            double *at = f + j * w + xc;
+            if (xc + 1 < w)
+                *reinterpret_cast<Pair<double> *>(at) = {x[k][0], x[k][1]};
+            else
+                *at = x[k][0];
+        }
+    };
+
+    // c: the values as their neighbours add them; lr: the horizontal pairs.
+    double c[S][2], lr[S][2];
+    const int top_row = max(2 * wave - 1, 0) * 64 + lane;  // the outermost waves meet their own row
+    const int bot_row = min(2 * wave + 2, 2 * nw - 1) * 64 + lane;
+    auto publish = [&](int s) {  // for sweep s, which reads buffer s & 1
+        double2 *X = lds + (s & 1) * XB;
+#pragma unroll
+        for (int k = 0; k < S; ++k)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) c[k][q] = DIFF ? a.alpha * x[k][q] : x[k][q];
+        X[2 * wave * 64 + lane] = {c[0][0], c[0][1]};
+        X[(2 * wave + 1) * 64 + lane] = {c[S - 1][0], c[S - 1][1]};
+#pragma unroll
+        for (int k = 0; k < S; ++k) {
+            lr[k][0] = from_left(c[k][1]) + c[k][1];
+            lr[k][1] = c[k][0] + from_right(c[k][0]);
+        }
+        __syncthreads();
+    };
+    auto sweep = [&](int s) {
+        const double2 *X = lds + (s & 1) * XB;
+        const double2 above = X[top_row], below = X[bot_row];
+        unsigned worst = 0;
+#pragma unroll
+        for (int k = 0; k < S; ++k)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const double T = k == 0 ? (q ? above.y : above.x) : c[k > 0 ? k - 1 : 0][q];
+                const double B = k == S - 1 ? (q ? below.y : below.x) : c[k + 1 < S ? k + 1 : k][q];
+                const double sum = lr[k][q] + T + B + 1.0 * (DIFF ? x[k][q] : rhs[k][q]);
+                if (DIFF) {
+                    x[k][q] = sum;  // the numerator
+                    // |sum| in [2^-900, 2^900), read off the exponent
+                    worst = max(worst, ((unsigned)__double2hiint(sum) & 0x7fffffffu) - (123u << 20));
+                } else {
+                    x[k][q] = sum * 0.25;  // / 4, exactly
+                }
+            }
+        if (!DIFF) return;
+        const bool fast = a.fast_div && __all(worst < (1800u << 20));
+        if (fast) {
+#pragma unroll
+            for (int k = 0; k < S; ++k)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const double n = x[k][q];
+                    double d = n * a.rcp_beta;
+                    d = fma(fma(-d, a.beta, n), a.rcp_beta, d);
+                    x[k][q] = fma(fma(-d, a.beta, n), a.rcp_beta, d);
+                }
+        } else {
+#pragma unroll
+            for (int k = 0; k < S; ++k)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) x[k][q] = x[k][q] / a.beta;
+        }
+    };
+    publish(1);
+#pragma unroll 1
+    for (int s = 1; s < a.ns; ++s) {
+        sweep(s);
+        publish(s + 1);
+    }
+    if (prev) store(prev);
+    sweep(a.ns);
+    store(dst);
+}
+
+// Workspace of the twin: four iterate planes (u and v, twice), b and three
+// pressure planes.
+size_t twin_ws_bytes(int w, int h) { return (size_t)w * h * 8 * sizeof(double); }
+
+// K sweeps, at most kTwinSweeps a launch, as even as possible.  Iterates go
+// from cur to next and back; the last one goes to `last`, and the one before
+// it to `prev` (unless null), which may be neither cur nor next at that time.
+template <bool DIFF>
+void twin_sweeps(TwinArgs a, int K, double *const (&cur)[2], double *const (&next)[2],
+                 double *const (&last)[2], double *const (&prev)[2], hipStream_t s) {
+    const int nchunks = (K + kTwinSweeps - 1) / kTwinSweeps, planes = DIFF ? 2 : 1;
+    double *const *from = cur, *const *to = next;
+    for (int c = 0; c < nchunks; ++c) {
+        a.ns = K / nchunks + (c < K % nchunks);
+        const bool end = c + 1 == nchunks;
+        for (int z = 0; z < 2; ++z) {
+            a.src[z] = from[z];
+            a.dst[z] = end ? last[z] : to[z];
+            a.prev[z] = end ? prev[z] : nullptr;
+        }
+        a.tiles_x = wave_tiles_x(a.w, a.ns);
+        const WaveShape sh = wave_shape(a.ns, device_cus(), [&](WaveShape x) {
+            return planes * wave_tiles(a.w, a.h, a.ns, x);
+        });
+        const dim3 grid((unsigned)wave_tiles(a.w, a.h, a.ns, sh), planes), block(64 * sh.nw);
+        if (sh.S == 2)
+            hipLaunchKernelGGL((k_t_sweeps<2, DIFF>), grid, block, 0, s, a);
+        else
+            hipLaunchKernelGGL((k_t_sweeps<4, DIFF>), grid, block, 0, s, a);
+        std::swap(from, to);
+    }
+}
 
 int twin_step(double *P, double *Q, int w, int h, double dt, double visc, int kd, int kp, void *ws,
               hipStream_t s) {
     const size_t N = (size_t)w * h;
-    double2 *d[2] = {static_cast<double2 *>(ws), static_cast<double2 *>(ws) + N};
-    double *b = reinterpret_cast<double *>(d[1] + N);
-    double *p[3] = {b + N, b + 2 * N, b + 3 * N};
+    double *pl[8];
+    for (int k = 0; k < 8; ++k) pl[k] = static_cast<double *>(ws) + k * N;
+    double *b = pl[4], *p0 = pl[5], *p1 = pl[6], *p2 = pl[7];
     const dim3 grid((w + kBX - 1) / kBX, (h + kBY * kRows - 1) / (kBY * kRows)), block(kBX, kBY);
     const double alpha = visc * dt;
     const double beta = 1.0 + 4.0 * alpha;  // src/fluid.cpp:145
     const double gamma = -1.0 / dt;         // src/fluid.cpp:218
-    hipLaunchKernelGGL(k_t_advect, grid, block, 0, s, P, d[0], w, h, dt, (double)w, (double)h,
+    const bool even = kd % 2 == 0;
+
+    // The chunks before the last alternate between planes {0, 1} and {2, 3};
+    // the last reads one pair and leaves E in the other.  For odd Kd, E is
+    // D^(Kd-1), and D^Kd lies in p1 and p2 until b is formed.
+    double *const A[2] = {pl[0], pl[1]}, *const B[2] = {pl[2], pl[3]}, *const none[2] = {nullptr, nullptr};
+    double *const pp[2] = {p1, p2};
+    const bool odd_chunks = ((kd + kTwinSweeps - 1) / kTwinSweeps) & 1;
+    double *const E[2] = {odd_chunks ? B[0] : A[0], odd_chunks ? B[1] : A[1]};
+    hipLaunchKernelGGL(k_t_advect, grid, block, 0, s, P, A[0], A[1], w, h, dt, (double)w, (double)h,
                        1.0 / w, 1.0 / h, (w & (w - 1)) == 0, (h & (h - 1)) == 0);
-    for (int k = 1; k <= kd; ++k)
-        hipLaunchKernelGGL(k_t_diffuse, grid, block, 0, s, d[(k - 1) & 1], d[k & 1], w, h, alpha,
-                           beta);
-    hipLaunchKernelGGL(k_t_divergence, grid, block, 0, s, d[kd & 1], P, Q, b, p[0], w, h, gamma,
-                       kd % 2 == 0);
-    for (int k = 1; k <= kp; ++k)
-        hipLaunchKernelGGL(k_t_pressure, grid, block, 0, s, p[(k - 1) % 3], p[k % 3], b, w, h);
-    hipLaunchKernelGGL(k_t_finalize, grid, block, 0, s, P, Q, d[kd & 1], d[(kd + 1) & 1], p[0],
-                       p[1], p[2], b, w, h, dt, kd, kp);
+    TwinArgs a{};
+    a.w = w;
+    a.h = h;
+    a.alpha = alpha;
+    a.beta = beta;
+    a.rcp_beta = 1.0 / beta;
+    a.fast_div = beta >= 0x1p-20 && beta <= 0x1p20;
+    if (even)
+        twin_sweeps<true>(a, kd, A, B, E, none, s);
+    else
+        twin_sweeps<true>(a, kd, A, B, pp, E, s);
+    hipLaunchKernelGGL(k_t_divergence, grid, block, 0, s, even ? E[0] : p1, even ? E[1] : p2,
+                       even ? Q : P, b, p0, w, h, gamma);
+    // Pressure: chunks alternate between p0 and p1; the last reads one and
+    // writes the other and p2.
+    const bool podd = ((kp + kTwinSweeps - 1) / kTwinSweeps) & 1;
+    double *pkm1 = podd ? p1 : p0;
+    double *const c0[2] = {p0, nullptr}, *const c1[2] = {p1, nullptr}, *const end[2] = {p2, nullptr};
+    double *const before[2] = {pkm1, nullptr};
+    a.rhs = b;
+    twin_sweeps<false>(a, kp, c0, c1, end, before, s);
+    hipLaunchKernelGGL(k_t_finalize, grid, block, 0, s, P, Q, E[0], E[1], p2, pkm1, b, w, h, dt);
     return check_launch("FP64 twin step");
 }
 

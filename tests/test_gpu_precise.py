@@ -34,6 +34,58 @@ def test_f64_twin_equals_oracle_double(orc64, shape, k):
     assert tmp.cpu().numpy().tobytes() == b.tobytes()
 
 
+@pytest.mark.parametrize("k", [7, 9, 16, 17, 30])
+@pytest.mark.parametrize("shape", [(127, 40), (128, 131), (401, 300), (1303, 1100)])
+def test_f64_twin_in_chunks_of_sweeps(orc64, shape, k):
+    """Chunks of every parity, on fields below and above a tile's width, of 2
+    and of 4 rows a wavefront."""
+    if shape[0] > 1000 and k not in (9, 16):
+        pytest.skip("two counts on the large field")
+    s = scenes.random_scene(*shape, 4, 4, seed=50 + k, dt=0.7, visc=0.3, iters=k)
+    vp, tmp = _dev64(s.vp), _dev64(s.tmp)
+    a, b = s.vp.astype(np.float64), s.tmp.astype(np.float64)
+    for _ in range(2):
+        fluid.simulate_fluid_step_f64(vp, tmp, s.dt, s.visc, k, k)
+        a, b = orc64.simulate_fluid_step(a, b, s.dt, s.visc, k)
+    assert vp.cpu().numpy().tobytes() == a.tobytes()
+    assert tmp.cpu().numpy().tobytes() == b.tobytes()
+
+
+@pytest.mark.parametrize("visc", [0.3, 0.0, 2.0 ** 21, float("inf")])
+@pytest.mark.parametrize("scale", [1.0, 0.0, 1e-290, 1e290])
+def test_f64_twin_every_division(orc64, visc, scale):
+    """Numerators and divisors inside and outside the fast division's range."""
+    s = scenes.random_scene(140, 70, 4, 4, seed=9, dt=0.5, visc=0.1, iters=5)
+    a, b = s.vp.astype(np.float64), s.tmp.astype(np.float64)
+    a[:, 60:, :2] *= scale
+    vp, tmp = torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()
+    fluid.simulate_fluid_step_f64(vp, tmp, 0.5, visc, 5, 5)
+    with np.errstate(all="ignore"):
+        a, b = orc64.simulate_fluid_step(a, b, 0.5, visc, 5)
+    np.testing.assert_array_equal(vp.cpu().numpy(), a)  # NaN equals NaN, of any payload
+    np.testing.assert_array_equal(tmp.cpu().numpy(), b)
+
+
+@pytest.mark.parametrize("kd,kp", [(17, 5), (16, 9), (9, 8), (3, 2)])
+def test_f64_twin_with_fewer_pressure_sweeps(kd, kp):
+    """The contract for Kp < Kd, its sweeps formed here with numpy.roll."""
+    s = scenes.random_scene(203, 90, 4, 4, seed=kd, dt=0.7, visc=0.3, iters=kd)
+    vp, tmp = _dev64(s.vp), _dev64(s.tmp)
+    start = (s.tmp if kd % 2 == 0 else s.vp)[..., 2].astype(np.float64)
+    fluid.simulate_fluid_step_f64(vp, tmp, s.dt, s.visc, kd, kp)
+    P, Q = vp.cpu().numpy(), tmp.cpu().numpy()
+    b, hist = Q[..., 3], [start]
+    for _ in range(kp):
+        p = hist[-1]
+        hist.append((np.roll(p, 1, 1) + np.roll(p, -1, 1) + np.roll(p, 1, 0) + np.roll(p, -1, 0) + b) / 4)
+    np.testing.assert_array_equal(Q[..., 2], hist[-1])
+    np.testing.assert_array_equal(P[..., 2], hist[-2])
+    p = hist[-1]
+    grad = [(np.roll(p, -1, ax) - np.roll(p, 1, ax)) * s.dt / 2.0 for ax in (1, 0)]
+    for c in (0, 1):
+        np.testing.assert_array_equal(P[..., c], Q[..., c] - grad[c])
+
+
 def _residual(q):
     p = q[..., 2].astype(np.float64)
     b = q[..., 3].astype(np.float64)
