@@ -495,6 +495,144 @@ __global__ __launch_bounds__(kWaveMax * 64, S == 2 ? 8 : 6) void k_diffuse_wave_
     diffuse_wave<H, FIRST ? From::Advect : From::Plane, LAST ? To::Step : To::Plane, S, true>(a, xcd_tile(blockIdx.x, a.ntiles));
 }
 
+// What a pressure launch does: the same in every workgroup, from the state the
+// launches before it left.
+struct PTask {
+    bool run;     // false: nothing to do
+    bool finish;  // re-run to the converged iterate
+    bool fin;     // write the outputs
+    int src, b0, ns;  // input plane, its iterate number, sweeps
+};
+__device__ __forceinline__ PTask pressure_task(const PreciseArgs &a) {
+    const int done = a.ctl->done, stop = a.ctl->stop;
+    PTask t{};
+    if (done) return t;
+    t.run = true;
+    if (stop >= 0) {
+        // The fold of launch k = launch - 1 (iterates kC .. kC + C - 1) found
+        // iterate `stop`: re-run from launch k's input, or from launch k-1's
+        // when `stop` is launch k's input itself (stop >= 1, so k >= 1 then).
+        const int k = a.launch - 1, kb = k * a.C;
+        t.finish = t.fin = true;
+        if (stop > kb) {
+            t.src = k % 3;
+            t.b0 = kb;
+        } else {
+            t.src = (k + 2) % 3;
+            t.b0 = kb - a.C;
+        }
+        t.ns = stop - t.b0;
+    } else if (a.launch < a.nchunks) {
+        t.src = a.launch % 3;
+        t.b0 = a.launch * a.C;
+        t.ns = min(a.C, a.K - t.b0);
+        t.fin = a.launch == a.nchunks - 1;
+    } else {
+        t.run = false;  // the fix-up launch, with nothing to fix
+    }
+    return t;
+}
+
+// A launch's end: this workgroup's FP64 sums go to its slots, and the last
+// workgroup to finish folds every row over the tiles and decides.
+// wsum[m][wave]: the residual sums of sweep m + 1 (m < C); rK and b2 are this
+// thread's shares of r(p^K)^2 and b^2; the workgroup has NT = blockDim.x
+// threads.  The slots are written past L2 (agent-scope stores) and waited for
+// before the workgroup counts itself finished, and read the same way: a full
+// release here would write every dirty line of the XCD's L2 back, once a
+// workgroup (a step at 2048^2, 16 sweeps: 369 us with it, 339 without).
+template <int NSLOT, int NWMAX>
+__device__ __forceinline__ void end_launch(const PreciseArgs &a, const PTask &t, int tile, double rK,
+                                           double b2, double (&wsum)[NSLOT][NWMAX],
+                                           double (&rowsum)[NSLOT], int &last_group) {
+    constexpr int C = NSLOT - 2;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, NW = blockDim.x >> 6;
+    const bool fin = t.fin;
+    const int b0 = t.b0, ns = t.ns;
+    auto put = [&](int row, double v) {
+        __hip_atomic_store(a.part + (size_t)row * a.ntiles + tile, v, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    };
+    if (!t.finish) {
+        const double tk = wave_sum(rK), tb = wave_sum(b2);
+        if (lane == 0) {
+            wsum[C][wv] = tk;
+            wsum[C + 1][wv] = tb;
+        }
+        __syncthreads();
+        if ((int)threadIdx.x < NSLOT) {
+            double t = 0.0;
+            for (int w = 0; w < NW; ++w) t += wsum[threadIdx.x][w];
+            rowsum[threadIdx.x] = t;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int m = 0; m < ns; ++m) put(b0 + m, rowsum[m]);
+            if (fin) put(a.K, rowsum[C]);
+            if (a.launch == 0) put(kRowB2, rowsum[C + 1]);
+        }
+    }
+    // ---- the last workgroup of the launch folds and decides -----------------
+    if (threadIdx.x == 0) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // keeps the compiler's order
+        __builtin_amdgcn_s_waitcnt(0);  // the slots are in memory before the count
+        const unsigned n = __hip_atomic_fetch_add(&a.ctl->count[a.launch], 1u, __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT);
+        last_group = n == (unsigned)a.ntiles - 1u;
+    }
+    __syncthreads();
+    if (!last_group) return;
+    if (t.finish) {
+        if (threadIdx.x == 0) {
+            a.ctl->kp = b0 + ns;
+            a.ctl->done = 1;
+        }
+        return;
+    }
+    // Slot m of this launch is row b0 + m (m < ns), then row K (fin), then
+    // b^2 (launch 0).  Wave w folds slots w, w + NW, ... over the tiles:
+    // lane j sums tiles j, j + 64, ... with four accumulators in a fixed
+    // pattern, then the butterfly; every total is the same on every run.
+    const int nrow = ns + (fin ? 1 : 0) + (a.launch == 0 ? 1 : 0);
+    for (int m = wv; m < nrow; m += NW) {
+        const int row = m < ns ? b0 + m : (fin && m == ns ? a.K : kRowB2);
+        const double *src = a.part + (size_t)row * a.ntiles;
+        double acc[4] = {0.0, 0.0, 0.0, 0.0};
+        int i = lane;
+        for (; i + 192 < a.ntiles; i += 256) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                acc[q] += __hip_atomic_load(src + i + 64 * q, __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_AGENT);
+        }
+        for (int q = 0; i < a.ntiles; i += 64, ++q)
+            acc[q] += __hip_atomic_load(src + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const double tot = wave_sum((acc[0] + acc[1]) + (acc[2] + acc[3]));
+        if (lane == 0) {
+            a.ctl->total[row] = tot;
+            rowsum[m] = tot;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const double b2 = a.launch == 0 ? rowsum[nrow - 1] : a.ctl->total[kRowB2];
+        const double lim = a.tol2 * b2;
+        int found = -1;
+        for (int m = b0 >= 1 ? 0 : 1; m < ns; ++m)
+            if (rowsum[m] <= lim) {
+                found = b0 + m;
+                break;
+            }
+        if (found >= 0) {
+            a.ctl->stop = found;
+        } else if (fin) {
+            a.ctl->kp = a.K;
+            a.ctl->done = 1;
+        }
+    }
+}
+
+
 // Up to C = H - 1 compensated pressure sweeps of one tile, the residual of
 // every iterate they read, and (on the launch that ends the solve) the
 // gradient subtraction and the outputs.  See the file comment for the
@@ -513,38 +651,13 @@ __attribute__((amdgpu_waves_per_eu(NTMAX == 512 ? 4 : 1))) void k_pressure_preci
     __shared__ double rowsum[NSLOT];
     __shared__ int last_group;
 
-    // ---- what this launch does: every workgroup reads the same state -------
-    const int done = a.ctl->done, stop = a.ctl->stop;
-    if (done) return;
-    bool finish, fin;  // finish: re-run to the converged iterate; fin: write the outputs
-    int src, b0, ns;   // input plane, its iterate number, sweeps
-    if (stop >= 0) {
-        // The fold of launch k = launch - 1 (iterates kC .. kC + C - 1) found
-        // iterate `stop`: re-run from launch k's input, or from launch k-1's
-        // when `stop` is launch k's input itself (stop >= 1, so k >= 1 then).
-        const int k = a.launch - 1, kb = k * a.C;
-        finish = fin = true;
-        if (stop > kb) {
-            src = k % 3;
-            b0 = kb;
-        } else {
-            src = (k + 2) % 3;
-            b0 = kb - a.C;
-        }
-        ns = stop - b0;
-    } else if (a.launch < a.nchunks) {
-        finish = false;
-        src = a.launch % 3;
-        b0 = a.launch * a.C;
-        ns = min(a.C, a.K - b0);
-        fin = a.launch == a.nchunks - 1;
-    } else {
-        return;  // the fix-up launch, with nothing to fix
-    }
-
+    const PTask task = pressure_task(a);
+    if (!task.run) return;
+    const bool fin = task.fin;
+    const int ns = task.ns;
     const int tile = xcd_tile(blockIdx.x, a.ntiles);
     const Strip<G> st(threadIdx.x, tile, a.tiles_x, a.w, a.h);
-    const float *__restrict__ in = a.pl[src];
+    const float *__restrict__ in = a.pl[task.src];
     float p[S], rhs[S];
     double b2 = 0.0;
 #pragma unroll
@@ -649,83 +762,7 @@ __attribute__((amdgpu_waves_per_eu(NTMAX == 512 ? 4 : 1))) void k_pressure_preci
         }
     }
 
-    // ---- this workgroup's FP64 sums into its slots -------------------------
-    if (!finish) {
-        const double tk = wave_sum(rK), tb = wave_sum(b2);
-        if (lane == 0) {
-            wsum[C][wv] = tk;
-            wsum[C + 1][wv] = tb;
-        }
-        __syncthreads();
-        if ((int)threadIdx.x < NSLOT) {
-            double t = 0.0;
-            for (int w = 0; w < NW; ++w) t += wsum[threadIdx.x][w];
-            rowsum[threadIdx.x] = t;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            for (int m = 0; m < ns; ++m) a.part[(size_t)(b0 + m) * a.ntiles + tile] = rowsum[m];
-            if (fin) a.part[(size_t)a.K * a.ntiles + tile] = rowsum[C];
-            if (a.launch == 0) a.part[(size_t)kRowB2 * a.ntiles + tile] = rowsum[C + 1];
-        }
-    }
-    // ---- the last workgroup of the launch folds and decides -----------------
-    if (threadIdx.x == 0) {
-        __threadfence();  // release: this workgroup's slots before its count
-        const unsigned n = atomicAdd(&a.ctl->count[a.launch], 1u);
-        last_group = n == (unsigned)a.ntiles - 1u;
-    }
-    __syncthreads();
-    if (!last_group) return;
-    __threadfence();  // acquire: every workgroup's slots
-    if (finish) {
-        if (threadIdx.x == 0) {
-            a.ctl->kp = stop;
-            a.ctl->done = 1;
-        }
-        return;
-    }
-    // Slot m of this launch is row b0 + m (m < ns), then row K (fin), then
-    // b^2 (launch 0).  Wave w folds slots w, w + NW, ... over the tiles:
-    // lane j sums tiles j, j + 64, ... with four accumulators in a fixed
-    // pattern, then the butterfly; every total is the same on every run.
-    const int nrow = ns + (fin ? 1 : 0) + (a.launch == 0 ? 1 : 0);
-    for (int m = wv; m < nrow; m += NW) {
-        const int row = m < ns ? b0 + m : (fin && m == ns ? a.K : kRowB2);
-        const double *src = a.part + (size_t)row * a.ntiles;
-        double t[4] = {0.0, 0.0, 0.0, 0.0};
-        int i = lane;
-        for (; i + 192 < a.ntiles; i += 256) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                t[q] += __hip_atomic_load(src + i + 64 * q, __ATOMIC_RELAXED,
-                                          __HIP_MEMORY_SCOPE_AGENT);
-        }
-        for (int q = 0; i < a.ntiles; i += 64, ++q)
-            t[q] += __hip_atomic_load(src + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const double tot = wave_sum((t[0] + t[1]) + (t[2] + t[3]));
-        if (lane == 0) {
-            a.ctl->total[row] = tot;
-            rowsum[m] = tot;
-        }
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const double b2 = a.launch == 0 ? rowsum[nrow - 1] : a.ctl->total[kRowB2];
-        const double lim = a.tol2 * b2;
-        int found = -1;
-        for (int m = b0 >= 1 ? 0 : 1; m < ns; ++m)
-            if (rowsum[m] <= lim) {
-                found = b0 + m;
-                break;
-            }
-        if (found >= 0) {
-            a.ctl->stop = found;
-        } else if (fin) {
-            a.ctl->kp = a.K;
-            a.ctl->done = 1;
-        }
-    }
+    end_launch<NSLOT, NW>(a, task, tile, rK, b2, wsum, rowsum, last_group);
 }
 
 // ---- host dispatch --------------------------------------------------------------
