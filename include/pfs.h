@@ -348,6 +348,10 @@ int pfs_ngrid_lists(const pfs_ngrid *g, const float *xs, const float *ys, const 
                     const uint32_t *cell_start, const uint32_t *cell_end, const uint32_t *counts,
                     uint32_t *offsets, uint32_t *nbr, size_t nbr_capacity, uint32_t *total,
                     void *workspace, size_t workspace_bytes, void *stream);
+/* The *total that the calling thread's last list call (pfs_ngrid_neighbors
+ * with nbr, pfs_ngrid_lists) waited for, also when it exceeded nbr_capacity;
+ * 0 before the first. */
+size_t pfs_ngrid_list_total(void);
 /* rho[i] = (mass * 4/(pi r^8)) * S, S the FP32 sum over i and its neighbours
  * of (r^2 - d^2)^3 (2D poly6) in the traversal order (i where its cell's
  * range meets it); counts (may be NULL) gets the neighbour counts of the same

@@ -1269,6 +1269,8 @@ PbfWs pbf_ws(void *ws, int n, int max_iters) {
     return w;
 }
 
+thread_local size_t t_list_total = 0;  // of this thread's last call of the next
+
 // Offsets and *total from counts, then the lists (checked against the
 // capacity first, which waits for *total).
 int lists_from_counts(const pfs_ngrid *g, const NArgs &a, const uint32_t *counts,
@@ -1278,6 +1280,7 @@ int lists_from_counts(const pfs_ngrid *g, const NArgs &a, const uint32_t *counts
     uint32_t h_total = 0;
     PFS_HIP_TRY(hipMemcpyAsync(&h_total, total, sizeof h_total, hipMemcpyDeviceToHost, s));
     PFS_HIP_TRY(hipStreamSynchronize(s));
+    t_list_total = h_total;
     if (h_total > nbr_capacity)
         return set_error(PFS_ERR_INVALID, "ngrid: neighbour list capacity " +
                                               std::to_string(nbr_capacity) + " < " +
@@ -1408,6 +1411,8 @@ int pfs_ngrid_neighbors(const pfs_ngrid *g, const float *xs, const float *ys, co
     if (!nbr) return scan_exclusive(counts, offsets, g->n, total, w.sums, s);  // no lists
     return lists_from_counts(g, a, counts, offsets, nbr, nbr_capacity, total, w, s);
 }
+
+size_t pfs_ngrid_list_total(void) { return t_list_total; }
 
 int pfs_ngrid_lists(const pfs_ngrid *g, const float *xs, const float *ys, const uint32_t *order,
                     const uint32_t *cell_start, const uint32_t *cell_end, const uint32_t *counts,

@@ -13,14 +13,14 @@ from typing import Tuple
 import torch
 
 from . import _lib
-from .fluid import VPField, _Bound, _stream
+from .fluid import VPField, _stream
 
 
 PfsNGrid = _lib.PfsNGrid
 
 
-def _ptr(t: torch.Tensor) -> ctypes.c_void_p:
-    return ctypes.c_void_p(t.data_ptr())
+def _ptr(t: torch.Tensor) -> int:
+    return t.data_ptr()
 
 
 def _check_xy(x: torch.Tensor, y: torch.Tensor) -> None:
@@ -33,8 +33,9 @@ def _check_xy(x: torch.Tensor, y: torch.Tensor) -> None:
 def advect(x: torch.Tensor, y: torch.Tensor, vp: VPField, dt: float, stream=None) -> None:
     """One forward step of the tracers through vp's velocity (in place)."""
     _check_xy(x, y)
-    b = _Bound(vp)
-    _lib.call("pfs_particles_advect", _ptr(x), _ptr(y), x.numel(), b.ptr(0), dt, _stream(stream))
+    field = vp._struct()
+    _lib.call("pfs_particles_advect", _ptr(x), _ptr(y), x.numel(), ctypes.byref(field), dt,
+              _stream(stream))
 
 
 def scan_exclusive(t: torch.Tensor, stream=None) -> Tuple[torch.Tensor, int]:
@@ -106,8 +107,8 @@ class NeighborGrid:
     def neighbors(self, stream=None, xs=None, ys=None, by_position=False, counted=False):
         """(counts, offsets, lists): particle i's neighbours are
         lists[offsets[i] : offsets[i] + counts[i]].  All three are the grid's
-        own buffers, overwritten by its next count or list call.  Synchronises
-        the stream to size the lists: one counting pass when the list buffer
+        own buffers, overwritten by its next count or list call.  Waits for the
+        counts to size the lists (the lists themselves are queued): one counting pass when the list buffer
         kept from an earlier call holds them, else a sizing pass first (the
         buffer then grows with 25% headroom).  counted=True: the grid's counts
         already hold those of these positions (density(..., with_counts=True)
@@ -118,7 +119,7 @@ class NeighborGrid:
             _lib.call(fn, *self._common(xs, ys, by_position), _ptr(self.counts),
                       _ptr(self.offsets), _ptr(self.nbr), self.nbr.numel(), _ptr(self.total),
                       _ptr(self.ws), self.ws.numel() * 4, _stream(stream))
-            return self.counts, self.offsets, self.nbr[:int(self.total.item()) & 0xFFFFFFFF]
+            return self.counts, self.offsets, self.nbr[:_lib.load().pfs_ngrid_list_total()]
 
         if self.nbr is None and counted:  # the first call sizes the buffer from its total
             self.nbr = torch.empty(1, dtype=torch.int32, device=self.keys.device)
