@@ -82,6 +82,17 @@ __device__ __forceinline__ TraceT<T> trace(T xp, T yp, int w, int h, T fw, T fh)
     return t;
 }
 
+// Counts the calling thread's workgroup finished and returns how many were
+// before it.  What the thread has written by agent-scope stores is then visible
+// to agent-scope loads of the workgroup that counts itself last: those stores go
+// past L2 and are waited for here.  (A release fence would instead write every
+// dirty line of the XCD's L2 back, once a workgroup.)
+__device__ __forceinline__ unsigned count_finished(unsigned *count) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // keeps the compiler's order
+    __builtin_amdgcn_s_waitcnt(0);
+    return __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Periodic neighbours, equal to ((i-1) % n + n) % n and (i+1) % n for i in [0, n).
 __device__ __forceinline__ int wrap_minus(int i, int n) { return i == 0 ? n - 1 : i - 1; }
 __device__ __forceinline__ int wrap_plus(int i, int n) { return i + 1 == n ? 0 : i + 1; }

@@ -829,6 +829,7 @@ struct PbfArgs {
     int n;
     float W, H, half_w, half_h;
     float h, h2, mc, gc, rho0, r0sq, eps;
+    int fast_w;      // spiky_w's short root and division
     float *lambda;   // [n] by sorted position
     float *nx, *ny;  // the next iterate
     double *part;    // [max_iters + 1][nblocks]: per-block sums of C^2
@@ -921,6 +922,17 @@ __device__ __forceinline__ uint32_t staged_slot(const Staged &st, uint32_t q) {
     return (uint32_t)kStage;
 }
 
+// A particle's position and list, loaded at a pass's entry (particle n - 1's
+// past the end), under the look at the control block and what follows it.
+struct PbfOwn {
+    float x, y;
+    uint32_t o, c;
+};
+__device__ __forceinline__ PbfOwn load_own(const PbfArgs &b, int p) {
+    p = min(p, b.n - 1);
+    return {b.xs[p], b.ys[p], b.noff[p], b.ncnt[p]};
+}
+
 // Every listed neighbour of p, in list order: f(q, slot, ok, dx, dy, d2) with
 // (dx, dy) = x_q - x_p, periodic (the lists were found at the start; the
 // positions have moved since), slot q's LDS slot (kStage: not staged), ok false
@@ -928,9 +940,10 @@ __device__ __forceinline__ uint32_t staged_slot(const Staged &st, uint32_t q) {
 // lanes, the entries of two steps loaded together.  QUAD = 1: eight loaded
 // together, and the list's last few in fours.
 template <int QUAD, typename F>
-__device__ __forceinline__ void for_listed(const PbfArgs &b, const Staged *st, int p, F &&f) {
-    const float px = b.xs[p], py = b.ys[p];
-    const uint32_t o = b.noff[p], c = b.ncnt[p];
+__device__ __forceinline__ void for_listed(const PbfArgs &b, const Staged *st, int p,
+                                           const PbfOwn &own, F &&f) {
+    const float px = own.x, py = own.y;
+    const uint32_t o = own.o, c = own.c;
     const bool on = QUAD == 1 && st->on;
     const uint32_t l = QUAD == 4 ? (uint32_t)quad_lane() : 0u;
     // n steps from entry k on; all of them listed unless masked.
@@ -956,8 +969,13 @@ __device__ __forceinline__ void for_listed(const PbfArgs &b, const Staged *st, i
         }
 #pragma unroll
         for (int j = 0; j < N; ++j) {
-            const float dx = periodic_diff(x[j], px, b.W, b.half_w);
-            const float dy = periodic_diff(y[j], py, b.H, b.half_h);
+            // periodic_diff's selects run only in a wavefront that has a pair
+            // across the wrap: they are 12 of an entry's 70 operations.
+            float dx = x[j] - px, dy = y[j] - py;
+            if (__any(fabsf(dx) > b.half_w || fabsf(dy) > b.half_h)) {
+                dx = periodic_diff(x[j], px, b.W, b.half_w);
+                dy = periodic_diff(y[j], py, b.H, b.half_h);
+            }
             f(q[j], sl[j], listed(j), dx, dy, dx * dx + dy * dy);
         }
     };
@@ -974,11 +992,35 @@ __device__ __forceinline__ void for_listed(const PbfArgs &b, const Staged *st, i
 // w with grad W_spiky(x_p - x_q) = -w * (dx, dy): ((gc * t) * t) / r,
 // t = h - r, r = sqrt(d2), for 0 < d2 < h^2; else 0 (selected, so that the
 // loops do not branch; adding +-0 leaves the sums unchanged).
+// Root and division correctly rounded without their range handling: r and an
+// approximation of 1/r from one reciprocal root by Goldschmidt's iteration and
+// a last residual step (exact for every d2 in [2^-100, 2^100), all 1.7e9 tried),
+// the division by Markstein's steps as in div_fast.  Their theorem needs 1/r
+// correctly rounded, which it is but for 5 significands of d2 in two binades,
+// all x tried for those: only r = 2 - 2^-23 (times a power of two) divides some
+// x wrongly, d2's significand then being all ones, the last bit aside.  Such a
+// d2 anywhere in the wavefront, one below 2^-100, or a radius that lets the
+// quotients' remainders underflow (b.fast_w, host) takes the plain forms.
 __device__ __forceinline__ float spiky_w(const PbfArgs &b, float d2) {
+    const bool in = d2 > 0.0f && d2 < b.h2;
+    const float d = in ? d2 : 1.0f;
+    if (b.fast_w && !__any(d < 0x1p-100f || (__float_as_uint(d) | 0xff800001u) == 0xffffffffu)) {
+        const float y0 = __builtin_amdgcn_rsqf(d);
+        float g = d * y0, y = 0.5f * y0;
+        const float e = fmaf(-y, g, 0.5f);
+        g = fmaf(g, e, g);
+        y = fmaf(y, e, y);
+        const float r = fmaf(fmaf(-g, g, d), y, g);
+        y = y + y;
+        y = fmaf(fmaf(-r, y, 1.0f), y, y);
+        const float t = b.h - r;
+        const float w = div_fast((b.gc * t) * t, r, y);
+        return in ? w : 0.0f;
+    }
     const float r = sqrtf(d2);
     const float t = b.h - r;
     const float w = ((b.gc * t) * t) / r;
-    return (d2 > 0.0f && d2 < b.h2) ? w : 0.0f;
+    return in ? w : 0.0f;
 }
 
 // A term of an order-bound sum: the quad's four in lane order, or this lane's.
@@ -987,24 +1029,51 @@ __device__ __forceinline__ float add_terms(float s, float t) {
     return QUAD == 4 ? quad_add(s, t) : s + t;
 }
 
-// Block-wide FP64 sum (thread 0 gets it): wave shuffles, then the waves in order.
+// Block-wide FP64 sum over NW wavefronts (thread 0 gets it): wave shuffles,
+// then the waves in order.
+template <int NW>
 __device__ __forceinline__ double block_sum(double v) {
-    __shared__ double part[16];
+    __shared__ double part[NW];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
     __syncthreads();
-    double s = 0.0;
-    if (threadIdx.x == 0)
-        for (int k = 0; k < (int)(blockDim.x >> 6); ++k) s += part[k];
+    double w[NW], s = 0.0;
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int k = 0; k < NW; ++k) w[k] = part[k];
+#pragma unroll
+        for (int k = 0; k < NW; ++k) s += w[k];
+    }
     return s;
 }
 
-// lambda of iterate b.it and the block sums of C^2.  Per listed neighbour the
-// two passes do about 85 operations, 27 of them the correctly rounded square
-// root and division.
+// The total of iterate b.it's block sums, for thread 0 of a block of 1024:
+// strided sums in block order, then the waves in order.
+__device__ __forceinline__ double fold_sums(const PbfArgs &b) {
+    double v = 0.0;
+    for (int k = threadIdx.x; k < b.nblocks; k += 1024) v += b.part[(size_t)b.it * b.nblocks + k];
+    return block_sum<16>(v);
+}
+// Writes iterate b.it's total and, at convergence, the verdict.
+__device__ __forceinline__ void record(const PbfArgs &b, double total) {
+    b.res[b.it] = total;
+    if (total <= b.tol2n) {
+        b.ctl->done = 1;
+        b.ctl->final_it = b.it;
+    }
+}
+
+// lambda of iterate b.it, and the block sums of C^2.  Short
+// lists are bound by the chain of loads (list, entries, positions), long ones by
+// VALU issue, about 45 operations an entry.  250,001 particles of 7 / 37
+// neighbours, 4 iterations of both passes: 145 / 327 us with the plain root and
+// division and every entry's wrap selects, 139 / 304 without; 135 / 297 with a
+// particle's own data loaded at entry and the sums folded in the update.
 template <int QUAD>
 __global__ __launch_bounds__(kPbfParticles *QUAD) void k_pbf_lambda(PbfArgs b) {
+    const int p = pbf_particle<QUAD>();
+    const PbfOwn own = load_own(b, p);
     if (b.ctl->done) return;  // the same verdict for every thread
     Staged *st = nullptr;
     if constexpr (QUAD == 1) {
@@ -1012,12 +1081,11 @@ __global__ __launch_bounds__(kPbfParticles *QUAD) void k_pbf_lambda(PbfArgs b) {
         st = &shared;
     }
     if constexpr (QUAD == 1) stage_windows<false>(b, *st);
-    const int p = pbf_particle<QUAD>();
     double c2 = 0.0;
     if (p < b.n) {
         float S = b.h2 * b.h2 * b.h2;  // p itself
         float gx = 0.0f, gy = 0.0f, g2 = 0.0f;
-        for_listed<QUAD>(b, st, p, [&](uint32_t, uint32_t, bool ok, float dx, float dy, float d2) {
+        for_listed<QUAD>(b, st, p, own, [&](uint32_t, uint32_t, bool ok, float dx, float dy, float d2) {
             const float t2 = ok ? fmaxf(b.h2 - d2, 0.0f) : 0.0f;
             S = add_terms<QUAD>(S, t2 * t2 * t2);
             const float w = spiky_w(b, d2);  // 0 past the list's end, where d2 = 0
@@ -1034,43 +1102,48 @@ __global__ __launch_bounds__(kPbfParticles *QUAD) void k_pbf_lambda(PbfArgs b) {
             c2 = (double)C * (double)C;
         }
     }
-    const double s = block_sum(c2);
+    const double s = block_sum<kPbfParticles * QUAD / 64>(c2);
     if (threadIdx.x == 0) b.part[(size_t)b.it * b.nblocks + blockIdx.x] = s;
 }
 
-// Folds iterate b.it's block sums (one block of 1024: strided sums in block
-// order, then the waves in order) and decides whether it has converged.  (A
-// fold by the last workgroup of k_pbf_lambda measured slower: the device-scope
-// fence every workgroup then needs writes its L2 back.)
+// Decides, between the passes, whether iterate b.it has converged, where the
+// update's workgroups don't do it themselves.  (A fold by the last workgroup of
+// k_pbf_lambda measured slower, with a release fence and without: every
+// workgroup then stays for its sum's way to memory; 262,144 particles of 7
+// neighbours, 4 iterations 158 us against 139.)
 __global__ __launch_bounds__(1024) void k_pbf_check(PbfArgs b) {
     if (b.ctl->done) return;
-    double v = 0.0;
-    for (int k = threadIdx.x; k < b.nblocks; k += 1024) v += b.part[(size_t)b.it * b.nblocks + k];
-    const double s = block_sum(v);
-    if (threadIdx.x == 0) {
-        b.res[b.it] = s;
-        if (s <= b.tol2n) {
-            b.ctl->done = 1;
-            b.ctl->final_it = b.it;
-        }
-    }
+    const double total = fold_sums(b);
+    if (threadIdx.x == 0) record(b, total);
 }
 
 // The update of iterate b.it into the next iterate (nx, ny).
 template <int QUAD>
 __global__ __launch_bounds__(kPbfParticles *QUAD) void k_pbf_delta(PbfArgs b) {
+    const int p = pbf_particle<QUAD>();
+    const PbfOwn own = load_own(b, p);
+    const float lp = b.lambda[min(p, b.n - 1)];
     if (b.ctl->done) return;
     Staged *st = nullptr;
     if constexpr (QUAD == 1) {
         __shared__ Staged shared;
         st = &shared;
+        stage_windows<true>(b, *st);
+    } else {
+        // Every workgroup folds the block sums for itself, a load or two a
+        // thread, and comes to the same verdict.
+        __shared__ int over;
+        const double total = fold_sums(b);
+        if (threadIdx.x == 0) {
+            over = total <= b.tol2n;
+            if (blockIdx.x == 0) record(b, total);
+        }
+        __syncthreads();
+        if (over) return;
     }
-    if constexpr (QUAD == 1) stage_windows<true>(b, *st);
-    const int p = pbf_particle<QUAD>();
     if (p >= b.n) return;
-    const float lp = b.lambda[p];
     float ax = 0.0f, ay = 0.0f;
-    for_listed<QUAD>(b, st, p, [&](uint32_t q, uint32_t slot, bool, float dx, float dy, float d2) {
+    for_listed<QUAD>(b, st, p, own, [&](uint32_t q, uint32_t slot, bool, float dx, float dy, float d2) {
         const float w = spiky_w(b, d2);
         float lq;
         if constexpr (QUAD == 1) {
@@ -1084,8 +1157,8 @@ __global__ __launch_bounds__(kPbfParticles *QUAD) void k_pbf_delta(PbfArgs b) {
         ay = add_terms<QUAD>(ay, s * (w * dy));
     });
     if (QUAD == 4 && quad_lane() != 0) return;
-    b.nx[p] = wrap_pos(b.xs[p] + -(ax / b.rho0), b.W);
-    b.ny[p] = wrap_pos(b.ys[p] + -(ay / b.rho0), b.H);
+    b.nx[p] = wrap_pos(own.x + -(ax / b.rho0), b.W);
+    b.ny[p] = wrap_pos(own.y + -(ay / b.rho0), b.H);
 }
 
 // Ends the solve on the caller's buffers: the final iterate f lives in the
@@ -1116,9 +1189,9 @@ int grid_for(int n) { return (n + 255) / 256; }
 // 14.9 / 12.0, 262,144 17.8 / 17.9, 1,048,576 41.3 / 60.8.
 constexpr int kSerialFrom = 1 << 18;
 // The same line for the constraint solve's passes.  4 iterations, one lane
-// against four, us: 65,536 particles of 7 / 37 neighbours 135 / 266 against
-// 81 / 130, 262,144 181 / 423 against 145 / 327, 1,048,576 438 / 1126 against
-// 547 / 1148.
+// against four, us: 65,536 particles of 7 / 37 neighbours 108 / 248 against
+// 68 / 119, 262,144 145 / 372 against 137 / 312, 393,216 171 / 498 against 183 /
+// 420, 1,048,576 360 / 1054 against 452 / 1027.
 constexpr int kPbfSerialFrom = 3 << 17;
 int quad_grid(int n) { return (n + 63) / 64; }  // 256 threads, four a particle
 
@@ -1477,6 +1550,9 @@ int pfs_pbf_solve(const pfs_ngrid *g, float *xs, float *ys, const uint32_t *cell
     const float coef = (float)(4.0 / (3.14159265358979323846 * h * h * h * h * h * h * h * h));
     b.mc = mass * coef;
     b.gc = (float)(-30.0 / (3.14159265358979323846 * h * h * h * h * h));
+    // Remainders of (gc * t) * t over r, t from an ulp of h to h, stay normal.
+    const float w_max = std::fabs(b.gc) * b.h2;
+    b.fast_w = b.h2 >= 0x1p-60f && b.h2 <= 0x1p60f && w_max >= 0x1p-30f && w_max <= 0x1p60f;
     b.rho0 = rho0;
     b.r0sq = rho0 * rho0;
     b.eps = eps;
@@ -1497,7 +1573,7 @@ int pfs_pbf_solve(const pfs_ngrid *g, float *xs, float *ys, const uint32_t *cell
         b.ny = by[(it + 1) & 1];
         hipLaunchKernelGGL(quad ? k_pbf_lambda<4> : k_pbf_lambda<1>, dim3(nb),
                            dim3(kPbfParticles * (quad ? 4 : 1)), 0, s, b);
-        hipLaunchKernelGGL(k_pbf_check, dim3(1), dim3(1024), 0, s, b);
+        if (!quad || it == max_iters) hipLaunchKernelGGL(k_pbf_check, dim3(1), dim3(1024), 0, s, b);
         if (it < max_iters)
             hipLaunchKernelGGL(quad ? k_pbf_delta<4> : k_pbf_delta<1>, dim3(nb),
                                dim3(kPbfParticles * (quad ? 4 : 1)), 0, s, b);

@@ -247,6 +247,32 @@ def test_pbf_either_side_of_the_lane_rule(n):
     np.testing.assert_allclose(res.cpu().numpy(), ores, rtol=1e-12)
 
 
+@pytest.mark.parametrize("scale", [1.0, 1e4], ids=["short-division", "plain-division"])
+@pytest.mark.parametrize("n", [4000, 3 << 17])
+def test_pbf_every_division(n, scale):
+    """Radii inside and outside the short root and division's range, distances
+    whose square's significand it excludes (1 - 2^-24 and its square), and
+    pairs across the wrap in only some wavefronts."""
+    rng = np.random.default_rng(17)
+    W = np.float32((400.0 if n > 10000 else 40.0) * scale)
+    x, y = ((rng.random(n) * W).astype(np.float32) for _ in range(2))
+    x[x >= W] = 0
+    y[y >= W] = 0
+    x[:40], x[40:80] = 0.0, np.float32(scale) * np.float32(1 - 2.0 ** -24)
+    y[40:80] = y[:40]
+    r = 1.5 * scale
+    ng = particles.NeighborGrid(n, float(W), float(W), r)
+    ng.build(torch.from_numpy(x).cuda(), torch.from_numpy(y).cuda())
+    og = op.Grid(x, y, float(W), float(W), r, ng.g.gx, ng.g.gy, ng.g.kx, ng.g.ky)
+    rho0 = float(np.median(og.density(1.0, by_position=True)))
+    ox, oy, olam, ores, _ = og.pbf(1.0, rho0, 5.0, 2)
+    lam, res, _ = ng.pbf(1.0, rho0, 5.0, 2)
+    assert ng.xs.cpu().numpy().tobytes() == ox.tobytes()
+    assert ng.ys.cpu().numpy().tobytes() == oy.tobytes()
+    assert lam.cpu().numpy().tobytes() == olam.tobytes()
+    np.testing.assert_allclose(res.cpu().numpy(), ores, rtol=1e-12)
+
+
 def test_pbf_on_tracers_and_errors():
     """Tracers.pbf works on the tracers' own (cell-ordered) positions; bad
     arguments are rejected before anything runs."""
