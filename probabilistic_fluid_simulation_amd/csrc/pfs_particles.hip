@@ -438,7 +438,7 @@ struct NArgs {
     __device__ uint32_t id(uint32_t p) const { return order ? order[p] : p; }
 };
 
-// ---- four lanes per particle ------------------------------------------------
+// ---- four (or 16) lanes per particle ----------------------------------------
 // The neighbour passes give a particle a quad of lanes: four candidates (or
 // listed neighbours) are loaded and evaluated side by side, and order-bound
 // sums are then added up one after another, each term broadcast over the quad
@@ -468,9 +468,15 @@ __device__ __forceinline__ float quad_add(float s, float t) {
 __device__ __forceinline__ uint32_t quad_total(uint32_t c) {
     return quad_bcast<0>(c) + quad_bcast<1>(c) + quad_bcast<2>(c) + quad_bcast<3>(c);
 }
-// The quad's bits of a wave-wide vote.
-__device__ __forceinline__ uint32_t quad_vote(bool b) {
-    return (uint32_t)(__ballot(b) >> (threadIdx.x & 60u)) & 0xfu;
+// Groups of L lanes (4 or 16) a particle: the lane's place in its group, and
+// the group's bits of a wave-wide vote.
+template <int L>
+__device__ __forceinline__ int group_lane() {
+    return (int)(threadIdx.x & (L - 1u));
+}
+template <int L>
+__device__ __forceinline__ uint32_t group_vote(bool b) {
+    return (uint32_t)(__ballot(b) >> (threadIdx.x & (64u - L))) & ((1u << L) - 1u);
 }
 
 // The sorted positions of one row of the 3x3 cells around cell (cx, cy): [s1,
@@ -558,16 +564,16 @@ __device__ __forceinline__ void visit_rows(const NArgs &a, int p, int cx, int cy
 }
 
 // Visits every particle q of the 3x3 cells around p's cell, p included (rows
-// then columns, -1..1, then q ascending), four at a time: f(q, ok, d2) on the
-// quad's lanes for consecutive q, ok false past a range's end.
-template <typename F>
+// then columns, -1..1, then q ascending), L at a time: f(q, ok, d2) on the
+// group's lanes for consecutive q, ok false past a range's end.
+template <int L, typename F>
 __device__ __forceinline__ void for_neighbors(const NArgs &a, int p, F &&f) {
     const uint32_t c = a.sk[p];
     if (c >= (uint32_t)a.gx * (uint32_t)a.gy) return;  // a cell by construction: kept as a bound
     const int cx = (int)(c % (uint32_t)a.gx), cy = (int)(c / (uint32_t)a.gx);
-    const int l = quad_lane();
-    // Lane j finds row j's ranges (lane 3 repeats row 2), all at once.
-    const RowRanges r = row_ranges(a, cx, cy, (l < 2 ? l : 2) - 1);
+    const int l = group_lane<L>();
+    // Lane j of a quad finds row j's ranges (lane 3 repeats row 2), all at once.
+    const RowRanges r = row_ranges(a, cx, cy, min(quad_lane(), 2) - 1);
     const uint32_t lo[3][2] = {{quad_bcast<0>(r.s1), quad_bcast<0>(r.s2)},
                                {quad_bcast<1>(r.s1), quad_bcast<1>(r.s2)},
                                {quad_bcast<2>(r.s1), quad_bcast<2>(r.s2)}};
@@ -581,7 +587,7 @@ __device__ __forceinline__ void for_neighbors(const NArgs &a, int p, F &&f) {
         y = a.ys[k];
     };
     auto scan = [&](uint32_t q, uint32_t end, auto &&d2_of) {
-        for (; q < end; q += 4) {
+        for (; q < end; q += L) {
             float x, y;
             at(q, end, x, y);
             f(q + l, q + l < end, d2_of(x, y));
@@ -597,7 +603,7 @@ __device__ __forceinline__ void for_neighbors(const NArgs &a, int p, F &&f) {
             for (int k = 0; k < 3; ++k) {
                 if (lo[k][0] < hi[k][0])
                     f(lo[k][0] + l, lo[k][0] + l < hi[k][0], d2_of(x[k], y[k]));
-                scan(lo[k][0] + 4, hi[k][0], d2_of);
+                scan(lo[k][0] + L, hi[k][0], d2_of);
             }
         },
         scan);
@@ -642,21 +648,22 @@ __device__ __forceinline__ void for_neighbors_serial(const NArgs &a, int p, F &&
         scan);
 }
 
-// 256 threads: 64 particles.
-__device__ __forceinline__ int quad_particle() {
-    return (int)(blockIdx.x * (blockDim.x >> 2) + (threadIdx.x >> 2));
+// 256 threads: 256 / L particles.
+template <int L>
+__device__ __forceinline__ int group_particle() {
+    return (int)(blockIdx.x * (blockDim.x / L) + threadIdx.x / L);
 }
 
+template <int L>
 __global__ __launch_bounds__(256) void k_nbr_count(NArgs a, uint32_t *__restrict__ counts) {
-    const int p = quad_particle();
+    const int p = group_particle<L>();
     if (p >= a.n) return;
     uint32_t c = 0;
-    for_neighbors(a, p, [&](uint32_t q, bool ok, float d2) {
-        c += ok && d2 < a.r2 && (int)q != p ? 1u : 0u;
+    for_neighbors<L>(a, p, [&](uint32_t q, bool ok, float d2) {
+        c += (uint32_t)__popc(group_vote<L>(ok && d2 < a.r2 && (int)q != p));
     });
-    c = quad_total(c);
     const uint32_t i = a.id((uint32_t)p);
-    if (quad_lane() == 0 && i < (uint32_t)a.n) counts[i] = c;
+    if (group_lane<L>() == 0 && i < (uint32_t)a.n) counts[i] = c;
 }
 
 __global__ __launch_bounds__(256) void k_nbr_count_serial(NArgs a, uint32_t *__restrict__ counts) {
@@ -668,17 +675,18 @@ __global__ __launch_bounds__(256) void k_nbr_count_serial(NArgs a, uint32_t *__r
     if (i < (uint32_t)a.n) counts[i] = c ? c - 1u : 0u;  // without p itself, as k_density
 }
 
+template <int L>
 __global__ __launch_bounds__(256) void k_nbr_fill(NArgs a, const uint32_t *__restrict__ offsets,
                                                   uint32_t *__restrict__ nbr, size_t capacity) {
-    const int p = quad_particle();
+    const int p = group_particle<L>();
     if (p >= a.n) return;
     const uint32_t i = a.id((uint32_t)p);
     if (i >= (uint32_t)a.n) return;
-    const uint32_t below = (1u << quad_lane()) - 1u;
+    const uint32_t below = (1u << group_lane<L>()) - 1u;
     size_t o = offsets[i];
-    for_neighbors(a, p, [&](uint32_t q, bool ok, float d2) {
+    for_neighbors<L>(a, p, [&](uint32_t q, bool ok, float d2) {
         const bool keep = ok && d2 < a.r2 && (int)q != p;
-        const uint32_t vote = quad_vote(keep);
+        const uint32_t vote = group_vote<L>(keep);
         const size_t to = o + __popc(vote & below);
         if (keep && to < capacity) nbr[to] = a.id(q);
         o += __popc(vote);
@@ -694,24 +702,26 @@ __global__ __launch_bounds__(256) void k_nbr_fill(NArgs a, const uint32_t *__res
 // complete in order.  1024 slots hold a wave's lists at 64 neighbours per
 // particle in one traversal (16 KB per workgroup).
 constexpr int kFillWin = 1024;
+template <int L>
 __global__ __launch_bounds__(256) void k_nbr_fill_lds(NArgs a, const uint32_t *__restrict__ offsets,
                                                       const uint32_t *__restrict__ counts,
                                                       uint32_t *__restrict__ nbr, size_t capacity) {
     __shared__ uint32_t win[4][kFillWin];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int p = quad_particle();
-    const int pw = blockIdx.x * (blockDim.x >> 2) + wave * 16;  // the wave's first particle
+    constexpr int PW = 64 / L;  // particles of a wave
+    const int p = group_particle<L>();
+    const int pw = blockIdx.x * (blockDim.x / L) + wave * PW;  // the wave's first particle
     if (pw >= a.n) return;                                     // the whole wave is past the end
-    const int plast = min(pw + 15, a.n - 1);
-    const uint32_t below = (1u << quad_lane()) - 1u;
+    const int plast = min(pw + PW - 1, a.n - 1);
+    const uint32_t below = (1u << group_lane<L>()) - 1u;
     const size_t base = offsets[pw], end = (size_t)offsets[plast] + counts[plast];
     uint32_t *buf = win[wave];
     for (size_t w0 = base; w0 < end; w0 += kFillWin) {
         if (p < a.n) {
             size_t o = offsets[p];
-            for_neighbors(a, p, [&](uint32_t q, bool ok, float d2) {
+            for_neighbors<L>(a, p, [&](uint32_t q, bool ok, float d2) {
                 const bool keep = ok && d2 < a.r2 && (int)q != p;
-                const uint32_t vote = quad_vote(keep);
+                const uint32_t vote = group_vote<L>(keep);
                 const size_t to = o + __popc(vote & below);
                 if (keep && to >= w0 && to < w0 + kFillWin) buf[to - w0] = q;
                 o += __popc(vote);
@@ -748,11 +758,11 @@ __device__ __forceinline__ void store_density(const NArgs &a, int p, float rho_p
 
 __global__ __launch_bounds__(256) void k_density(NArgs a, float mc, float *__restrict__ rho,
                                                  uint32_t *__restrict__ counts) {
-    const int p = quad_particle();
+    const int p = group_particle<4>();
     if (p >= a.n) return;
     float sum = 0.0f;
     uint32_t cnt = 0;
-    for_neighbors(a, p, [&](uint32_t, bool ok, float d2) {
+    for_neighbors<4>(a, p, [&](uint32_t, bool ok, float d2) {
         const float t = ok ? fmaxf(a.r2 - d2, 0.0f) : 0.0f;
         sum = quad_add(sum, t * t * t);
         cnt += ok && d2 < a.r2 ? 1u : 0u;
@@ -1193,7 +1203,13 @@ constexpr int kSerialFrom = 1 << 18;
 // 68 / 119, 262,144 145 / 372 against 137 / 312, 393,216 171 / 498 against 183 /
 // 420, 1,048,576 360 / 1054 against 452 / 1027.
 constexpr int kPbfSerialFrom = 3 << 17;
-int quad_grid(int n) { return (n + 63) / 64; }  // 256 threads, four a particle
+int group_grid(int n, int L) { return (int)(((long long)n * L + 255) / 256); }  // 256 threads, L a particle
+// Lanes a particle of the counts and lists (which no order binds): 16 where four
+// leave the GPU short of wavefronts and a row's candidates are several loads one
+// after another.  Grid's counts, scan, fill, four lanes against 16, us: 16,384
+// particles of 7 / 20 / 37 neighbours 41 / 50 / 62 against 39 / 39 / 42, 65,536
+// 44 / 55 / 67 against 45 / 49 / 55, 131,072 47 / 62 / 81 against 57 / 65 / 77.
+int list_lanes(int n) { return n <= 1 << 16 ? 16 : 4; }
 
 // The digit plan for keys below ncells: the fewest passes, 8-bit digits
 // where they suffice for that many passes, else 10-bit.
@@ -1358,12 +1374,14 @@ int lists_from_counts(const pfs_ngrid *g, const NArgs &a, const uint32_t *counts
         return set_error(PFS_ERR_INVALID, "ngrid: neighbour list capacity " +
                                               std::to_string(nbr_capacity) + " < " +
                                               std::to_string(h_total));
+    const int L = list_lanes(g->n);
+    const dim3 grid(group_grid(g->n, L));
     if (a.order)
-        hipLaunchKernelGGL(k_nbr_fill, dim3(quad_grid(g->n)), dim3(256), 0, s, a, offsets, nbr,
-                           nbr_capacity);
+        hipLaunchKernelGGL(L == 16 ? k_nbr_fill<16> : k_nbr_fill<4>, grid, dim3(256), 0, s, a,
+                           offsets, nbr, nbr_capacity);
     else
-        hipLaunchKernelGGL(k_nbr_fill_lds, dim3(quad_grid(g->n)), dim3(256), 0, s, a, offsets,
-                           counts, nbr, nbr_capacity);
+        hipLaunchKernelGGL(L == 16 ? k_nbr_fill_lds<16> : k_nbr_fill_lds<4>, grid, dim3(256), 0, s, a,
+                           offsets, counts, nbr, nbr_capacity);
     return check_launch("neighbour lists");
 }
 
@@ -1478,7 +1496,8 @@ int pfs_ngrid_neighbors(const pfs_ngrid *g, const float *xs, const float *ys, co
     SortWs w = sort_ws(ws, g->n);
     const NArgs a = nargs(g, xs, ys, order, w.k0, cell_start, cell_end);
     if (g->n < kSerialFrom)
-        hipLaunchKernelGGL(k_nbr_count, dim3(quad_grid(g->n)), dim3(256), 0, s, a, counts);
+        hipLaunchKernelGGL(list_lanes(g->n) == 16 ? k_nbr_count<16> : k_nbr_count<4>,
+                           dim3(group_grid(g->n, list_lanes(g->n))), dim3(256), 0, s, a, counts);
     else
         hipLaunchKernelGGL(k_nbr_count_serial, dim3(grid_for(g->n)), dim3(256), 0, s, a, counts);
     if (!nbr) return scan_exclusive(counts, offsets, g->n, total, w.sums, s);  // no lists
@@ -1600,7 +1619,7 @@ int pfs_ngrid_density(const pfs_ngrid *g, const float *xs, const float *ys, cons
     const float coef = (float)(4.0 / (3.14159265358979323846 * r * r * r * r * r * r * r * r));
     const float mc = mass * coef;
     if (g->n < kSerialFrom)
-        hipLaunchKernelGGL(k_density, dim3(quad_grid(g->n)), dim3(256), 0, s, a, mc, rho, counts);
+        hipLaunchKernelGGL(k_density, dim3(group_grid(g->n, 4)), dim3(256), 0, s, a, mc, rho, counts);
     else
         hipLaunchKernelGGL(k_density_serial, dim3(grid_for(g->n)), dim3(256), 0, s, a, mc, rho, counts);
     return check_launch("density");

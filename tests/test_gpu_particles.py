@@ -122,6 +122,19 @@ def test_grid_at_the_edges_of_the_sorts_tiles(n, W, H):
     np.testing.assert_array_equal(ng.ys.cpu().numpy(), y[order])
 
 
+@pytest.mark.parametrize("n", [(1 << 16) - 3, 1 << 16, (1 << 16) + 1])
+@pytest.mark.parametrize("r", [1.4, 3.1], ids=["short-rows", "long-rows"])
+def test_either_side_of_the_list_lanes(n, r):
+    """16 lanes a particle up to 2^16 (counts and lists, by id and by sorted
+    position), four above."""
+    x, y = _positions(n, 220.0, 160.0, seed=n)
+    ng = _check_grid(x, y, 220.0, 160.0, r)
+    og = op.Grid(x, y, 220.0, 160.0, r, ng.g.gx, ng.g.gy, ng.g.kx, ng.g.ky)
+    got, want = ng.neighbors(by_position=True), og.neighbors(by_position=True)
+    for t, w in zip(got, want):
+        np.testing.assert_array_equal(_u32(t), w)
+
+
 def test_clustered_particles_and_empty_cells():
     """Many particles in few cells (long equal-key runs across sort tiles)."""
     rng = np.random.default_rng(11)
