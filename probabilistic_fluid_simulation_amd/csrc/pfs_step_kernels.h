@@ -190,48 +190,31 @@ __device__ __forceinline__ void pressure_sum_comp(float l, float r, float t, flo
     s = u;
 }
 
-// min over the bit patterns read as unsigned: of x and x - n it picks the one
-// in [0, n) for x in [0, 2n), a negative number having the larger pattern.
-__device__ __forceinline__ float min_bits(float a, float b) {
-    return __uint_as_float(min(__float_as_uint(a), __float_as_uint(b)));
-}
-
-// wrap_coord's value for |x| < n (see there): x + n brought into [0, n) by at
-// most two subtractions of n.
-__device__ __forceinline__ float wrap_near(float x, float n) {
-    float s = x + n;
-    s = min_bits(s, s - n);
-    return min_bits(s, s - n);
-}
-
-// Region coordinate of global index g (0 <= g < n) on an axis whose staged
-// region starts at global coordinate o in [-n, n) (periodic), if it is staged;
-// else some value past the region.
-__device__ __forceinline__ unsigned region_of(int g, int o, int n) {
-    const int r = g - o;
-    return min(min((unsigned)r, (unsigned)(r + n)), (unsigned)(r - n));
-}
-
 // The back-trace (src/fluid.cpp:36-61) of cell (fi, fj) with velocity c, as
 // staged corners: (rx, ry) the first corner's coordinates in a staged region
-// of nx x ny cells whose cell (0, 0) is global (ox, oy), `on` whether all four
-// corners are staged.  Traces longer than the field, and all of them where
-// the two-operation division by the field's sides is not proven, are not `on`.
+// of nx x ny cells, `on` whether all four corners are staged.  (kx, ky) place
+// the cell itself: kx = w + fi - its region column, and so for ky.
+// With |x| < n, wrap_coord's value is x + n (rounded once) less n or 2n
+// exactly, so its fraction is that of x + n, and the corner lies as many
+// columns from the cell as trunc(x + n) from fi + n, whatever side of the wrap
+// either is on.  (Wrapping both and looking the corner up in the region took 15
+// operations of 70 more a cell.)  Traces longer than the field, and all of them
+// where the two-operation division by the field's sides is not proven, are not
+// `on`.
 struct Near {
     float sx, sy;
     unsigned rx, ry;
     bool on;
 };
-__device__ __forceinline__ Near near_trace(const DiffuseArgs &a, float fi, float fj, float2 c, int ox,
-                                           int oy, int nx, int ny) {
+__device__ __forceinline__ Near near_trace(const DiffuseArgs &a, float fi, float fj, float2 c, int kx,
+                                           int ky, int nx, int ny) {
     const float xp = fi - div_fast2(a.dt * c.x, a.dw), yp = fj - div_fast2(a.dt * c.y, a.dh);
-    const float xw = wrap_near(xp, a.fw), yw = wrap_near(yp, a.fh);
-    const int i0 = (int)xw, j0 = (int)yw;
+    const float xs = xp + a.fw, ys = yp + a.fh;
     Near r;
-    r.sx = xw - (float)i0;
-    r.sy = yw - (float)j0;
-    r.rx = region_of(i0, ox, a.w);
-    r.ry = region_of(j0, oy, a.h);
+    r.sx = __builtin_amdgcn_fractf(xs);
+    r.sy = __builtin_amdgcn_fractf(ys);
+    r.rx = (unsigned)((int)xs - kx);
+    r.ry = (unsigned)((int)ys - ky);
     r.on = a.dw.ok && a.dh.ok && fabsf(xp) < a.fw && fabsf(yp) < a.fh && r.rx < (unsigned)nx - 1u &&
            r.ry < (unsigned)ny - 1u;
     return r;
@@ -291,7 +274,8 @@ __device__ __forceinline__ void diffuse_tile(const DiffuseArgs &a, int tile) {
         bool off[S], any_off = false;
 #pragma unroll
         for (int k = 0; k < S; ++k) {
-            const Near r = near_trace(a, (float)st.gi, (float)st.gj[k], c[k], st.x0 - 1, st.y0 - 1, VP, RY + 2);
+            const Near r = near_trace(a, (float)st.gi, (float)st.gj[k], c[k], a.w + st.gi - (st.x + 1),
+                                      a.h + st.gj[k] - (st.r0 + k + 1), VP, RY + 2);
             off[k] = !r.on;
             any_off = any_off || off[k];
             const float2 *F = plane + PL + (r.on ? r.ry * VP + r.rx : 0u);

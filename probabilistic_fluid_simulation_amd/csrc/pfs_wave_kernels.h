@@ -181,18 +181,22 @@ __device__ __forceinline__ void diffuse_wave(const DiffuseArgs &a, int tile) {
         }
         __syncthreads();
         // Every cell's back-trace (src/fluid.cpp:36-67), its corners from the
-        // staged velocities.  A trace that near_trace does not take is noted
-        // and redone below, so that this loop has no branch.
-        unsigned off = 0;
+        // staged velocities.  A trace that near_trace does not take is redone
+        // below, so that this loop has no branch.
         const float fi[2] = {(float)t.gi[0], (float)t.gi[1]};
+        const int kx[2] = {a.w + t.gi[0] - (2 * t.lane + 1), a.w + t.gi[1] - (2 * t.lane + 2)};
+        auto trace_of = [&](int k, int q, int gj, float2 c) {
+            return near_trace(a, fi[q], (float)gj, c, kx[q], a.h + gj - (t.r0 + k + 1), VP, t.ry + 2);
+        };
+        unsigned long long off = 0;
         int gj = t.first_row(a.h);
 #pragma unroll
         for (int k = 0; k < S; ++k) {
             const float2 c2[2] = {V[(t.r0 + k) * VP + 2 * t.lane], V[(t.r0 + k) * VP + 2 * t.lane + 1]};
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
-                const Near r = near_trace(a, fi[q], (float)gj, c2[q], t.x0 - 1, t.y0 - 1, kWaveRX + 2, t.ry + 2);
-                off |= r.on ? 0u : 1u << (2 * k + q);
+                const Near r = trace_of(k, q, gj, c2[q]);
+                off |= __ballot(!r.on);
                 const float2 *F = reinterpret_cast<const float2 *>(lds) + (r.on ? r.ry * VP + r.rx : 0u);
                 const float2 f00 = F[0], f10 = F[1], f01 = F[VP], f11 = F[VP + 1];
                 u[k][q] = bilerp(r.sx, r.sy, f00.x, f10.x, f01.x, f11.x);
@@ -201,13 +205,13 @@ __device__ __forceinline__ void diffuse_wave(const DiffuseArgs &a, int tile) {
             gj = t.next_row(gj, a.h);
             __builtin_amdgcn_sched_barrier(0);  // one row's corners in registers at a time
         }
-        if (__any(off != 0)) {
+        if (off != 0) {
 #pragma unroll 1
             for (int m = 0; m < 2 * S; ++m) {
-                if (!((off >> m) & 1u)) continue;
                 const int k = m >> 1, q = m & 1;
                 const float2 c = V[(t.r0 + k) * VP + 2 * t.lane + q];
                 const int row = wrap_index(t.y0 + t.r0 + k, a.h);
+                if ((q ? trace_of(k, 1, row, c) : trace_of(k, 0, row, c)).on) continue;
                 const float2 n = far_advect(a, q ? t.gi[1] : t.gi[0], row, c);
 #pragma unroll
                 for (int kk = 0; kk < S; ++kk)
