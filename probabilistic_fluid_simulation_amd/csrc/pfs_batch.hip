@@ -342,7 +342,7 @@ struct pfs_batch {
                         const int cur = (int)((s.cur(t_build) + q) & 1);
                         PressureArgs a = p[k];
                         pressure_chunk(a, c, g.plan[c], s.ws, s.dye_fused ? s.dye[cur].data : nullptr,
-                                       s.dye_fused ? s.dye[cur ^ 1].data : nullptr);
+                                       s.dye_fused ? s.dye[cur ^ 1].data : nullptr, g.nchunks);
                         std::memcpy(img.data() + o.ptab[q][c] + k * sizeof(PressureArgs), &a,
                                     sizeof(a));
                     }

@@ -86,26 +86,28 @@ __global__ __launch_bounds__(kWaveMax * 64, S == 2 ? 8 : 6) void k_pressure_op(P
 using DiffuseFn = void (*)(DiffuseArgs);
 using PressureFn = void (*)(PressureArgs);
 
-#define PFS_H_CASES(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9)
+// Halos of a last chunk; one that is not the last runs kMaxChunk or kLongChunk
+// sweeps.
+#define PFS_H_CASES(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11)
 
 DiffuseFn diffuse_small_for(int H, bool last) {
+    if (!last) return H == kLongChunk ? k_diffuse<kLongChunk, false> : k_diffuse<kMaxChunk, false>;
     switch (H) {
 #define PFS_CASE(h) \
     case h:         \
-        return last ? k_diffuse<h, true> : k_diffuse<h, false>;
+        return k_diffuse<h, true>;
         PFS_H_CASES(PFS_CASE)
 #undef PFS_CASE
     }
     return nullptr;
 }
 
-// A chunk that is not the last runs kMaxChunk sweeps.
 template <int S>
 DiffuseFn diffuse_wave_for(int H, bool first, bool last) {
+    if (!last && H == kLongChunk)
+        return first ? k_diffuse_wave<kLongChunk, true, false, S> : k_diffuse_wave<kLongChunk, false, false, S>;
     if (!last)
-        return H != kMaxChunk ? nullptr
-                              : first ? k_diffuse_wave<kMaxChunk, true, false, S>
-                                      : k_diffuse_wave<kMaxChunk, false, false, S>;
+        return first ? k_diffuse_wave<kMaxChunk, true, false, S> : k_diffuse_wave<kMaxChunk, false, false, S>;
     switch (H) {
 #define PFS_CASE(h) \
     case h:         \
@@ -118,10 +120,11 @@ DiffuseFn diffuse_wave_for(int H, bool first, bool last) {
 
 template <int TS>
 PressureFn pressure_for_ts(int H, bool last) {
+    if (!last) return H == kLongChunk ? k_pressure<kLongChunk, false, TS> : k_pressure<kMaxChunk, false, TS>;
     switch (H) {
 #define PFS_CASE(h) \
     case h:         \
-        return last ? k_pressure<h, true, TS> : k_pressure<h, false, TS>;
+        return k_pressure<h, true, TS>;
         PFS_H_CASES(PFS_CASE)
 #undef PFS_CASE
     }
@@ -159,28 +162,39 @@ WaveShape wave_args(Args &d, int H) {
 // An operator's sweeps in launches.  The first reads the field and writes
 // planes, the last reads planes and writes both fields (a launch that read a
 // field and wrote one would race with its own halo reads), so there are at
-// least two: 4 + the rest up to 8 sweeps, else 8 at a time and the rest last.
+// least two: 4 + the rest up to 8 sweeps, else 8 (or 10, sweeps_per_launch) at a
+// time and the rest last.
 struct OpPlan {
     int first, middles, last;
 };
-OpPlan op_plan(int iters) {
+OpPlan op_plan(int iters, int w, int h) {
     if (iters <= kMaxChunk) return {4, 0, iters - 4};
-    const int rest = (iters - 1) % kMaxChunk + 1;
-    return {kMaxChunk, (iters - rest) / kMaxChunk - 1, rest};
+    int n = kMaxChunk;
+    if (iters > kLongChunk) {
+        DiffuseArgs longer{};
+        longer.w = w;
+        longer.h = h;
+        (void)wave_args(longer, kLongChunk);
+        n = sweeps_per_launch(iters, longer.ntiles <= device_cus());
+    }
+    const int rest = (iters - 1) % n + 1;
+    return {n, (iters - rest) / n - 1, rest};
 }
 
 template <int S>
 DiffuseFn diffuse_op_for(int ns, From from, To to) {
     if (to == To::Plane) {
-        if (from == From::Plane) return k_diffuse_wave<kMaxChunk, false, false, S>;
-        return ns == 4 ? k_diffuse_op<4, From::Field, To::Plane, S>
-                       : k_diffuse_op<kMaxChunk, From::Field, To::Plane, S>;
+        if (from == From::Plane) return diffuse_wave_for<S>(ns, false, false);
+        return ns == 4           ? k_diffuse_op<4, From::Field, To::Plane, S>
+               : ns == kMaxChunk ? k_diffuse_op<kMaxChunk, From::Field, To::Plane, S>
+                                 : k_diffuse_op<kLongChunk, From::Field, To::Plane, S>;
     }
     switch (ns) {
 #define PFS_CASE(n) \
     case n:         \
         return k_diffuse_op<n, From::Plane, To::Field, S>;
         PFS_CASE(1) PFS_CASE(2) PFS_CASE(3) PFS_CASE(4) PFS_CASE(5) PFS_CASE(6) PFS_CASE(7) PFS_CASE(8)
+        PFS_CASE(9) PFS_CASE(10)
 #undef PFS_CASE
     }
     return nullptr;
@@ -189,15 +203,19 @@ DiffuseFn diffuse_op_for(int ns, From from, To to) {
 template <int S>
 PressureFn pressure_op_for(int ns, From from, To to) {
     if (to == To::Plane) {
-        if (from == From::Plane) return k_pressure_op<kMaxChunk, From::Plane, To::Plane, S>;
-        return ns == 4 ? k_pressure_op<4, From::Field, To::Plane, S>
-                       : k_pressure_op<kMaxChunk, From::Field, To::Plane, S>;
+        if (from == From::Plane)
+            return ns == kMaxChunk ? k_pressure_op<kMaxChunk, From::Plane, To::Plane, S>
+                                   : k_pressure_op<kLongChunk, From::Plane, To::Plane, S>;
+        return ns == 4           ? k_pressure_op<4, From::Field, To::Plane, S>
+               : ns == kMaxChunk ? k_pressure_op<kMaxChunk, From::Field, To::Plane, S>
+                                 : k_pressure_op<kLongChunk, From::Field, To::Plane, S>;
     }
     switch (ns) {
 #define PFS_CASE(n) \
     case n:         \
         return k_pressure_op<n, From::Plane, To::Field, S>;
         PFS_CASE(1) PFS_CASE(2) PFS_CASE(3) PFS_CASE(4) PFS_CASE(5) PFS_CASE(6) PFS_CASE(7) PFS_CASE(8)
+        PFS_CASE(9) PFS_CASE(10)
 #undef PFS_CASE
     }
     return nullptr;
@@ -215,19 +233,23 @@ size_t fused_workspace_bytes(int w, int h) {
 
 int fused_step(const StepArgs &s, float *ws, hipStream_t stream, hipEvent_t *ev, int reps) {
     if (s.iters < 1) return set_error(PFS_ERR_INVALID, "fused step needs iters >= 1");
-    Chunk plan[64];
-    const int nchunks = chunk_plan(s.iters, plan, 64);
-    if (plan[nchunks - 1].last == false)
+    Chunk plan[64], pplan[64];  // the diffusion's and the pressure's launches
+    if (s.iters > 64 * kMaxChunk)
         return set_error(PFS_ERR_UNSUPPORTED, "iters too large for one step plan");
     if (!valid_tile_side(s.tile)) return set_error(PFS_ERR_INVALID, "tile side must be 16, 32 or 64");
     DiffuseArgs d = diffuse_args(s.P, s.Q, s.w, s.h, s.dt, s.visc, s.iters, ws, s.tile);
     PressureArgs p = pressure_args(s.P, s.Q, s.image, s.itmp, s.w, s.h, s.dt, ws, s.tile);
     const dim3 grid(d.ntiles);
+    DiffuseArgs longer = d;
+    if (s.tile != 16) (void)wave_args(longer, kLongChunk);
+    const int nd = chunk_plan(s.iters, plan, 64,
+                              sweeps_per_launch(s.iters, s.tile != 16 && longer.ntiles <= device_cus()));
+    const int np = chunk_plan(s.iters, pplan, 64, sweeps_per_launch(s.iters, d.ntiles <= device_cus()));
 
     if (!ev) reps = 1;
     if (ev) PFS_HIP_TRY(hipEventRecord(ev[0], stream));
     for (int r = 0; r < reps; ++r)
-        for (int c = 0; c < nchunks; ++c) {
+        for (int c = 0; c < nd; ++c) {
             diffuse_chunk(d, c, plan[c], ws);
             const Chunk &k = plan[c];
             if (s.tile == 16) {
@@ -245,15 +267,15 @@ int fused_step(const StepArgs &s, float *ws, hipStream_t stream, hipEvent_t *ev,
     if (ev) PFS_HIP_TRY(hipEventRecord(ev[1], stream));
     if (ev) PFS_HIP_TRY(hipEventRecord(ev[2], stream));
     for (int r = 0; r < reps; ++r)
-        for (int c = 0; c < nchunks; ++c) {
-            pressure_chunk(p, c, plan[c], ws, s.image, s.itmp);
-            const Chunk &k = plan[c];
+        for (int c = 0; c < np; ++c) {
+            pressure_chunk(p, c, pplan[c], ws, s.image, s.itmp, nd);
+            const Chunk &k = pplan[c];
             PressureArgs w = p;
             // Only whole chunks of fields with two workgroups for every CU:
             // below that the square tiles are as fast (2048^2: 22.5 us against
             // 24; 1024^2: equal).
             const WaveShape sh = k.last || s.tile != 64 ? WaveShape{0, 0} : wave_args(w, k.H);
-            if (sh.S == 4 && w.ntiles >= 2 * device_cus())
+            if (sh.S == 4 && k.H == kMaxChunk && w.ntiles >= 2 * device_cus())
                 hipLaunchKernelGGL(k_pressure_wave, dim3(w.ntiles), dim3(64 * sh.nw), 0, stream, w);
             else
                 hipLaunchKernelGGL(pressure_for(k.H, k.last, s.tile), grid,
@@ -273,10 +295,10 @@ int diffuse_op(const float *a, float *last, float *before, int w, int h, float d
     DiffuseArgs d = diffuse_args(a, a, w, h, dt, visc, iters, ws);
     d.field[0] = last;
     d.field[1] = before;
-    const OpPlan plan = op_plan(iters);
+    const OpPlan plan = op_plan(iters, w, h);
     const int n = plan.middles + 2;
     for (int c = 0; c < n; ++c) {
-        const int ns = c == 0 ? plan.first : c == n - 1 ? plan.last : kMaxChunk;
+        const int ns = c == 0 ? plan.first : c == n - 1 ? plan.last : plan.first;
         const From from = c == 0 ? From::Field : From::Plane;
         const To to = c == n - 1 ? To::Field : To::Plane;
         diffuse_chunk(d, c, Chunk{ns, ns, c == 0, c == n - 1}, ws);
@@ -295,13 +317,13 @@ int pressure_op(float *a, float *last, float *before, int w, int h, float dt, in
     p.bdst = ws + (size_t)w * h;  // what bpl reads
     p.field[0] = last;
     p.field[1] = before;
-    const OpPlan plan = op_plan(iters);
+    const OpPlan plan = op_plan(iters, w, h);
     const int n = plan.middles + 2;
     for (int c = 0; c < n; ++c) {
-        const int ns = c == 0 ? plan.first : c == n - 1 ? plan.last : kMaxChunk;
+        const int ns = c == 0 ? plan.first : c == n - 1 ? plan.last : plan.first;
         const From from = c == 0 ? From::Field : From::Plane;
         const To to = c == n - 1 ? To::Field : To::Plane;
-        pressure_chunk(p, c, Chunk{ns, ns, false, c == n - 1}, ws, nullptr, nullptr);
+        pressure_chunk(p, c, Chunk{ns, ns, false, c == n - 1}, ws, nullptr, nullptr, 1);
         const WaveShape sh = wave_args(p, ns);
         hipLaunchKernelGGL(sh.S == 2 ? pressure_op_for<2>(ns, from, to) : pressure_op_for<4>(ns, from, to),
                            dim3(p.ntiles), dim3(64 * sh.nw), 0, stream, p);

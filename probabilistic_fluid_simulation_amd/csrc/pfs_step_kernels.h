@@ -11,19 +11,21 @@ namespace pfs {
 constexpr int kTile = 64;    // the largest tile side (the default)
 constexpr int kSegs = 12;    // row segments per staged column of a 64-wide tile
 constexpr int kMaxChunk = 8; // sweeps per launch
+constexpr int kLongChunk = 10;  // where that saves a launch (sweeps_per_launch)
 
 template <int H_, int TS_ = kTile, int NTMAX = 1024>
 struct Geo {
     static constexpr int H = H_;
     static constexpr int TX = TS_, TY = TS_;
     static constexpr int RX = TX + 2 * H, RY = TY + 2 * H;
-    // Rows per thread: a 64-wide tile keeps 12 segments per column; smaller
-    // tiles take as many segments as 1024 threads allow, rows split evenly.
+    // Rows per thread: a 64-wide tile keeps 12 segments per column where 1024
+    // threads allow; smaller tiles take as many segments as 1024 threads allow, rows split evenly.
     // NTMAX < 1024: workgroups of at most NTMAX threads (longer strips), so
     // that two fit a CU.
-    static constexpr int MAXSEG = (TS_ == kTile && NTMAX == 1024) ? kSegs : NTMAX / RX;
+    static constexpr bool TWELVE = TS_ == kTile && NTMAX == 1024 && kSegs * RX <= NTMAX;
+    static constexpr int MAXSEG = TWELVE ? kSegs : NTMAX / RX;
     static constexpr int S = (RY + MAXSEG - 1) / MAXSEG;
-    static constexpr int SEGS = (TS_ == kTile && NTMAX == 1024) ? kSegs : (RY + S - 1) / S;
+    static constexpr int SEGS = TWELVE ? kSegs : (RY + S - 1) / S;
     static constexpr int RYP = SEGS * S;                // rows of an LDS plane (>= RY)
     static constexpr int NTH = RX * SEGS;               // threads owning cells
     static constexpr int NT = ((NTH + 63) / 64) * 64;   // whole wavefronts
@@ -555,6 +557,18 @@ inline size_t scene_ws_floats(int w, int h, int iters) {
     return (iters > kMaxChunk ? 8 : 4) * (size_t)w * (size_t)h;
 }
 
+// Sweeps per launch of a step's diffusion or pressure, or of an operator's.
+// kLongChunk where all sweeps then fit one launch (9 or 10 sweeps, diffusion +
+// pressure: 128^2 13.5 -> 10.8 us, 1024^2 46.6 -> 38.8, 3840x2160 309 -> 263),
+// and where it saves one of several and its tiles leave CUs `idle`, so that the
+// wider halos cost no time (20 sweeps: 611x397 40.2 -> 36.1 us, 1024^2 70 -> 64;
+// 30: 1024^2 92 -> 86; with more tiles than CUs the halos cost more than a
+// launch: 2048^2 at 30 253 -> 262).
+inline int sweeps_per_launch(int iters, bool idle) {
+    const int few = (iters + kLongChunk - 1) / kLongChunk, many = (iters + kMaxChunk - 1) / kMaxChunk;
+    return few == 1 || (idle && few < many) ? kLongChunk : kMaxChunk;
+}
+
 // The launch sequence of one step: chunk c runs ns sweeps with halo H.
 struct Chunk {
     int ns, H;
@@ -653,11 +667,12 @@ inline PressureArgs pressure_args(float *P, float *Q, const float *image, float 
     return p;
 }
 
+// nd: the diffusion's chunks, the last of which left E.
 inline void pressure_chunk(PressureArgs &p, int c, const Chunk &ch, float *ws,
-                           const float *image, float *itmp) {
+                           const float *image, float *itmp, int nd) {
     const size_t N = (size_t)p.w * p.h;
     float *ppl[2] = {ws + 6 * N, ws + 7 * N};
-    p.E = reinterpret_cast<const float2 *>(ws + 2 * N + 2 * N * (c & 1));
+    p.E = reinterpret_cast<const float2 *>(ws + 2 * N + 2 * N * ((nd - 1) & 1));
     p.first = ch.first;
     p.psrc = ppl[(c + 1) & 1];
     p.pdst = ppl[c & 1];

@@ -335,6 +335,20 @@ def test_wave_tiles_bitexact(orc, shape, k):
     assert_bitexact(gpu_run(s, 1, combined=True), oracle_run(orc, s, 1))
 
 
+@pytest.mark.parametrize("k", [9, 10, 11, 17, 20, 25, 30, 31])
+@pytest.mark.parametrize("shape", [(53, 37), (333, 250), (700, 520), (1801, 1310)])
+def test_launches_of_ten_sweeps(orc, shape, k):
+    """9 and 10 sweeps are one launch, and more go 10 at a time where that
+    saves a launch and leaves CUs idle (diffusion and pressure choose apart):
+    the step with its dye, and both operators, on either side of those lines."""
+    if shape[0] > 1000 and k not in (9, 10, 20):
+        pytest.skip("three counts on the large field")
+    s = scenes.random_scene(*shape, *shape, seed=100 + k, dt=0.5, visc=0.15, iters=k, vel_scale=40.0)
+    assert_bitexact(gpu_run(s, 2, combined=True), oracle_run(orc, s, 2))
+    got, want = _both_operators(orc, s, k)
+    assert_bitexact(got, want, ("d.vp", "d.out", "p.vp", "p.out"))
+
+
 @pytest.mark.parametrize("visc", [0.0, 0.1, 0.113, 2.5, 40.0, 1e9, -0.4])
 def test_wave_tiles_every_division(orc, visc):
     """Every form of the sweep's division: two operations (proven divisors),
