@@ -875,7 +875,7 @@ int precise_step(float *P, float *Q, int w, int h, float dt, float visc, int K, 
         } else {
             DiffuseArgs wd = d;
             const WaveShape sh =
-                wave_shape(k.H, device_cus(), [&](WaveShape x) { return wave_tiles(w, h, k.H, x); });
+                wave_shape(k.H, device_cus(), [&](WaveShape x) { return wave_tiles(w, h, k.H, x); }, 16);
             wd.tiles_x = wave_tiles_x(w, k.H);
             wd.ntiles = (int)wave_tiles(w, h, k.H, sh);
             hipLaunchKernelGGL(sh.S == 2 ? diffuse_precise_wave<2>(k.H, k.first, k.last)

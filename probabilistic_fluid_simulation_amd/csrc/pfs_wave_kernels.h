@@ -598,15 +598,18 @@ inline long long wave_tiles(int w, int h, int H, WaveShape s) {
 //     16 waves of 2 rows, 10.8 with 8 of 4; 611x397, 30 sweeps: 29 us against 34);
 //   - else 4 rows per wave, likewise (1024^2, 8 sweeps: 20.2 us with 15 waves,
 //     250 tiles; 21.1 with 12, 350 tiles);
-//   - else 12 waves of 4 rows, two workgroups per CU, one's memory phases
-//     under the other's sweeps (2048^2, 8 sweeps: 54 us; 67 with 16 waves,
-//     which leave no room for a second workgroup).
+//   - else `many` waves of 4 rows: 12 make two workgroups per CU, one's memory
+//     phases under the other's sweeps (2048^2, 8 sweeps: 54 us; 67 with 16 waves,
+//     which leave no room for a second workgroup); the compensated sums, with
+//     twice the arithmetic, gain more from 16 waves' narrower share of halo
+//     rows (a precise step of 16 + 16 sweeps at 3840x2160 569 -> 539 us, at
+//     2048^2 304 -> 303).
 template <typename Count>
-WaveShape wave_shape(int H, int cus, Count &&count) {
+WaveShape wave_shape(int H, int cus, Count &&count, int many = 12) {
     for (int S = 2; S <= 4; S += 2)
         for (int nw = (2 * H + 4 + S - 1) / S; nw <= kWaveMax; ++nw)
             if (count(WaveShape{S, nw}) <= cus) return {S, nw};
-    return {4, 12};
+    return {4, many};
 }
 
 }  // namespace pfs
