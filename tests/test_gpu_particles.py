@@ -30,6 +30,11 @@ def test_scan_exclusive(n):
     assert total == int(a.sum())
 
 
+@pytest.mark.parametrize("n", [4096 * 8 - 1, 4096 * 8, 4096 * 8 + 1])
+def test_scan_in_one_and_two_launches(n):
+    test_scan_exclusive(n)
+
+
 def _positions(n, W, H, seed):
     rng = np.random.default_rng(seed)
     x = np.minimum((rng.random(n) * W).astype(np.float32), np.nextafter(np.float32(W), np.float32(0)))
