@@ -165,15 +165,16 @@ int pfs_fluid_run(pfs_field *vp, pfs_field *tmp, pfs_field *image, pfs_field *it
 int pfs_set_step_path(int path);
 int pfs_get_step_path(void);
 
-/* Tile side of the fused step's workgroups (process-wide).  No counterpart
+/* Tile class of the fused step's workgroups (process-wide).  No counterpart
  * in the reference, whose CUDA kernels use fixed 16x16 blocks
- * (src/fluid.cu:14-15).  Each workgroup of the fused kernels owns a side x
- * side tile of cells; results do not depend on the side.  Unless forced
- * here, a step takes the side pfs_autotune_step measured fastest for its
- * shape (field size, iters, dye fused or not), else the largest side whose
- * tiles fill every CU (a small field: 16).  side 0 clears a forced side. */
+ * (src/fluid.cu:14-15).  A workgroup of the square-tile kernels owns a tile of
+ * 8 to 24 cells a side (class 16), 32 to 40 (class 32) or 48 to 64 (class 64),
+ * the smallest of its class whose tiles the CUs hold at once; results do not
+ * depend on it.  Unless forced here, a step takes the class pfs_autotune_step
+ * measured fastest for its shape (field size, iters, dye fused or not), else
+ * the first that has such a side.  side 0 clears a forced class. */
 int pfs_set_step_tile(int side);
-/* The side a step of this shape takes now (16, 32 or 64), or < 0 on error. */
+/* The class a step of this shape takes now (16, 32 or 64), or < 0 on error. */
 int pfs_get_step_tile(int vx, int vy, int iters, int dye_fused);
 /* Times pfs_fluid_timestep (image/itmp NULL: pfs_simulate_fluid_step) on
  * scratch copies of the buffers, `reps` steps per side after one untimed

@@ -140,7 +140,10 @@ long long tile_count(int w, int h, int ts) {
 }
 
 namespace {
-int rule_tile(int w, int h) { return tile_for_counts(tile_count(w, h, 64), tile_count(w, h, 32)); }
+// The class whose sides (tile_side) let the CUs hold every tile at once.
+int rule_tile(int w, int h) {
+    return tile_count(w, h, 24) <= device_cus() ? 16 : tile_count(w, h, 40) <= device_cus() ? 32 : 64;
+}
 
 int step_tile(int w, int h, int iters, bool dye_fused) {
     if (const int forced = g_step_tile.load()) return forced;

@@ -1,7 +1,7 @@
 // Fused, temporally blocked fluid step for gfx950.
 //
 // One call of the reference's simulate_fluid_step (src/fluid.cpp:298-310)
-// is 2K+3 full-grid passes there.  Here it is two kernels (for K <= 8):
+// is 2K+3 full-grid passes there.  Here it is two kernels (for K <= 10):
 //
 //   D: advect (src/fluid.cpp:24-70) + K diffusion sweeps (:129-196) +
 //      divergence (:221-237), temporally blocked in LDS;
@@ -13,20 +13,20 @@
 // Each workgroup owns a tile of cells and stages it plus a halo of H = sweeps
 // (+1 for the final stencil) cells, periodic wrap folded into the staged
 // coordinates.  Two forms:
-//   - square tiles (64, 32 or 16 wide: kernel P, and kernel D at side 16;
-//     pfs_step_kernels.h): thread (x, seg) owns column x of the staged region,
+//   - square tiles (8 to 64 wide: kernel P, and kernel D on small fields, up to
+//     side 24; pfs_step_kernels.h): thread (x, seg) owns column x of the staged region,
 //     rows [seg*S, seg*S + S), in registers; every sweep it publishes its cells
 //     (alpha-scaled for diffusion) to an LDS plane, waits at one barrier
 //     (planes alternate), and updates its cells from the left/right columns in
 //     LDS and its own registers above and below;
-//   - wave tiles (kernel D on every field past side 16; pfs_wave_kernels.h):
+//   - wave tiles (kernel D on every larger field; pfs_wave_kernels.h):
 //     a wavefront owns whole rows and takes its horizontal neighbours by DPP.
 // Cells of the outer ring read clamped or missing neighbours and become
 // garbage; that ring grows by one cell per sweep exactly as the valid region
 // shrinks, so the tile is never touched by it.  Halo cells are recomputed by
 // both neighbouring tiles with the same operations in the same order: every
-// value is bit-identical to the reference's global sweep.  For K > 8 the
-// sweeps run in chunks of 8 with the iterate in workspace planes between
+// value is bit-identical to the reference's global sweep.  For K > 10 the
+// sweeps run in chunks of 8 or 10 with the iterate in workspace planes between
 // chunks.
 //
 // Buffer contract (equal to fluid.cpp's, derived from its pointer swaps):
@@ -39,31 +39,21 @@
 // both outputs whole (32 B per cell) without reading them.
 
 #include <cmath>
+#include <initializer_list>
 
 #include "pfs_internal.h"
-#include "pfs_step_kernels.h"
+#include "pfs_step_launch.h"
 #include "pfs_wave_kernels.h"
 
 namespace pfs {
 
 namespace {
 
-// Side 16 (small fields).
-template <int H, bool LAST>
-__global__ __launch_bounds__((Geo<H, 16>::NT)) void k_diffuse(DiffuseArgs a) {
-    diffuse_tile<H, LAST, 16>(a, xcd_tile(blockIdx.x, a.ntiles));
-}
-
 // Larger fields.
 template <int H, bool FIRST, bool LAST, int S>
 __global__ __launch_bounds__(kWaveMax * 64, S == 2 ? 8 : 6) void k_diffuse_wave(DiffuseArgs a) {
     diffuse_wave<H, FIRST ? From::Advect : From::Plane, LAST ? To::Step : To::Plane, S>(
         a, xcd_tile(blockIdx.x, a.ntiles));
-}
-
-template <int H, bool LAST, int TS>
-__global__ __launch_bounds__((Geo<H, TS>::NT)) void k_pressure(PressureArgs a) {
-    pressure_tile<H, LAST, TS>(a, xcd_tile(blockIdx.x, a.ntiles));
 }
 
 // Chunks of the pressure that are not the last, on larger fields.
@@ -83,25 +73,6 @@ __global__ __launch_bounds__(kWaveMax * 64, S == 2 ? 8 : 6) void k_pressure_op(P
 }
 
 // ---- host dispatch over the compile-time halo and tile side ----------------
-using DiffuseFn = void (*)(DiffuseArgs);
-using PressureFn = void (*)(PressureArgs);
-
-// Halos of a last chunk; one that is not the last runs kMaxChunk or kLongChunk
-// sweeps.
-#define PFS_H_CASES(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(11)
-
-DiffuseFn diffuse_small_for(int H, bool last) {
-    if (!last) return H == kLongChunk ? k_diffuse<kLongChunk, false> : k_diffuse<kMaxChunk, false>;
-    switch (H) {
-#define PFS_CASE(h) \
-    case h:         \
-        return k_diffuse<h, true>;
-        PFS_H_CASES(PFS_CASE)
-#undef PFS_CASE
-    }
-    return nullptr;
-}
-
 template <int S>
 DiffuseFn diffuse_wave_for(int H, bool first, bool last) {
     if (!last && H == kLongChunk)
@@ -118,22 +89,15 @@ DiffuseFn diffuse_wave_for(int H, bool first, bool last) {
     return nullptr;
 }
 
-template <int TS>
-PressureFn pressure_for_ts(int H, bool last) {
-    if (!last) return H == kLongChunk ? k_pressure<kLongChunk, false, TS> : k_pressure<kMaxChunk, false, TS>;
-    switch (H) {
-#define PFS_CASE(h) \
-    case h:         \
-        return k_pressure<h, true, TS>;
-        PFS_H_CASES(PFS_CASE)
+PressureFn pressure_for(int H, bool last, int ts) {
+    switch (ts) {
+#define PFS_CASE(t) \
+    case t:         \
+        return pressure_for_ts<t>(H, last);
+        PFS_LARGE_SIDES(PFS_CASE)
 #undef PFS_CASE
     }
-    return nullptr;
-}
-
-PressureFn pressure_for(int H, bool last, int ts) {
-    return ts == 16 ? pressure_for_ts<16>(H, last)
-                    : ts == 32 ? pressure_for_ts<32>(H, last) : pressure_for_ts<64>(H, last);
+    return pressure_small_for(H, last, ts);
 }
 
 template <int TS>
@@ -224,11 +188,39 @@ PressureFn pressure_op_for(int ns, From from, To to) {
 }  // namespace
 
 int threads_for(int H, int ts) {
-    return ts == 16 ? threads_for_ts<16>(H) : ts == 32 ? threads_for_ts<32>(H) : threads_for_ts<64>(H);
+    switch (ts) {
+#define PFS_CASE(t) \
+    case t:         \
+        return threads_for_ts<t>(H);
+        PFS_SMALL_SIDES(PFS_CASE)
+        PFS_LARGE_SIDES(PFS_CASE)
+#undef PFS_CASE
+    }
+    return 0;
 }
 
 size_t fused_workspace_bytes(int w, int h) {
     return scene_ws_floats(w, h, kMaxChunk + 1) * sizeof(float);
+}
+
+// The side of the square tiles for a step of tile class `tile`: the smallest of
+// the class whose tiles the CUs hold at once.  Small tiles keep a launch's
+// chain of phases short, a second round of workgroups on part of the CUs costs
+// up to half the launch again.  Diffusion + pressure at 8 sweeps, us, by side:
+// 128^2 8: 8.7, 12: 9.3, 16: 10.2; 320x240 16 (300 tiles): 13.8, 20: 11.5, 24:
+// 12.4; 360^2 24: 13.1, 32: 15.2.  The pressure alone: 611x397 32 (260 tiles) 12.8,
+// 36: 8.7; 800x600 48: 12.2, 56: 13.6, 64: 15.2; 1200x1024, more than a tile a CU
+// at 64 (30.0), 56: 22.1.
+int tile_side(int tile, int w, int h) {
+    auto smallest = [&](std::initializer_list<int> sides, int limit) {
+        for (int side : sides)
+            if (tile_count(w, h, side) <= limit) return side;
+        return tile;
+    };
+    if (tile == 16) return smallest({8, 12, 16, 20, 24}, device_cus());
+    if (tile == 32) return smallest({32, 36, 40}, device_cus());
+    const int side = smallest({48, 56}, device_cus());
+    return side != 64 || tile_count(w, h, 64) <= device_cus() ? side : smallest({56}, 2 * device_cus());
 }
 
 int fused_step(const StepArgs &s, float *ws, hipStream_t stream, hipEvent_t *ev, int reps) {
@@ -237,13 +229,15 @@ int fused_step(const StepArgs &s, float *ws, hipStream_t stream, hipEvent_t *ev,
     if (s.iters > 64 * kMaxChunk)
         return set_error(PFS_ERR_UNSUPPORTED, "iters too large for one step plan");
     if (!valid_tile_side(s.tile)) return set_error(PFS_ERR_INVALID, "tile side must be 16, 32 or 64");
-    DiffuseArgs d = diffuse_args(s.P, s.Q, s.w, s.h, s.dt, s.visc, s.iters, ws, s.tile);
-    PressureArgs p = pressure_args(s.P, s.Q, s.image, s.itmp, s.w, s.h, s.dt, ws, s.tile);
+    const bool small = s.tile == 16;
+    const int side = tile_side(s.tile, s.w, s.h);
+    DiffuseArgs d = diffuse_args(s.P, s.Q, s.w, s.h, s.dt, s.visc, s.iters, ws, side);
+    PressureArgs p = pressure_args(s.P, s.Q, s.image, s.itmp, s.w, s.h, s.dt, ws, side);
     const dim3 grid(d.ntiles);
     DiffuseArgs longer = d;
-    if (s.tile != 16) (void)wave_args(longer, kLongChunk);
+    if (!small) (void)wave_args(longer, kLongChunk);
     const int nd = chunk_plan(s.iters, plan, 64,
-                              sweeps_per_launch(s.iters, s.tile != 16 && longer.ntiles <= device_cus()));
+                              sweeps_per_launch(s.iters, !small && longer.ntiles <= device_cus()));
     const int np = chunk_plan(s.iters, pplan, 64, sweeps_per_launch(s.iters, d.ntiles <= device_cus()));
 
     if (!ev) reps = 1;
@@ -252,9 +246,9 @@ int fused_step(const StepArgs &s, float *ws, hipStream_t stream, hipEvent_t *ev,
         for (int c = 0; c < nd; ++c) {
             diffuse_chunk(d, c, plan[c], ws);
             const Chunk &k = plan[c];
-            if (s.tile == 16) {
-                hipLaunchKernelGGL(diffuse_small_for(k.H, k.last), grid,
-                                   dim3(threads_for(k.H, s.tile)), 0, stream, d);
+            if (small) {
+                hipLaunchKernelGGL(diffuse_small_for(k.H, k.last, side), grid,
+                                   dim3(threads_for(k.H, side)), 0, stream, d);
             } else {
                 DiffuseArgs w = d;
                 const WaveShape sh = wave_args(w, k.H);
@@ -278,8 +272,8 @@ int fused_step(const StepArgs &s, float *ws, hipStream_t stream, hipEvent_t *ev,
             if (sh.S == 4 && k.H == kMaxChunk && w.ntiles >= 2 * device_cus())
                 hipLaunchKernelGGL(k_pressure_wave, dim3(w.ntiles), dim3(64 * sh.nw), 0, stream, w);
             else
-                hipLaunchKernelGGL(pressure_for(k.H, k.last, s.tile), grid,
-                                   dim3(threads_for(k.H, s.tile)), 0, stream, p);
+                hipLaunchKernelGGL(pressure_for(k.H, k.last, side), grid,
+                                   dim3(threads_for(k.H, side)), 0, stream, p);
             PFS_TRY(check_launch("fused pressure"));
         }
     if (ev) PFS_HIP_TRY(hipEventRecord(ev[3], stream));

@@ -349,6 +349,20 @@ def test_launches_of_ten_sweeps(orc, shape, k):
     assert_bitexact(got, want, ("d.vp", "d.out", "p.vp", "p.out"))
 
 
+@pytest.mark.parametrize("k", [1, 8, 10, 13])
+@pytest.mark.parametrize("shape", [(101, 83), (181, 150), (251, 240), (311, 300), (371, 330),
+                                   (500, 401), (601, 430), (641, 620), (761, 700), (881, 870),
+                                   (1001, 980), (1201, 1023)],
+                         ids=["8", "12", "16", "20", "24", "32", "36", "40", "48", "56", "64", "56-large"])
+def test_every_side_of_the_square_tiles(orc, shape, k):
+    """The automatic choice from 8 to 64 cells a side, partial tiles on both
+    edges, one launch and several, the dye within the last."""
+    if shape[0] > 700 and k in (1, 10):
+        pytest.skip("two counts on the large fields")
+    s = scenes.random_scene(*shape, *shape, seed=120 + k, dt=0.5, visc=0.15, iters=k, vel_scale=40.0)
+    assert_bitexact(gpu_run(s, 1, combined=True), oracle_run(orc, s, 1))
+
+
 @pytest.mark.parametrize("visc", [0.0, 0.1, 0.113, 2.5, 40.0, 1e9, -0.4])
 def test_wave_tiles_every_division(orc, visc):
     """Every form of the sweep's division: two operations (proven divisors),
