@@ -70,7 +70,10 @@ int pfs_advect_color(const pfs_field *image, pfs_field *out, const pfs_field *vp
 
 /* includes/fluid.hpp:58 / src/fluid.cpp:129-196.  `iters` Jacobi smoothing
  * sweeps of channels 0,1 between vp and vp_out; swaps the two structs' data
- * pointers after every sweep but the last. */
+ * pointers after every sweep but the last.  From 5 sweeps on, 4-channel fields
+ * aligned to 16 bytes run several sweeps a launch in the stream's workspace
+ * (the step's); otherwise, and while the stream is being captured, each sweep
+ * is a launch.  Same results either way; pfs_compute_pressure likewise. */
 int pfs_diffuse(pfs_field *vp, pfs_field *vp_out, float viscosity, float dt, int iters,
                 void *stream);
 
@@ -172,9 +175,10 @@ int pfs_get_step_path(void);
  * the smallest of its class whose tiles the CUs hold at once; results do not
  * depend on it.  Unless forced here, a step takes the class pfs_autotune_step
  * measured fastest for its shape (field size, iters, dye fused or not), else
- * the first that has such a side.  side 0 clears a forced class. */
+ * the smallest such side of all.  side 0 clears a forced class. */
 int pfs_set_step_tile(int side);
-/* The class a step of this shape takes now (16, 32 or 64), or < 0 on error. */
+/* The class forced or measured for this shape, else the largest of 64, 32 and
+ * 16 with a tile for every two CUs (16 if none); < 0 on error. */
 int pfs_get_step_tile(int vx, int vy, int iters, int dye_fused);
 /* Times pfs_fluid_timestep (image/itmp NULL: pfs_simulate_fluid_step) on
  * scratch copies of the buffers, `reps` steps per side after one untimed

@@ -102,8 +102,9 @@ bool same_shape(const pfs_field *a, const pfs_field *b) {
     return a->x == b->x && a->y == b->y && a->z == b->z;
 }
 
-// Tile side of the fused step: the side pfs_set_step_tile forced, else the
-// side pfs_autotune_step measured fastest for this shape, else the rule.
+// Tile class of the fused step: the one pfs_set_step_tile forced, else the one
+// pfs_autotune_step measured fastest for this shape, else the step's own choice
+// (pfs_step.hip, tile_side).
 std::atomic<int> g_step_tile{0};  // 0: not forced
 std::mutex g_tune_mutex;
 std::map<std::tuple<int, int, int, int>, int> g_tuned;  // (w, h, iters, dye fused) -> side
@@ -111,25 +112,24 @@ std::map<std::tuple<int, int, int, int>, int> g_tuned;  // (w, h, iters, dye fus
 }  // namespace
 
 int device_cus() {
-    static std::mutex m;
-    static std::map<int, int> cus;
+    static std::atomic<int> known[64];  // by device; 0: not asked yet
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 256;
-    std::lock_guard<std::mutex> lock(m);
-    auto it = cus.find(dev);
-    if (it != cus.end()) return it->second;
+    const bool keep = dev >= 0 && dev < 64;
+    if (keep)
+        if (const int n = known[dev].load(std::memory_order_relaxed)) return n;
     int n = 0;
     if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1)
         n = 256;
-    cus[dev] = n;
+    if (keep) known[dev].store(n, std::memory_order_relaxed);
     return n;
 }
 
-// The rule: the largest side with at least one tile for every two CUs; a
-// field too small for that takes the smallest side, whose workgroups each
-// hold the fewest rows per thread.  (Measured on MI355X, 256 CUs: 64-wide
-// tiles win from 144 tiles up (768^2), 32-wide ones at 512^2, 16-wide ones
-// at 256^2 and below.)
+// The rule of the batched and the precision form, which have sides 64, 32 and
+// 16 only (and what pfs_get_step_tile reports of a shape neither forced nor
+// tuned): the largest side with at least one tile for every two CUs; a field too
+// small for that takes the smallest side, whose workgroups each hold the fewest
+// rows per thread.
 int tile_for_counts(long long tiles64, long long tiles32) {
     const long long half = device_cus() / 2;
     return tiles64 >= half ? 64 : tiles32 >= half ? 32 : 16;
@@ -140,19 +140,12 @@ long long tile_count(int w, int h, int ts) {
 }
 
 namespace {
-// The class whose sides (tile_side) let the CUs hold every tile at once.
-int rule_tile(int w, int h) {
-    return tile_count(w, h, 24) <= device_cus() ? 16 : tile_count(w, h, 40) <= device_cus() ? 32 : 64;
-}
-
-int step_tile(int w, int h, int iters, bool dye_fused) {
+// The class forced or tuned for a shape; 0: neither, the step chooses its side.
+int set_tile(int w, int h, int iters, bool dye_fused) {
     if (const int forced = g_step_tile.load()) return forced;
-    {
-        std::lock_guard<std::mutex> lock(g_tune_mutex);
-        auto it = g_tuned.find({w, h, iters, dye_fused ? 1 : 0});
-        if (it != g_tuned.end()) return it->second;
-    }
-    return rule_tile(w, h);
+    std::lock_guard<std::mutex> lock(g_tune_mutex);
+    auto it = g_tuned.find({w, h, iters, dye_fused ? 1 : 0});
+    return it != g_tuned.end() ? it->second : 0;
 }
 }  // namespace
 
@@ -376,7 +369,7 @@ static int timestep(pfs_field *vp, pfs_field *tmp, pfs_field *image, pfs_field *
     }
     StepArgs a{vp->data, tmp->data, dye_fused ? image->data : nullptr,
                dye_fused ? itmp->data : nullptr, vp->x, vp->y, dt, viscosity, iters,
-               tile ? tile : step_tile(vp->x, vp->y, iters, dye_fused)};
+               tile ? tile : set_tile(vp->x, vp->y, iters, dye_fused)};
     PFS_TRY(fused_step(a, ws, (hipStream_t)stream, ev, reps));
     if (!image) return PFS_OK;
     if (!dye_fused) return pfs_advect_color_step(image, itmp, vp, dt, stream);
@@ -495,7 +488,7 @@ int pfs_fluid_run(pfs_field *vp, pfs_field *tmp, pfs_field *image, pfs_field *it
     want.ws = lease.ptr;
     const bool dye_fused = image->x == vp->x && image->y == vp->y && image->z == 4 &&
                            aligned16(image->data) && aligned16(itmp->data);
-    want.tile = step_tile(vp->x, vp->y, iters, dye_fused);
+    want.tile = set_tile(vp->x, vp->y, iters, dye_fused);
 
     std::lock_guard<std::mutex> lock(g_graph_mutex);
     hipGraphExec_t exec = nullptr;
@@ -609,7 +602,8 @@ int pfs_set_step_tile(int side) {
 
 int pfs_get_step_tile(int vx, int vy, int iters, int dye_fused) {
     if (vx < 1 || vy < 1 || iters < 1) return set_error(PFS_ERR_INVALID, "bad step shape");
-    return step_tile(vx, vy, iters, dye_fused != 0);
+    const int tile = set_tile(vx, vy, iters, dye_fused != 0);
+    return tile ? tile : tile_for_counts(tile_count(vx, vy, 64), tile_count(vx, vy, 32));
 }
 
 int pfs_autotune_step(const pfs_field *vp, const pfs_field *tmp, const pfs_field *image,

@@ -78,10 +78,11 @@ int launch_advect_color_keys(const float *vp, int *keys, int iw, int ih, int vw,
                              float dt, hipStream_t s);
 
 // ---- fused step (pfs_step.hip) -------------------------------------------
-// Tile sides the fused kernels are built for.  A small field has few tiles
-// of the largest side, leaving most CUs idle; smaller tiles spread it over
-// more workgroups, each with fewer rows per thread, at the price of a
-// relatively wider halo.
+// Tile classes of the single-scene step (pfs_step.hip's tile_side gives the
+// side, 8 to 64), and the sides of the batched and the precision form.  A small
+// field has few tiles of a large side, leaving most CUs idle; smaller tiles
+// spread it over more workgroups, each with fewer rows per thread, at the price
+// of a relatively wider halo.
 constexpr int kTileSides[3] = {64, 32, 16};
 inline bool valid_tile_side(int ts) { return ts == 64 || ts == 32 || ts == 16; }
 int device_cus();  // CUs of the current device (256 if it does not answer)
@@ -97,7 +98,7 @@ struct StepArgs {
     int w, h;
     float dt, visc;
     int iters;
-    int tile;  // tile side of the fused kernels: 64, 32 or 16
+    int tile;  // tile class of the fused kernels: 64, 32 or 16; 0: any
 };
 // `ws` is a device workspace of fused_workspace_bytes(w, h).  Optional
 // per-kernel event timing: if `ev` is non-null, events ev[2k] and ev[2k+1]

@@ -203,8 +203,8 @@ size_t fused_workspace_bytes(int w, int h) {
     return scene_ws_floats(w, h, kMaxChunk + 1) * sizeof(float);
 }
 
-// The side of the square tiles for a step of tile class `tile`: the smallest of
-// the class whose tiles the CUs hold at once.  Small tiles keep a launch's
+// The side of the square tiles for a step: the smallest of its class (of all,
+// tile 0) whose tiles the CUs hold at once.  Small tiles keep a launch's
 // chain of phases short, a second round of workgroups on part of the CUs costs
 // up to half the launch again.  Diffusion + pressure at 8 sweeps, us, by side:
 // 128^2 8: 8.7, 12: 9.3, 16: 10.2; 320x240 16 (300 tiles): 13.8, 20: 11.5, 24:
@@ -212,15 +212,19 @@ size_t fused_workspace_bytes(int w, int h) {
 // 36: 8.7; 800x600 48: 12.2, 56: 13.6, 64: 15.2; 1200x1024, more than a tile a CU
 // at 64 (30.0), 56: 22.1.
 int tile_side(int tile, int w, int h) {
-    auto smallest = [&](std::initializer_list<int> sides, int limit) {
+    const int cus = device_cus();
+    auto smallest = [&](std::initializer_list<int> sides) {
         for (int side : sides)
-            if (tile_count(w, h, side) <= limit) return side;
-        return tile;
+            if (tile_count(w, h, side) <= cus) return side;
+        return 0;
     };
-    if (tile == 16) return smallest({8, 12, 16, 20, 24}, device_cus());
-    if (tile == 32) return smallest({32, 36, 40}, device_cus());
-    const int side = smallest({48, 56}, device_cus());
-    return side != 64 || tile_count(w, h, 64) <= device_cus() ? side : smallest({56}, 2 * device_cus());
+    int side = 0;
+    if (tile == 16 || tile == 0) side = smallest({8, 12, 16, 20, 24});
+    if (side || tile == 16) return side ? side : 16;
+    if (tile == 32 || tile == 0) side = smallest({32, 36, 40});
+    if (side || tile == 32) return side ? side : 32;
+    if ((side = smallest({48, 56, 64}))) return side;
+    return tile_count(w, h, 56) <= 2 * cus ? 56 : 64;
 }
 
 int fused_step(const StepArgs &s, float *ws, hipStream_t stream, hipEvent_t *ev, int reps) {
@@ -228,9 +232,10 @@ int fused_step(const StepArgs &s, float *ws, hipStream_t stream, hipEvent_t *ev,
     Chunk plan[64], pplan[64];  // the diffusion's and the pressure's launches
     if (s.iters > 64 * kMaxChunk)
         return set_error(PFS_ERR_UNSUPPORTED, "iters too large for one step plan");
-    if (!valid_tile_side(s.tile)) return set_error(PFS_ERR_INVALID, "tile side must be 16, 32 or 64");
-    const bool small = s.tile == 16;
+    if (s.tile != 0 && !valid_tile_side(s.tile))
+        return set_error(PFS_ERR_INVALID, "tile side must be 16, 32 or 64");
     const int side = tile_side(s.tile, s.w, s.h);
+    const bool small = side <= 24;
     DiffuseArgs d = diffuse_args(s.P, s.Q, s.w, s.h, s.dt, s.visc, s.iters, ws, side);
     PressureArgs p = pressure_args(s.P, s.Q, s.image, s.itmp, s.w, s.h, s.dt, ws, side);
     const dim3 grid(d.ntiles);
@@ -268,7 +273,7 @@ int fused_step(const StepArgs &s, float *ws, hipStream_t stream, hipEvent_t *ev,
             // Only whole chunks of fields with two workgroups for every CU:
             // below that the square tiles are as fast (2048^2: 22.5 us against
             // 24; 1024^2: equal).
-            const WaveShape sh = k.last || s.tile != 64 ? WaveShape{0, 0} : wave_args(w, k.H);
+            const WaveShape sh = k.last || side < 48 ? WaveShape{0, 0} : wave_args(w, k.H);
             if (sh.S == 4 && k.H == kMaxChunk && w.ntiles >= 2 * device_cus())
                 hipLaunchKernelGGL(k_pressure_wave, dim3(w.ntiles), dim3(64 * sh.nw), 0, stream, w);
             else
