@@ -16,13 +16,14 @@
 //   - the pressure iteration stops at the first iterate i >= 1 with
 //     ||r(p^i)|| <= tol ||b||, at most K sweeps, decided on the device.
 //
-// Kernels (temporally blocked like the plain step, pfs_step.hip, on the
-// same register-strip tiles, pfs_step_kernels.h):
+// Kernels (temporally blocked like the plain step, pfs_step.hip, in the same
+// wave tiles, pfs_wave_kernels.h, and square tiles, pfs_step_kernels.h):
 //
-//   k_diffuse_precise     advect + C diffusion sweeps per launch (compensated),
+//   k_diffuse_wave_precise, on small fields k_diffuse_precise
+//                         advect + C diffusion sweeps per launch (compensated),
 //                         the last launch also the divergence and the
-//                         pressure start (diffuse_tile<..., COMP = true>);
-//                         the first also clears the step's control block
+//                         pressure start (diffuse_wave / diffuse_tile with COMP
+//                         = true); the first also clears the step's control block
 //   k_pressure_precise    C pressure sweeps per launch from an iterate plane,
 //                         with the FP64 residual of every iterate the launch
 //                         reads on the tile's own cells; launch `launch`
