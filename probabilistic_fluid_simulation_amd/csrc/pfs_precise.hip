@@ -799,36 +799,24 @@ DiffuseFn diffuse_precise_wave(int H, bool first, bool last) {
 
 template <int H>
 PressureFn pressure_precise_h(int ts, bool half) {
-    if (ts == 64 && half) return k_pressure_precise<H, 64, 512>;
-    return ts == 16 ? k_pressure_precise<H, 16, 1024>
-                    : ts == 32 ? k_pressure_precise<H, 32, 1024> : k_pressure_precise<H, 64, 1024>;
+    switch (ts) {
+#define PFS_CASE(t) \
+    case t:         \
+        return k_pressure_precise<H, t, 1024>;
+        PFS_CASE(16) PFS_CASE(20) PFS_CASE(24) PFS_CASE(32) PFS_CASE(36) PFS_CASE(40) PFS_CASE(48)
+        PFS_CASE(56)
+#undef PFS_CASE
+    }
+    return half ? k_pressure_precise<H, 64, 512> : k_pressure_precise<H, 64, 1024>;
 }
 
 PressureFn pressure_precise_for(int C, int ts, bool half) {
     return C == 4 ? pressure_precise_h<5>(ts, half) : pressure_precise_h<9>(ts, half);
 }
 
-template <int TS>
-int threads_precise_ts(int H) {
-    switch (H) {
-#define PFS_CASE(h) \
-    case h:         \
-        return Geo<h, TS>::NT;
-        PFS_CASE(2) PFS_CASE(3) PFS_CASE(4) PFS_CASE(5) PFS_CASE(6) PFS_CASE(7) PFS_CASE(8)
-        PFS_CASE(9)
-#undef PFS_CASE
-    }
-    return 0;
-}
-
-int threads_precise(int H, int ts) {
-    return ts == 16 ? threads_precise_ts<16>(H)
-                    : ts == 32 ? threads_precise_ts<32>(H) : threads_precise_ts<64>(H);
-}
-
 int threads_pressure_precise(int C, int ts, bool half) {
     if (ts == 64 && half) return C == 4 ? Geo<5, 64, 512>::NT : Geo<9, 64, 512>::NT;
-    return threads_precise(C + 1, ts);
+    return threads_for(C + 1, ts);
 }
 
 // Sweeps per launch (4 or 8) and tile side (16, 32, 64; 0: the plain
@@ -849,6 +837,18 @@ size_t precise_ws_bytes(int w, int h) {
     const size_t planes = ((8 * N * sizeof(float)) + 255) / 256 * 256;
     return planes + kPCtlBytes + (size_t)kNRows * (size_t)tile_count(w, h, 16) * sizeof(double) +
            256;
+}
+
+// The pressure's side on a field whose side by the rule is ts: the smallest near
+// it whose tiles the CUs hold at once, else ts (the workspace's slots hold what
+// side 16 gives).  A step of 8 + 8 sweeps at 640x480, side 32 (300 tiles) 43.8 us,
+// 36: 36.4; of 16 + 16 at 800x600, 64: 96.7, 48: 85.3; 320x240, 16: 49.7, 20: 46.2.  Past
+// one tile a CU side 64's pairs of 512-thread workgroups are the faster
+// (1200x1024: 144 us against 152 at side 56).
+int pressure_side(int ts, int w, int h) {
+    for (int side : {16, 20, 24, 32, 36, 40, 48, 56})
+        if ((ts == 16) == (side < 32) && tile_count(w, h, side) <= device_cus()) return side;
+    return ts;
 }
 
 int precise_step(float *P, float *Q, int w, int h, float dt, float visc, int K, double tol,
@@ -872,7 +872,7 @@ int precise_step(float *P, float *Q, int w, int h, float dt, float visc, int K, 
         PCtl *clear = c == 0 ? ctl : nullptr;
         if (ts == 16) {
             hipLaunchKernelGGL(diffuse_precise_small(k.H, k.last), dim3(d.ntiles),
-                               dim3(threads_precise(k.H, ts)), 0, s, d, clear);
+                               dim3(threads_for(k.H, ts)), 0, s, d, clear);
         } else {
             DiffuseArgs wd = d;
             const WaveShape sh =
@@ -897,16 +897,17 @@ int precise_step(float *P, float *Q, int w, int h, float dt, float visc, int K, 
     pa.ctl = ctl;
     pa.w = w;
     pa.h = h;
-    pa.tiles_x = d.tiles_x;
-    pa.ntiles = d.ntiles;
+    const int side = forced ? forced : pressure_side(ts, w, h);
+    pa.tiles_x = (w + side - 1) / side;
+    pa.ntiles = (int)tile_count(w, h, side);
     pa.dt = dt;
     pa.K = K;
     pa.C = C;
     pa.nchunks = (K + C - 1) / C;
     pa.tol2 = tol * tol;
     const bool half = g_precise_half.load() != 0;
-    const PressureFn pf = pressure_precise_for(C, ts, half);
-    const int nt = threads_pressure_precise(C, ts, half);
+    const PressureFn pf = pressure_precise_for(C, side, half);
+    const int nt = threads_pressure_precise(C, side, half);
     for (int l = 0; l <= pa.nchunks; ++l) {  // the chunks, then the fix-up
         pa.launch = l;
         hipLaunchKernelGGL(pf, dim3(pa.ntiles), dim3(nt), 0, s, pa);

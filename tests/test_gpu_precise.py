@@ -300,3 +300,25 @@ def test_precise_sweep_counts(k):
     scale = np.abs(ref[..., :2]).max(axis=(0, 1))
     err = np.abs(a[1][..., :2] - ref[..., :2]).max(axis=(0, 1)) / scale
     assert np.all(err < 1e-5), err
+
+
+@pytest.mark.parametrize("shape", [(250, 240), (310, 300), (371, 330), (500, 401), (601, 430),
+                                   (641, 620), (761, 700), (881, 870), (1001, 980)],
+                         ids=["16", "20", "24", "32", "36", "40", "48", "56", "64"])
+def test_precise_pressure_at_every_side(shape):
+    """The automatic side of the pressure against a forced one: the same
+    outputs, and the residuals to the rounding of their FP64 partition."""
+    s = scenes.random_scene(*shape, 4, 4, seed=shape[0], dt=0.5, visc=0.2, iters=9)
+    got = []
+    for tile in (0, 16 if shape[0] > 400 else 32):
+        fluid.set_precise_schedule(0, tile, 0)
+        try:
+            vp, tmp = VPField.from_numpy(s.vp), VPField.from_numpy(s.tmp)
+            rep = fluid.simulate_fluid_step_precise(vp, tmp, s.dt, s.visc, 9, 0.0)
+        finally:
+            fluid.set_precise_schedule(0, 0, 0)
+        got.append((vp.numpy(), tmp.numpy(), rep))
+    (a, b, ra), (c, d, rb) = got
+    assert a.tobytes() == c.tobytes() and b.tobytes() == d.tobytes()
+    assert ra["iters_used"] == rb["iters_used"]
+    np.testing.assert_allclose(ra["residual_history"], rb["residual_history"], rtol=1e-12)
