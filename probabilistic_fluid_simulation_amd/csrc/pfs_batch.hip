@@ -7,13 +7,15 @@
 // simulate_fluid_step + advect_color_step — with one launch per kernel
 // stage for all scenes together:
 //
-//   k_diffuse_batch   every tile of every scene (scenes grouped by K)
+//   k_diffuse_wave_batch (small batches: k_diffuse_batch)
+//                     every tile of every scene (scenes grouped by K)
 //   k_pressure_batch  every tile of every scene, dye fused where the dye has
 //                     the field's size
 //   k_color_batch     the dye of the remaining scenes
 //
 // Each workgroup finds its scene through a tile -> scene table and runs the
-// same per-tile body as the single-scene kernels (pfs_step_kernels.h), so
+// same per-tile body as the single-scene kernels (pfs_wave_kernels.h,
+// pfs_step_kernels.h), so
 // every scene's result is bit-identical to stepping it alone.  The launch
 // sequences of 8 and of 2 consecutive steps (the dye buffers swap every step)
 // are captured once in hipGraphs and replayed while membership is unchanged;

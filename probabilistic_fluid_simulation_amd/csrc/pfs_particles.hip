@@ -11,9 +11,9 @@
 //                            (key, particle) pairs, 8- or 10-bit digits: per-block
 //                            LDS histograms, a DPP prefix scan, and a scatter
 //                            whose in-block ranks come from wavefront ballots;
-//                            cell start/end tables (the scan of the cell
-//                            counts: every cell, empty or not, gets its
-//                            lower bound); positions in sorted order;
+//                            cell start/end tables (every cell, empty or
+//                            not, gets its lower bound, found by searches of
+//                            the sorted keys); positions in sorted order;
 //   pfs_ngrid_neighbors      neighbour counts, their exclusive scan, and the
 //                            lists (CSR) of every particle within radius r,
 //                            visiting the 3x3 cells in a fixed order;
@@ -38,9 +38,9 @@
 namespace pfs {
 namespace {
 
-constexpr int kThreads = 1024;              // sort, scan and grid kernels
-constexpr int kItems = 4;                   // keys per thread
-constexpr int kTile = kThreads * kItems;    // keys per block
+constexpr int kThreads = 1024;              // scan kernels, and the sort's large tiles
+constexpr int kItems = 4;                   // values or keys per thread
+constexpr int kTile = kThreads * kItems;    // values per block
 constexpr int kWaves = kThreads / 64;
 constexpr int kMaxRadixBits = 10;           // digits of 8 or 10 bits
 

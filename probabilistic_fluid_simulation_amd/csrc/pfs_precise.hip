@@ -824,7 +824,7 @@ int threads_pressure_precise(int C, int ts, bool half) {
 std::atomic<int> g_precise_chunk{8};
 std::atomic<int> g_precise_tile{0};
 // 1: 512-thread pressure workgroups at tile side 64 (two per CU: one's
-// loads and barriers overlap the other's sweeps; 0.37 against 0.42 ms per
+// loads and barriers overlap the other's sweeps; 0.30 against 0.33 ms per
 // 2048^2 step with 1024).
 std::atomic<int> g_precise_half{1};
 

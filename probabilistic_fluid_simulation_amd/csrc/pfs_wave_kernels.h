@@ -20,10 +20,11 @@
 // sweep: one product (alpha), the four additions of the reference, the
 // division in two operations, half a min3 for its range test.
 // Measured (1024^2 / 2048^2 at 8 sweeps, 3840x2160 at 30, all launches of the
-// diffusion): square tiles 25.9 / 96.9 / 511 us; this form 20.2 / 54 / 261 us.
-// Of that, the ring of one cell around the staged velocities (without it the
-// region's outermost cells trace out of it in every wave and gather from
-// memory) took 23.9 / 63.9 / 285 to 21.1 / 54.2 / 261 at 12 waves of 4 rows.
+// diffusion): square tiles 25.9 / 96.9 / 511 us; this form 18.6 / 51 / 241 us.
+// Of that, before the back-trace lost its wraps (near_trace), the ring of one
+// cell around the staged velocities (without it the region's outermost cells
+// trace out of it in every wave and gather from memory) took 23.9 / 63.9 / 285 to
+// 21.1 / 54.2 / 261 at 12 waves of 4 rows.
 #pragma once
 
 #include <type_traits>
