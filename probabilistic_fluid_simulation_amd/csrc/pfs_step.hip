@@ -209,8 +209,8 @@ size_t fused_workspace_bytes(int w, int h) {
 // up to half the launch again.  Diffusion + pressure at 8 sweeps, us, by side:
 // 128^2 8: 8.7, 12: 9.3, 16: 10.2; 320x240 16 (300 tiles): 13.8, 20: 11.5, 24:
 // 12.4; 360^2 24: 13.1, 32: 15.2.  The pressure alone: 611x397 32 (260 tiles) 12.8,
-// 36: 8.7; 800x600 48: 12.2, 56: 13.6, 64: 15.2; 1200x1024, more than a tile a CU
-// at 64 (30.0), 56: 22.1.
+// 36: 8.7; 800x600 48: 12.2, 56: 13.6, 64: 15.2; past a tile a CU at 64, two at 48
+// or 56: 1100x1024 48: 19.2, 56: 21.4, 64: 24.5, 1200x1024 56: 21.8, 64: 25.0.
 int tile_side(int tile, int w, int h) {
     const int cus = device_cus();
     auto smallest = [&](std::initializer_list<int> sides) {
@@ -224,7 +224,9 @@ int tile_side(int tile, int w, int h) {
     if (tile == 32 || tile == 0) side = smallest({32, 36, 40});
     if (side || tile == 32) return side ? side : 32;
     if ((side = smallest({48, 56, 64}))) return side;
-    return tile_count(w, h, 56) <= 2 * cus ? 56 : 64;
+    for (int two : {48, 56})  // two workgroups a CU
+        if (tile_count(w, h, two) <= 2 * cus) return two;
+    return 64;
 }
 
 int fused_step(const StepArgs &s, float *ws, hipStream_t stream, hipEvent_t *ev, int reps) {

@@ -352,8 +352,8 @@ def test_launches_of_ten_sweeps(orc, shape, k):
 @pytest.mark.parametrize("k", [1, 8, 10, 13])
 @pytest.mark.parametrize("shape", [(101, 83), (181, 150), (251, 240), (311, 300), (371, 330),
                                    (500, 401), (601, 430), (641, 620), (761, 700), (881, 870),
-                                   (1001, 980), (1201, 1023)],
-                         ids=["8", "12", "16", "20", "24", "32", "36", "40", "48", "56", "64", "56-large"])
+                                   (1001, 980), (1101, 1023), (1201, 1023), (1501, 1100)],
+                         ids=["8", "12", "16", "20", "24", "32", "36", "40", "48", "56", "64", "48-pairs", "56-pairs", "64-pairs"])
 def test_every_side_of_the_square_tiles(orc, shape, k):
     """The automatic choice from 8 to 64 cells a side, partial tiles on both
     edges, one launch and several, the dye within the last."""
