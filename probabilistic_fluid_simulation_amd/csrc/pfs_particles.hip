@@ -260,9 +260,13 @@ __global__ __launch_bounds__(NT) void k_radix_scatter(
     const float *__restrict__ y, float *__restrict__ xs, float *__restrict__ ys) {
     constexpr int R = 1 << RB, NW = NT / 64, TILE = sort_tile<NT>();
     constexpr int DPT = R > NT ? R / NT : 1;  // digits per thread, consecutive
-    __shared__ uint32_t wcount[NW][R];
+    // The tile in digit order lies over the waves' counts, which it replaces: two
+    // large tiles then share a CU.
+    constexpr int WORDS = NW * R > 2 * TILE ? NW * R : 2 * TILE;
+    __shared__ uint32_t words[WORDS];
+    uint32_t(*wcount)[R] = reinterpret_cast<uint32_t(*)[R]>(words);
+    uint32_t *lkey = words, *lval = words + TILE;
     __shared__ uint32_t gofs[R], loff[R];
-    __shared__ uint32_t lkey[TILE], lval[TILE];
     __shared__ uint32_t sh[NW + 1];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int tb = xcd_block(blockIdx.x, nb);  // the tile of this workgroup
@@ -277,7 +281,7 @@ __global__ __launch_bounds__(NT) void k_radix_scatter(
         key[r] = valid ? kin[i] : 0u;
         val[r] = valid ? (vin ? vin[i] : (uint32_t)i) : 0u;
     }
-    for (int e = threadIdx.x; e < NW * R; e += NT) (&wcount[0][0])[e] = 0;
+    for (int e = threadIdx.x; e < NW * R; e += NT) words[e] = 0;
     {
         uint32_t t[DPT], before[DPT], s = 0;
 #pragma unroll
@@ -360,14 +364,16 @@ __global__ __launch_bounds__(NT) void k_radix_scatter(
         __syncthreads();
     }
 #pragma unroll
-    for (int r = 0; r < kItems; ++r) {
-        if (base + (size_t)r * 64 >= (size_t)n) continue;
-        const uint32_t li = loff[dig[r]] + wcount[wave][dig[r]] + local[r];
-        if (li < (uint32_t)TILE) {  // always: kept as a bound
-            lkey[li] = key[r];
-            lval[li] = val[r];
+    for (int r = 0; r < kItems; ++r)
+        local[r] = base + (size_t)r * 64 < (size_t)n ? loff[dig[r]] + wcount[wave][dig[r]] + local[r]
+                                                     : (uint32_t)TILE;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kItems; ++r)
+        if (local[r] < (uint32_t)TILE) {
+            lkey[local[r]] = key[r];
+            lval[local[r]] = val[r];
         }
-    }
     __syncthreads();
     const int count = (int)min((size_t)TILE, (size_t)n - (size_t)tb * TILE);
     for (int j = threadIdx.x; j < count; j += NT) {
