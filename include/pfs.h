@@ -392,7 +392,8 @@ int pfs_pbf_solve(const pfs_ngrid *g, float *xs, float *ys, const uint32_t *cell
 /* out[p] = in[index[p]]: permutes per-particle data into sorted order. */
 int pfs_gather_u32(const uint32_t *index, const uint32_t *in, uint32_t *out, int n, void *stream);
 /* Exclusive prefix sum of n uint32 (wavefront DPP scans); *total (device,
- * may be NULL) gets the sum.  Workspace: (ceil(n / 4096) + 1) * 4 bytes. */
+ * may be NULL) gets the sum.  out may be in.
+ * Workspace: (ceil(n / 4096) + 1) * 4 bytes. */
 int pfs_scan_exclusive_u32(const uint32_t *in, uint32_t *out, int n, uint32_t *total,
                            void *workspace, size_t workspace_bytes, void *stream);
 

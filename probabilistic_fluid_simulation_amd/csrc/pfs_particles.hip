@@ -96,9 +96,9 @@ __global__ __launch_bounds__(kThreads) void k_scan_reduce(const uint32_t *__rest
 
 // Block b adds up the totals of blocks [0, b) itself (a few hundred at
 // most), then scans its tile; the last block also writes the grand total.  sums
-// null (few blocks): it adds up their values instead.
-__global__ __launch_bounds__(kThreads) void k_scan_down(const uint32_t *__restrict__ in,
-                                                        uint32_t *__restrict__ out, int n,
+// null (few blocks): it adds up their values instead, which out then may not
+// overlap.
+__global__ __launch_bounds__(kThreads) void k_scan_down(const uint32_t *in, uint32_t *out, int n,
                                                         const uint32_t *__restrict__ sums,
                                                         uint32_t *__restrict__ grand) {
     __shared__ uint32_t sh[kWaves + 1];
@@ -138,14 +138,19 @@ constexpr int kOneScan = 8;
 
 // Exclusive scan of n values in two kernels (block totals, then blocks
 // scanned from the totals before them), or one for few blocks; grand (device, may be null) gets the
-// total.  ws: nblocks_for(n) words.
+// total.  ws: nblocks_for(n) words.  out may be in: the totals then come from a
+// launch of their own at any count, since blocks that read what precedes their
+// tile would meet what others have written there.
 int scan_exclusive(const uint32_t *in, uint32_t *out, int n, uint32_t *grand, uint32_t *ws,
                    hipStream_t s) {
     const int nb = nblocks_for((size_t)n);
     if (nb == 0) return PFS_OK;
-    if (nb > kOneScan) hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(kThreads), 0, s, in, n, ws);
+    const uintptr_t i0 = (uintptr_t)in, o0 = (uintptr_t)out, bytes = (uintptr_t)n * sizeof *in;
+    const bool apart = i0 + bytes <= o0 || o0 + bytes <= i0;
+    const bool totals = nb > kOneScan || (nb > 1 && !apart);
+    if (totals) hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(kThreads), 0, s, in, n, ws);
     hipLaunchKernelGGL(k_scan_down, dim3(nb), dim3(kThreads), 0, s, in, out, n,
-                       nb > kOneScan ? ws : nullptr, grand);
+                       totals ? ws : nullptr, grand);
     return check_launch("exclusive scan");
 }
 

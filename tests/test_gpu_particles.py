@@ -35,6 +35,22 @@ def test_scan_in_one_and_two_launches(n):
     test_scan_exclusive(n)
 
 
+@pytest.mark.parametrize("n", [4096, 4097, 8192, 4096 * 8, 4096 * 8 + 1])
+def test_scan_in_place(n):
+    """out == in: one block, blocks that may not read what others write, and
+    the count past which totals have a launch of their own anyway."""
+    from probabilistic_fluid_simulation_amd import _lib
+
+    a = np.random.default_rng(n).integers(0, 50, size=n).astype(np.int32)
+    t = torch.from_numpy(a).cuda()
+    total = torch.zeros(1, dtype=torch.int32, device="cuda")
+    ws = torch.empty((n + 4095) // 4096 + 1, dtype=torch.int32, device="cuda")
+    _lib.call("pfs_scan_exclusive_u32", t.data_ptr(), t.data_ptr(), n, total.data_ptr(),
+              ws.data_ptr(), ws.numel() * 4, torch.cuda.current_stream().cuda_stream)
+    np.testing.assert_array_equal(t.cpu().numpy(), np.cumsum(a) - a)
+    assert int(total.item()) == int(a.sum())
+
+
 def _positions(n, W, H, seed):
     rng = np.random.default_rng(seed)
     x = np.minimum((rng.random(n) * W).astype(np.float32), np.nextafter(np.float32(W), np.float32(0)))
