@@ -852,7 +852,7 @@ __global__ void k_tracer_advect(float *__restrict__ x, float *__restrict__ y, in
 // -30/(pi h^5) (h - r)^2 d / r for 0 < r < h (zero outside).  All updates
 // of an iteration read the same iterate (Jacobi); positions wrap.
 struct PbfCtl {
-    int done, final_it;  // converged flag; the iterate the solve ends on
+    int done;  // 0, or 1 + the iterate the solve converged on
 };
 
 struct PbfArgs {
@@ -1092,10 +1092,7 @@ __device__ __forceinline__ double fold_sums(const PbfArgs &b) {
 // Writes iterate b.it's total and, at convergence, the verdict.
 __device__ __forceinline__ void record(const PbfArgs &b, double total) {
     b.res[b.it] = total;
-    if (total <= b.tol2n) {
-        b.ctl->done = 1;
-        b.ctl->final_it = b.it;
-    }
+    if (total <= b.tol2n) b.ctl->done = 1 + b.it;
 }
 
 // lambda of iterate b.it, and the block sums of C^2.  Short
@@ -1157,15 +1154,20 @@ __global__ __launch_bounds__(kPbfParticles *QUAD) void k_pbf_delta(PbfArgs b) {
     const int p = pbf_particle<QUAD>();
     const PbfOwn own = load_own(b, p);
     const float lp = b.lambda[min(p, b.n - 1)];
-    if (b.ctl->done) return;
+    const int done = b.ctl->done;
     Staged *st = nullptr;
     if constexpr (QUAD == 1) {
+        if (done) return;  // as k_pbf_check left it
         __shared__ Staged shared;
         st = &shared;
         stage_windows<true>(b, *st);
     } else {
         // Every workgroup folds the block sums for itself, a load or two a
-        // thread, and comes to the same verdict.
+        // thread, and comes to the same verdict; the first one records it.  A
+        // thread that already reads this iterate's record goes on like those that
+        // read none, so that a workgroup meets the fold's barriers as a whole:
+        // only an earlier iterate's ends it here.
+        if (done != 0 && done <= b.it) return;
         __shared__ int over;
         const double total = fold_sums(b);
         if (threadIdx.x == 0) {
@@ -1199,7 +1201,7 @@ __global__ __launch_bounds__(kPbfParticles *QUAD) void k_pbf_delta(PbfArgs b) {
 // scratch pair when f is odd.
 __global__ void k_pbf_finish(const PbfCtl *ctl, int iters, const float *sx, const float *sy,
                              float *xs, float *ys, int *iters_used, int n) {
-    const int f = ctl->done ? ctl->final_it : iters;
+    const int f = ctl->done ? ctl->done - 1 : iters;
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p == 0 && iters_used) *iters_used = f;
     if (p < n && (f & 1)) {
@@ -1209,10 +1211,7 @@ __global__ void k_pbf_finish(const PbfCtl *ctl, int iters, const float *sx, cons
 }
 
 __global__ void k_pbf_init(PbfCtl *ctl, double *res, int nres) {
-    if (threadIdx.x == 0) {
-        ctl->done = 0;
-        ctl->final_it = 0;
-    }
+    if (threadIdx.x == 0) ctl->done = 0;
     for (int k = threadIdx.x; k < nres; k += blockDim.x) res[k] = -1.0;  // not computed
 }
 

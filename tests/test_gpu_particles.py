@@ -269,6 +269,27 @@ def test_pbf_matches_oracle(iters, stop):
     np.testing.assert_allclose(r[done], ores[done], rtol=1e-12)
 
 
+@pytest.mark.parametrize("stop", [1, 2])
+@pytest.mark.parametrize("n", [200001, 3 << 17], ids=["four-lanes", "one-lane"])
+def test_pbf_converges_in_the_middle_of_a_launch(n, stop):
+    """An iterate found converged while workgroups of the launch that records it
+    are still to start (782 workgroups of 1024 threads, where 512 run at once),
+    at an odd and an even iterate: the buffers and the residuals are those of
+    a solve of that many iterations, and nothing follows it."""
+    ng, og, rho0 = _pbf_setup(n, 1000.0, 1.5, 19, 130.0)
+    _, _, _, res_all, _ = og.pbf(1.0, rho0, 5.0, 3)
+    tol = float(np.sqrt((res_all[stop - 1] + res_all[stop]) / 2 / og.n))
+    ox, oy, olam, ores, oused = og.pbf(1.0, rho0, 5.0, 4, tol)
+    lam, res, used = ng.pbf(1.0, rho0, 5.0, 4, tol)
+    assert int(used.item()) == oused == stop
+    assert ng.xs.cpu().numpy().tobytes() == ox.tobytes()
+    assert ng.ys.cpu().numpy().tobytes() == oy.tobytes()
+    assert lam.cpu().numpy().tobytes() == olam.tobytes()
+    r = res.cpu().numpy()
+    np.testing.assert_allclose(r[:stop + 1], ores[:stop + 1], rtol=1e-12)
+    assert (r[stop + 1:] == -1).all()
+
+
 @pytest.mark.parametrize("n", [(3 << 17) - 1, 3 << 17])
 def test_pbf_either_side_of_the_lane_rule(n):
     ng, og, rho0 = _pbf_setup(n, 1000.0, 1.5, 13, 130.0)
