@@ -23,6 +23,11 @@ def _ptr(t: torch.Tensor) -> int:
     return t.data_ptr()
 
 
+def _wait(stream) -> None:
+    """Until the work queued on `stream` (None: the current one) is done."""
+    (stream if stream is not None else torch.cuda.current_stream()).synchronize()
+
+
 def _check_xy(x: torch.Tensor, y: torch.Tensor) -> None:
     if x.dtype != torch.float32 or y.dtype != torch.float32 or x.shape != y.shape or x.dim() != 1:
         raise ValueError("x, y must be 1-D float32 tensors of one length")
@@ -46,8 +51,11 @@ def scan_exclusive(t: torch.Tensor, stream=None) -> Tuple[torch.Tensor, int]:
     out = torch.empty_like(t)
     total = torch.zeros(1, dtype=torch.int32, device=t.device)
     ws = torch.empty(((n + 4095) // 4096 + 1,), dtype=torch.int32, device=t.device)
+    if stream is not None:  # total's zero was queued on the current stream
+        stream.wait_stream(torch.cuda.current_stream())
     _lib.call("pfs_scan_exclusive_u32", _ptr(t), _ptr(out), n, _ptr(total), _ptr(ws),
               ws.numel() * 4, _stream(stream))
+    _wait(stream)
     return out, int(total.item()) & 0xFFFFFFFF
 
 
@@ -131,6 +139,7 @@ class NeighborGrid:
                     raise
         else:
             self.neighbor_counts(stream, xs, ys, by_position)
+        _wait(stream)
         total = int(self.total.item()) & 0xFFFFFFFF
         self.nbr = torch.empty(max(total + total // 4, 1), dtype=torch.int32,
                                device=self.keys.device)

@@ -394,6 +394,26 @@ def test_lists_from_density_counts(order):
     assert ng.nbr.numel() >= len(on)
 
 
+def test_sizes_of_work_on_another_stream():
+    """A scan's total and the first lists' size are read after the stream they
+    are made on, here busy for milliseconds, and not after the current one."""
+    st = torch.cuda.Stream()
+    m = torch.rand(8192, 8192, device="cuda")
+    a = torch.ones(100000, dtype=torch.int32, device="cuda")
+    x, y = (torch.from_numpy(p).cuda() for p in _positions(20000, 100.0, 100.0, seed=41))
+    ng = particles.NeighborGrid(20000, 100.0, 100.0, 1.5)
+    ng.build(x, y)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(st):
+        m @ m
+    assert particles.scan_exclusive(a, stream=st)[1] == 100000
+    with torch.cuda.stream(st):
+        m @ m
+    counts, _, nbr = ng.neighbors(stream=st)
+    torch.cuda.synchronize()
+    assert nbr.numel() == int(counts.sum().item()) > 0
+
+
 @pytest.mark.parametrize("spread", [2.5, 4.0], ids=["dense", "sparse"])
 def test_lists_by_position_bitexact(spread):
     """Lists by sorted position (written through LDS windows): a dense blob
