@@ -116,11 +116,19 @@ class NeighborGrid:
         """(counts, offsets, lists): particle i's neighbours are
         lists[offsets[i] : offsets[i] + counts[i]].  All three are the grid's
         own buffers, overwritten by its next count or list call.  Waits for the
-        counts to size the lists (the lists themselves are queued): one counting pass when the list buffer
-        kept from an earlier call holds them, else a sizing pass first (the
-        buffer then grows with 25% headroom).  counted=True: the grid's counts
-        already hold those of these positions (density(..., with_counts=True)
-        just ran on them), so no counting pass runs (pfs_ngrid_lists)."""
+        stream, so that any stream and the host may read them: one counting
+        pass when the list buffer kept from an earlier call holds them, else a
+        sizing pass first (the buffer then grows with 25% headroom).
+        counted=True: the grid's counts already hold those of these positions
+        (density(..., with_counts=True) just ran on them), so no counting pass
+        runs (pfs_ngrid_lists)."""
+        out = self._lists(stream, xs, ys, by_position, counted)
+        _wait(stream)
+        return out
+
+    def _lists(self, stream, xs, ys, by_position, counted=False):
+        """neighbors() with the lists queued on the stream: it waits for their
+        size only."""
         fn = "pfs_ngrid_lists" if counted else "pfs_ngrid_neighbors"
 
         def lists():
@@ -176,7 +184,7 @@ class NeighborGrid:
         # lists: (counts, offsets, nbr) of these positions by sorted position,
         # from neighbors(by_position=True), when the caller already has them.
         counts, offsets, nbr = (lists if lists is not None
-                                else self.neighbors(stream, xs, ys, by_position=True))
+                                else self._lists(stream, xs, ys, by_position=True))
         if nbr.numel() == 0:  # no neighbours at all: the C ABI still wants a buffer
             nbr = torch.zeros(1, dtype=torch.int32, device=xs.device)
         if getattr(self, "_pbf_ws", None) is None or self._pbf_ws.numel() < nbytes + 256:

@@ -414,6 +414,25 @@ def test_sizes_of_work_on_another_stream():
     assert nbr.numel() == int(counts.sum().item()) > 0
 
 
+@pytest.mark.parametrize("own_stream", [False, True], ids=["current-stream", "own-stream"])
+@pytest.mark.parametrize("counted", [False, True], ids=["counting", "counted"])
+def test_neighbors_returns_finished_lists(own_stream, counted):
+    """Nothing is left queued when neighbors() returns, so that another stream
+    reads whole lists: 1M particles of 37 neighbours, whose lists take far longer
+    than the return."""
+    n, W = 1 << 20, 512.0
+    x, y = (torch.rand(n, device="cuda", generator=torch.Generator("cuda").manual_seed(s)) * 511.0
+            for s in (31, 32))
+    torch.cuda.synchronize()
+    st = torch.cuda.Stream() if own_stream else torch.cuda.current_stream()
+    ng = particles.NeighborGrid(n, W, W, 1.7)
+    ng.build(x, y, st)
+    for _ in range(3):
+        ng.density(1.0, st, with_counts=True)
+        ng.neighbors(st if own_stream else None, counted=counted)
+        assert st.query()
+
+
 @pytest.mark.parametrize("spread", [2.5, 4.0], ids=["dense", "sparse"])
 def test_lists_by_position_bitexact(spread):
     """Lists by sorted position (written through LDS windows): a dense blob
