@@ -224,14 +224,15 @@ int pfs_advect_color(const pfs_field *image, pfs_field *out, const pfs_field *vp
                                vp->x, vp->y, vp->z, dt, (hipStream_t)stream);
 }
 
-int pfs_diffuse(pfs_field *vp, pfs_field *vp_out, float viscosity, float dt, int iters,
-                void *stream) {
+// pfs_diffuse; no_alloc: a launch per sweep, which needs no workspace.
+static int diffuse(pfs_field *vp, pfs_field *vp_out, float viscosity, float dt, int iters,
+                   void *stream, bool no_alloc) {
     PFS_TRY(check_field(vp, "vp", 2));
     PFS_TRY(check_field(vp_out, "vp_out", 2));
     if (!same_shape(vp, vp_out)) return set_error(PFS_ERR_INVALID, "vp_out shape != vp shape");
     if (vp->data == vp_out->data) return set_error(PFS_ERR_INVALID, "vp and vp_out alias");
     if (iters < 0) return set_error(PFS_ERR_INVALID, "iters < 0");
-    if (Lease ws; op_workspace(vp, vp_out, iters, (hipStream_t)stream, &ws)) {
+    if (Lease ws; !no_alloc && op_workspace(vp, vp_out, iters, (hipStream_t)stream, &ws)) {
         // K - 1 swaps (src/fluid.cpp:188-194) leave the structs exchanged for
         // even K; the last sweep writes what is then vp_out.
         if (iters % 2 == 0) std::swap(vp->data, vp_out->data);
@@ -246,6 +247,11 @@ int pfs_diffuse(pfs_field *vp, pfs_field *vp_out, float viscosity, float dt, int
         if (it != iters - 1) std::swap(vp->data, vp_out->data);  // src/fluid.cpp:188-194
     }
     return PFS_OK;
+}
+
+int pfs_diffuse(pfs_field *vp, pfs_field *vp_out, float viscosity, float dt, int iters,
+                void *stream) {
+    return diffuse(vp, vp_out, viscosity, dt, iters, stream, false);
 }
 
 int pfs_add_forces(pfs_field *vp, const float *forces, void *stream) {
@@ -263,14 +269,15 @@ int pfs_add_forces_apply(pfs_field *vp, const float *forces, int fz, float dt, v
     return launch_add_forces(vp->data, forces, vp->x, vp->y, vp->z, fz, dt, (hipStream_t)stream);
 }
 
-int pfs_compute_pressure(pfs_field *vp, pfs_field *vp_out, float dt, int iters, void *stream) {
+static int compute_pressure(pfs_field *vp, pfs_field *vp_out, float dt, int iters, void *stream,
+                            bool no_alloc) {  // as diffuse
     PFS_TRY(check_field(vp, "vp", 4));
     PFS_TRY(check_field(vp_out, "vp_out", 4));
     if (!same_shape(vp, vp_out)) return set_error(PFS_ERR_INVALID, "vp_out shape != vp shape");
     if (vp->data == vp_out->data) return set_error(PFS_ERR_INVALID, "vp and vp_out alias");
     if (iters < 0) return set_error(PFS_ERR_INVALID, "iters < 0");
     hipStream_t s = (hipStream_t)stream;
-    if (Lease ws; op_workspace(vp, vp_out, iters, s, &ws)) {
+    if (Lease ws; !no_alloc && op_workspace(vp, vp_out, iters, s, &ws)) {
         if (iters % 2 == 0) std::swap(vp->data, vp_out->data);  // as in pfs_diffuse
         return pressure_op(iters % 2 == 0 ? vp_out->data : vp->data, vp_out->data, vp->data, vp->x,
                            vp->y, dt, iters, ws.ptr, s);
@@ -281,6 +288,10 @@ int pfs_compute_pressure(pfs_field *vp, pfs_field *vp_out, float dt, int iters, 
         if (it != iters - 1) std::swap(vp->data, vp_out->data);  // src/fluid.cpp:260-265
     }
     return PFS_OK;
+}
+
+int pfs_compute_pressure(pfs_field *vp, pfs_field *vp_out, float dt, int iters, void *stream) {
+    return compute_pressure(vp, vp_out, dt, iters, stream, false);
 }
 
 int pfs_subtract_pressure_gradient(const pfs_field *vp, pfs_field *vp_out, float dt,
@@ -295,11 +306,11 @@ int pfs_subtract_pressure_gradient(const pfs_field *vp, pfs_field *vp_out, float
 }
 
 static int step_per_op(pfs_field *vp, pfs_field *tmp, float dt, float viscosity, int iters,
-                       void *stream) {
+                       void *stream, bool no_alloc) {
     // src/fluid.cpp:298-310, struct swaps included.
     PFS_TRY(pfs_advect(vp, tmp, dt, stream));
-    PFS_TRY(pfs_diffuse(tmp, vp, viscosity, dt, iters, stream));
-    PFS_TRY(pfs_compute_pressure(vp, tmp, dt, iters, stream));
+    PFS_TRY(diffuse(tmp, vp, viscosity, dt, iters, stream, no_alloc));
+    PFS_TRY(compute_pressure(vp, tmp, dt, iters, stream, no_alloc));
     return pfs_subtract_pressure_gradient(tmp, vp, dt, stream);
 }
 
@@ -346,7 +357,7 @@ static int timestep(pfs_field *vp, pfs_field *tmp, pfs_field *image, pfs_field *
     }
     if (!fused_ok(vp, tmp, iters)) {
         if (ev) return set_error(PFS_ERR_UNSUPPORTED, "profiling needs the fused path");
-        PFS_TRY(step_per_op(vp, tmp, dt, viscosity, iters, stream));
+        PFS_TRY(step_per_op(vp, tmp, dt, viscosity, iters, stream, ws_given != nullptr));
         return image ? pfs_advect_color_step(image, itmp, vp, dt, stream) : PFS_OK;
     }
     // The dye rides in the pressure kernel when pixel (i, j) samples cell

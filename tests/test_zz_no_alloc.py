@@ -63,3 +63,19 @@ def test_noalloc_timestep_rejects_fields_past_the_array():
     assert [f.numpy().tobytes() for f in bufs] == before
     small = scenes.random_scene(64, 48, 64, 48, seed=64, dt=0.5, visc=0.1, iters=4)
     _assert_same(*_both(small, 2), "after a rejection")
+
+
+def test_noalloc_timestep_allocates_nothing_past_the_fused_plan():
+    """513 sweeps take the per-operator sequence: on a stream that holds no
+    workspace yet, no block the size of one appears."""
+    small = scenes.random_scene(40, 30, 40, 30, seed=65, dt=0.6, visc=0.2, iters=513)
+    _assert_same(*_both(small, 2), "K=513")
+    s = scenes.make_scene(1500, 1000, 8, 8, kind="tg", seed=0, iters=513)
+    bufs, warm, st = _dev(s), _dev(small), torch.cuda.Stream()
+    for _ in range(3):  # the stream's own memory: queue, launch arguments
+        fluid.fluid_timestep_noalloc(*warm, small.dt, small.visc, small.iters, stream=st)
+        torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    fluid.fluid_timestep_noalloc(*bufs, s.dt, s.visc, s.iters, stream=st)
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] < 16 << 20  # a workspace is 16 or 32 B a cell
