@@ -32,7 +32,7 @@ struct Workspace {
     float *ptr = nullptr;
     size_t bytes = 0;
 };
-std::mutex g_ws_mutex;  // of the map
+std::mutex g_ws_mutex;  // of the maps
 std::map<std::pair<int, hipStream_t>, Workspace> g_ws;
 
 // A stream's workspace, held while the launches that use it are queued: two
@@ -43,41 +43,99 @@ struct Lease {
     float *ptr = nullptr;
 };
 
+// Makes w, held, at least `bytes` large.
+int grow(Workspace &w, size_t bytes, hipStream_t s) {
+    if (w.bytes >= bytes) return PFS_OK;
+    if (w.ptr) {
+        // Work already queued on this stream may still use the old block.
+        PFS_HIP_TRY(hipStreamSynchronize(s));
+        PFS_HIP_TRY(hipFree(w.ptr));
+        w.ptr = nullptr;
+        w.bytes = 0;
+    }
+    void *p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return set_error(PFS_ERR_NOMEM, "workspace allocation of " + std::to_string(bytes) +
+                                            " bytes failed");
+    }
+    w.ptr = static_cast<float *>(p);
+    w.bytes = bytes;
+    return PFS_OK;
+}
+
+// The operators' workspaces, by (device, stream).  Apart from the step's, whose
+// addresses a caller's captured steps may hold: an operator on a larger field
+// does not move those.  An operator that finds no room runs without, so that
+// all of a device's together stay within kOpBytes, and a step that finds no
+// memory has them back.
+constexpr size_t kOpBytes = (size_t)256 << 20;
+std::map<std::pair<int, hipStream_t>, Workspace> g_op_ws;
+std::map<int, size_t> g_op_held;  // bytes by device; both under g_ws_mutex
+
+Workspace &find(std::map<std::pair<int, hipStream_t>, Workspace> &all, int dev, hipStream_t s) {
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    return all[{dev, s}];  // entries stay where they are
+}
+
+// Frees the device's operator workspaces that no thread is using; hipFree waits
+// for the work queued on them.
+void free_op_workspaces(int dev) {
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    for (auto &e : g_op_ws) {
+        Workspace &w = e.second;
+        std::unique_lock<std::mutex> held(w.m, std::try_to_lock);
+        if (e.first.first != dev || !held || !w.ptr) continue;
+        if (hipFree(w.ptr) != hipSuccess) {
+            (void)hipGetLastError();
+            continue;
+        }
+        g_op_held[dev] -= w.bytes;
+        w.ptr = nullptr;
+        w.bytes = 0;
+    }
+}
+
 int get_workspace(size_t bytes, hipStream_t s, Lease *out) {
     int dev = 0;
     PFS_HIP_TRY(hipGetDevice(&dev));
-    Workspace *entry;
-    {
-        std::lock_guard<std::mutex> lock(g_ws_mutex);
-        entry = &g_ws[{dev, s}];  // entries stay where they are
+    Workspace &w = find(g_ws, dev, s);
+    out->held = std::unique_lock<std::mutex>(w.m);
+    int rc = grow(w, bytes, s);
+    if (rc == PFS_ERR_NOMEM) {
+        free_op_workspaces(dev);
+        clear_error();
+        rc = grow(w, bytes, s);
     }
-    std::unique_lock<std::mutex> held(entry->m);
-    Workspace &w = *entry;
+    out->ptr = w.ptr;
+    return rc;
+}
+
+bool get_op_workspace(size_t bytes, hipStream_t s, Lease *out) {
+    int dev = 0;
+    if (bytes > kOpBytes || hipGetDevice(&dev) != hipSuccess) return false;
+    Workspace &w = find(g_op_ws, dev, s);
+    std::unique_lock<std::mutex> held(w.m);
     if (w.bytes < bytes) {
-        if (w.ptr) {
-            // Work already queued on this stream may still use the old block.
-            PFS_HIP_TRY(hipStreamSynchronize(s));
-            PFS_HIP_TRY(hipFree(w.ptr));
-            w.ptr = nullptr;
-            w.bytes = 0;
+        std::lock_guard<std::mutex> lock(g_ws_mutex);
+        size_t &total = g_op_held[dev];
+        if (total - w.bytes + bytes > kOpBytes) return false;
+        total -= w.bytes;
+        const int rc = grow(w, bytes, s);
+        total += w.bytes;
+        if (rc != PFS_OK) {
+            clear_error();
+            return false;
         }
-        void *p = nullptr;
-        if (hipMalloc(&p, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            return set_error(PFS_ERR_NOMEM, "workspace allocation of " + std::to_string(bytes) +
-                                                " bytes failed");
-        }
-        w.ptr = static_cast<float *>(p);
-        w.bytes = bytes;
     }
     out->held = std::move(held);
     out->ptr = w.ptr;
-    return PFS_OK;
+    return true;
 }
 
 // The workspace of an operator's fused sweeps; false where the one-launch-
 // per-sweep form is to run instead: a stream that is being captured (that form
-// allocates nothing and leaves no address in the graph), no memory, or the
+// allocates nothing and leaves no address in the graph), no room, or the
 // per-operator path asked for.  The allocation is made with the thread's
 // capture checks relaxed: a capture on another stream goes on undisturbed.
 bool op_workspace(const pfs_field *a, const pfs_field *b, int iters, hipStream_t s, Lease *out) {
@@ -92,8 +150,7 @@ bool op_workspace(const pfs_field *a, const pfs_field *b, int iters, hipStream_t
     if (st != hipStreamCaptureStatusNone) return false;
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     (void)hipThreadExchangeStreamCaptureMode(&mode);
-    const bool ok = get_workspace(fused_workspace_bytes(a->x, a->y), s, out) == PFS_OK;
-    if (!ok) clear_error();
+    const bool ok = get_op_workspace(op_workspace_bytes(a->x, a->y), s, out);
     (void)hipThreadExchangeStreamCaptureMode(&mode);
     return ok;
 }

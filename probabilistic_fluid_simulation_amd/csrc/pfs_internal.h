@@ -109,9 +109,10 @@ struct StepArgs {
 int fused_step(const StepArgs &a, float *ws, hipStream_t s, hipEvent_t *ev, int reps = 1);
 size_t fused_workspace_bytes(int w, int h);
 // The sweeps of the operators diffuse and computePressure on 4-channel,
-// 16-byte aligned fields, kOpMinIters sweeps or more, in a few launches (the
-// same workspace).
+// 16-byte aligned fields, kOpMinIters sweeps or more, in a few launches (a
+// workspace of op_workspace_bytes(w, h)).
 constexpr int kOpMinIters = 5;
+size_t op_workspace_bytes(int w, int h);
 int diffuse_op(const float *a, float *last, float *before, int w, int h, float dt, float visc,
                int iters, float *ws, hipStream_t s);
 int pressure_op(float *a, float *last, float *before, int w, int h, float dt, int iters, float *ws,

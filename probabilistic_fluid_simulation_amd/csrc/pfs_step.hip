@@ -291,9 +291,14 @@ int fused_step(const StepArgs &s, float *ws, hipStream_t stream, hipEvent_t *ev,
 // the step's wave tiles.  a holds the input; on return the last iterate is in
 // `last` and the one before it in `before` (the two fields, in the order the
 // reference's pointer swaps leave them).  Other channels keep their values.
+// Workspace (floats, N = w*h): the iterates of u and v in [0, 2N) and [2N, 4N),
+// or the divergence in [0, N) and the iterates of p in [N, 2N) and [2N, 3N).
+size_t op_workspace_bytes(int w, int h) { return 4 * (size_t)w * h * sizeof(float); }
+
 int diffuse_op(const float *a, float *last, float *before, int w, int h, float dt, float visc,
                int iters, float *ws, hipStream_t stream) {
     DiffuseArgs d = diffuse_args(a, a, w, h, dt, visc, iters, ws);
+    float2 *plane[2] = {reinterpret_cast<float2 *>(ws), reinterpret_cast<float2 *>(ws) + (size_t)w * h};
     d.field[0] = last;
     d.field[1] = before;
     const OpPlan plan = op_plan(iters, w, h);
@@ -302,7 +307,8 @@ int diffuse_op(const float *a, float *last, float *before, int w, int h, float d
         const int ns = c == 0 ? plan.first : c == n - 1 ? plan.last : plan.first;
         const From from = c == 0 ? From::Field : From::Plane;
         const To to = c == n - 1 ? To::Field : To::Plane;
-        diffuse_chunk(d, c, Chunk{ns, ns, c == 0, c == n - 1}, ws);
+        d.dsrc = plane[(c + 1) & 1];
+        d.ddst = plane[c & 1];
         const WaveShape sh = wave_args(d, ns);
         hipLaunchKernelGGL(sh.S == 2 ? diffuse_op_for<2>(ns, from, to) : diffuse_op_for<4>(ns, from, to),
                            dim3(d.ntiles), dim3(64 * sh.nw), 0, stream, d);
@@ -314,8 +320,9 @@ int diffuse_op(const float *a, float *last, float *before, int w, int h, float d
 int pressure_op(float *a, float *last, float *before, int w, int h, float dt, int iters, float *ws,
                 hipStream_t stream) {
     PressureArgs p = pressure_args(a, a, nullptr, nullptr, w, h, dt, ws);
+    float *plane[2] = {ws + (size_t)w * h, ws + 2 * (size_t)w * h};
     p.gamma = pressure_gamma(dt);
-    p.bdst = ws + (size_t)w * h;  // what bpl reads
+    p.bpl = p.bdst = ws;
     p.field[0] = last;
     p.field[1] = before;
     const OpPlan plan = op_plan(iters, w, h);
@@ -324,7 +331,8 @@ int pressure_op(float *a, float *last, float *before, int w, int h, float dt, in
         const int ns = c == 0 ? plan.first : c == n - 1 ? plan.last : plan.first;
         const From from = c == 0 ? From::Field : From::Plane;
         const To to = c == n - 1 ? To::Field : To::Plane;
-        pressure_chunk(p, c, Chunk{ns, ns, false, c == n - 1}, ws, nullptr, nullptr, 1);
+        p.psrc = plane[(c + 1) & 1];
+        p.pdst = plane[c & 1];
         const WaveShape sh = wave_args(p, ns);
         hipLaunchKernelGGL(sh.S == 2 ? pressure_op_for<2>(ns, from, to) : pressure_op_for<4>(ns, from, to),
                            dim3(p.ntiles), dim3(64 * sh.nw), 0, stream, p);

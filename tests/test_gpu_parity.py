@@ -160,6 +160,80 @@ def test_operator_sweeps_on_general_path():
         assert (vp.numpy().tobytes(), tmp.numpy().tobytes()) == want
 
 
+def test_operators_leave_a_captured_step_its_workspace(orc):
+    """A step captured by the caller replays after operators on a larger field
+    have run on its stream: their workspace is not the one the graph names."""
+    s = scenes.random_scene(64, 48, 64, 48, seed=91, dt=0.7, visc=0.3, iters=12)
+    big = scenes.random_scene(700, 500, 1, 1, seed=92, dt=0.7, visc=0.3)
+    bufs, (a, b) = to_dev(s), (VPField.from_numpy(x) for x in (big.vp, big.tmp))
+    st = torch.cuda.Stream()
+    fluid.fluid_timestep(*bufs, s.dt, s.visc, s.iters, stream=st)  # sizes the workspace
+    fluid.fluid_timestep(*bufs, s.dt, s.visc, s.iters, stream=st)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        for _ in range(2):
+            fluid.fluid_timestep(*bufs, s.dt, s.visc, s.iters, stream=torch.cuda.current_stream())
+    for _ in range(3):
+        with torch.cuda.stream(st):
+            g.replay()
+            fluid.diffuse(a, b, big.visc, big.dt, 12)
+            fluid.computePressure(b, a, big.dt, 12)
+        torch.cuda.synchronize()
+    assert_bitexact(tuple(f.numpy() for f in bufs), oracle_run(orc, s, 8))
+
+
+def _held(run):
+    """Device memory that run() leaves taken."""
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    run()
+    torch.cuda.synchronize()
+    return before - torch.cuda.mem_get_info()[0]
+
+
+def test_operators_workspaces_stay_bounded():
+    """The operators keep 256 MiB a device at most: a field that needs more runs a
+    launch per sweep, and so do streams that come after the bound is reached;
+    results as on the per-operator path."""
+    k, visc, dt = 7, 0.3, 0.7
+    gen = torch.Generator("cuda").manual_seed(93)
+
+    def fields(w, h):
+        return [VPField(torch.rand(h, w, 4, device="cuda", generator=gen)) for _ in range(2)]
+
+    def both(f, st=None):
+        fluid.diffuse(*f, visc, dt, k, stream=st)
+        fluid.computePressure(*f, dt, k, stream=st)
+
+    warm, big = fields(64, 64), fields(6000, 3000)
+    keep = [VPField(f.data.clone()) for f in big]
+    both(warm)
+    assert _held(lambda: both(big)) < 16 << 20  # 275 MiB at 16 B a cell
+    fluid.set_step_path("per_op")
+    both(keep)
+    fluid.set_step_path("auto")
+    assert all(torch.equal(p.data, q.data) for p, q in zip(big, keep))
+    del big, keep
+
+    streams = [torch.cuda.Stream() for _ in range(12)]
+    sets = [fields(2000, 1500) for _ in streams]  # 46 MiB each
+    want = [f.data.clone() for f in sets[0]]
+    for f in sets:
+        for p, q in zip(f, want):
+            p.data.copy_(q)
+    for st in streams:  # the streams' own memory
+        for _ in range(3):
+            both(warm, st)
+
+    def each():
+        for f, st in zip(sets, streams):
+            both(f, st)
+
+    assert _held(each) < 272 << 20
+    assert all(torch.equal(p.data, q.data) for f in sets[1:] for p, q in zip(f, sets[0]))
+
+
 def test_operators_from_threads_on_one_stream(orc):
     """Threads that share a stream share its workspace: their calls' launches
     do not interleave."""
