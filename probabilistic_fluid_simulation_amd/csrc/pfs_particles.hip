@@ -33,6 +33,7 @@
 
 #include "pfs.h"
 #include "pfs_device.h"
+#include "pfs_grid.h"
 #include "pfs_internal.h"
 
 namespace pfs {
@@ -1215,7 +1216,7 @@ __global__ void k_pbf_init(PbfCtl *ctl, double *res, int nres) {
     for (int k = threadIdx.x; k < nres; k += blockDim.x) res[k] = -1.0;  // not computed
 }
 
-int grid_for(int n) { return (n + 255) / 256; }
+int grid_for(int n) { return blocks_for(n, 256); }
 // Particles from which the density and the counts take one lane each instead
 // of four: 4 wavefronts for every SIMD then.  Density with counts, one lane
 // against four, us: 65,536 particles of 20 neighbours 14.2 / 9.9, 131,072
@@ -1306,7 +1307,7 @@ struct SortArgs {
 
 template <int RB, int NT>
 void sort_passes(const SortArgs &a, int passes) {
-    const int nb = (a.n + sort_tile<NT>() - 1) / sort_tile<NT>();
+    const int nb = blocks_for(a.n, sort_tile<NT>());
     const uint32_t *kin = a.keys;
     for (int p = 0; p < passes; ++p) {
         const int shift = RB * p;

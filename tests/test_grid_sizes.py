@@ -1,0 +1,37 @@
+"""Launch sizes at the counts where 32 bits end (csrc/pfs_grid.h), CPU only:
+the header itself, compiled with g++."""
+from __future__ import annotations
+
+import os
+import shutil
+import subprocess
+import tempfile
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
+                    "probabilistic_fluid_simulation_amd", "csrc")
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+
+
+def _run(body):
+    with tempfile.TemporaryDirectory() as d:
+        src, exe = os.path.join(d, "t.cpp"), os.path.join(d, "t")
+        with open(src, "w") as f:
+            f.write('#include "pfs_grid.h"\n#include <cstdio>\nint main() {\n' + body + "}\n")
+        subprocess.run(["g++", "-O1", "-std=c++17", "-fsanitize=undefined", "-I", CSRC, src, "-o", exe],
+                       check=True)
+        out = subprocess.run([exe], capture_output=True, text=True, check=True)
+    assert out.stderr == ""
+    return [[int(t) for t in line.split()] for line in out.stdout.splitlines()]
+
+
+COUNTS = [1, 255, 256, 257, 2**30, 2**30 + 1, 2**31 - 4096, 2**31 - 4095, 2**31 - 256, 2**31 - 1]
+
+
+@pytest.mark.parametrize("per", [256, 1024, 2048, 4096])
+def test_block_counts(per):
+    """A block for every `per` items, up to the last int (the sort's tiles and
+    one thread a particle)."""
+    rows = _run("".join(f'  std::printf("%d\\n", pfs::blocks_for({n}, {per}));\n' for n in COUNTS))
+    assert [r[0] for r in rows] == [-(-n // per) for n in COUNTS]
