@@ -673,10 +673,14 @@ __device__ __forceinline__ void for_neighbors_serial(const NArgs &a, int p, F &&
         scan);
 }
 
-// 256 threads: 256 / L particles.
+// 256 threads: 256 / L particles; blocks in rows (pfs_grid.h).
+template <int L>
+__device__ __forceinline__ unsigned group_first() {
+    return (blockIdx.y * gridDim.x + blockIdx.x) * (256 / L);
+}
 template <int L>
 __device__ __forceinline__ int group_particle() {
-    return (int)(blockIdx.x * (blockDim.x / L) + threadIdx.x / L);
+    return (int)(group_first<L>() + threadIdx.x / L);
 }
 
 template <int L>
@@ -735,8 +739,8 @@ __global__ __launch_bounds__(256) void k_nbr_fill_lds(NArgs a, const uint32_t *_
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     constexpr int PW = 64 / L;  // particles of a wave
     const int p = group_particle<L>();
-    const int pw = blockIdx.x * (blockDim.x / L) + wave * PW;  // the wave's first particle
-    if (pw >= a.n) return;                                     // the whole wave is past the end
+    const int pw = (int)group_first<L>() + wave * PW;  // the wave's first particle
+    if (pw >= a.n) return;                             // the whole wave is past the end
     const int plast = min(pw + PW - 1, a.n - 1);
     const uint32_t below = (1u << group_lane<L>()) - 1u;
     const size_t base = offsets[pw], end = (size_t)offsets[plast] + counts[plast];
@@ -1227,7 +1231,10 @@ constexpr int kSerialFrom = 1 << 18;
 // 68 / 119, 262,144 145 / 372 against 137 / 312, 393,216 171 / 498 against 183 /
 // 420, 1,048,576 360 / 1054 against 452 / 1027.
 constexpr int kPbfSerialFrom = 3 << 17;
-int group_grid(int n, int L) { return (int)(((long long)n * L + 255) / 256); }  // 256 threads, L a particle
+dim3 group_grid(int n, int L) {  // 256 threads, L a particle
+    const Blocks b = block_rows(blocks_for(n, 256 / L));
+    return dim3(b.x, b.y);
+}
 // Lanes a particle of the counts and lists (which no order binds): 16 where four
 // leave the GPU short of wavefronts and a row's candidates are several loads one
 // after another.  Grid's counts, scan, fill, four lanes against 16, us: 16,384
@@ -1399,7 +1406,7 @@ int lists_from_counts(const pfs_ngrid *g, const NArgs &a, const uint32_t *counts
                                               std::to_string(nbr_capacity) + " < " +
                                               std::to_string(h_total));
     const int L = list_lanes(g->n);
-    const dim3 grid(group_grid(g->n, L));
+    const dim3 grid = group_grid(g->n, L);
     if (a.order)
         hipLaunchKernelGGL(L == 16 ? k_nbr_fill<16> : k_nbr_fill<4>, grid, dim3(256), 0, s, a,
                            offsets, nbr, nbr_capacity);
@@ -1521,7 +1528,7 @@ int pfs_ngrid_neighbors(const pfs_ngrid *g, const float *xs, const float *ys, co
     const NArgs a = nargs(g, xs, ys, order, w.k0, cell_start, cell_end);
     if (g->n < kSerialFrom)
         hipLaunchKernelGGL(list_lanes(g->n) == 16 ? k_nbr_count<16> : k_nbr_count<4>,
-                           dim3(group_grid(g->n, list_lanes(g->n))), dim3(256), 0, s, a, counts);
+                           group_grid(g->n, list_lanes(g->n)), dim3(256), 0, s, a, counts);
     else
         hipLaunchKernelGGL(k_nbr_count_serial, dim3(grid_for(g->n)), dim3(256), 0, s, a, counts);
     if (!nbr) return scan_exclusive(counts, offsets, g->n, total, w.sums, s);  // no lists
@@ -1643,7 +1650,7 @@ int pfs_ngrid_density(const pfs_ngrid *g, const float *xs, const float *ys, cons
     const float coef = (float)(4.0 / (3.14159265358979323846 * r * r * r * r * r * r * r * r));
     const float mc = mass * coef;
     if (g->n < kSerialFrom)
-        hipLaunchKernelGGL(k_density, dim3(group_grid(g->n, 4)), dim3(256), 0, s, a, mc, rho, counts);
+        hipLaunchKernelGGL(k_density, group_grid(g->n, 4), dim3(256), 0, s, a, mc, rho, counts);
     else
         hipLaunchKernelGGL(k_density_serial, dim3(grid_for(g->n)), dim3(256), 0, s, a, mc, rho, counts);
     return check_launch("density");

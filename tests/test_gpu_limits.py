@@ -76,3 +76,46 @@ def test_largest_fields_fixed_point(w, h):
     assert torch.equal(_bits(I.data), _bits(img0)), "dye after advect_color_step"
     del V, T, I, IT, vp, img, vp0, img0
     torch.cuda.empty_cache()
+
+
+def test_lists_of_more_than_2_30_particles():
+    """2^30 + 2 particles in 2^30 cells: pairs 0.25 apart and more than a radius
+    from any other, and one place of four.  Every count, offset and list, by
+    particle and by sorted position (four lanes a particle: 2^32 threads)."""
+    from probabilistic_fluid_simulation_amd import particles
+
+    n, side = 2**30 + 2, 32768
+    need = 120 << 30
+    free, _ = torch.cuda.mem_get_info()
+    if free < need:
+        pytest.skip(f"needs {need / 2**30:.0f} GiB of free device memory, {free / 2**30:.0f} free")
+    k = torch.arange(n, device="cuda", dtype=torch.int32)
+    x = (k >> 1) % (side // 2) * 2 + (k & 1) * 0.25 + 0.25
+    y = torch.div(k >> 1, side // 2, rounding_mode="floor") + 0.5
+    x[-2:], y[-2:] = x[:2], y[:2]
+    ng = particles.NeighborGrid(n, float(side), float(side), 1.0)
+    assert ng.cells == (side, side)
+    ng.build(x, y)
+    assert torch.equal(ng.xs[4:], x[2:-2]) and torch.equal(ng.ys[4:], y[2:-2])
+    del x, y
+
+    def check(four, rest, partners):
+        counts, offsets, nbr = ng.neighbors(by_position=four is None)
+        quad = [0, 1, 2, 3] if four is None else four
+        assert nbr.numel() == n - 4 + 12
+        assert counts[quad].tolist() == [3] * 4 and int((counts == 1).sum()) == n - 4
+        for i in quad:
+            o = int(offsets[i])
+            assert nbr[o:o + 3].tolist() == [j for j in quad if j != i]
+        lo, hi = rest
+        first = int(offsets[lo])
+        assert torch.equal(offsets[lo:hi], torch.arange(first, first + hi - lo, device="cuda", dtype=torch.int32))
+        assert torch.equal(nbr[first:first + hi - lo], partners(lo, hi))
+
+    def xor1(lo, hi):
+        return torch.arange(lo, hi, device="cuda", dtype=torch.int32) ^ 1
+
+    check([0, 1, n - 2, n - 1], (2, n - 2), xor1)
+    check(None, (4, n), xor1)
+    del ng, k
+    torch.cuda.empty_cache()

@@ -35,3 +35,14 @@ def test_block_counts(per):
     one thread a particle)."""
     rows = _run("".join(f'  std::printf("%d\\n", pfs::blocks_for({n}, {per}));\n' for n in COUNTS))
     assert [r[0] for r in rows] == [-(-n // per) for n in COUNTS]
+
+
+def test_block_rows():
+    """Four lanes a particle (64 particles a block): every block is there, no
+    row reaches 2^32 threads, no block's first particle passes 2^31 - 1."""
+    blocks = [1, 2**23 - 1, 2**23, 2**23 + 1, 2**24, 2**24 + 1, -(-(2**31 - 1) // 64)]
+    rows = _run("".join(f'  {{ auto b = pfs::block_rows({k}); std::printf("%u %u\\n", b.x, b.y); }}\n'
+                        for k in blocks))
+    for k, (x, y) in zip(blocks, rows):
+        assert k <= x * y < k + x and x * 256 < 2**32 and y < 2**16
+        assert (x * y - 1) * 64 + 63 < 2**31
