@@ -41,10 +41,11 @@ __device__ __forceinline__ T div_n(T x, T n, T inv_n, bool n_pow2) {
 __device__ __forceinline__ float div_fast2(float x, const FixedDiv &d) {
     return fmaf(x, d.hi, x * d.lo);
 }
-// A back-trace's displacement x / n.  x needs no range test: below 2^-96,
-// where x*lo may round as a subnormal, the quotient only ever meets a cell
-// coordinate (0 or at least 1) in a subtraction and the wrap's addition of n,
-// neither of which it can change.
+// A back-trace's displacement x / n.  x needs no range test: a product x*lo that
+// rounds as a subnormal is off by 2^-150 at most, which only a quotient below
+// 2^-103 can show, and the quotient only ever meets a cell coordinate (0 or at
+// least 1) in a subtraction and the wrap's addition of n, neither of which one
+// that small can change.
 __device__ __forceinline__ float div_const(float x, float n, const FixedDiv &d) {
     return d.ok ? div_fast2(x, d) : x / n;
 }

@@ -55,4 +55,17 @@ inline FixedDiv prove_fixed_div(float d) {
     return f;
 }
 
+// The constants for a field's side n up to 2^24 (every such side is a float),
+// from those that `fixed` (prove_fixed_div) gives up to 2^17: a larger side's are
+// its 128th's, scaled exactly.  Every side up to 4,159,486 is proven.
+template <typename Fixed>
+inline FixedDiv side_div(float n, Fixed &&fixed) {
+    if (n <= 131072.0f) return fixed(n);
+    if (!(n <= 16777216.0f)) return FixedDiv{0.0f, 0.0f, 0};
+    FixedDiv f = fixed(n * 0x1p-7f);
+    f.hi *= 0x1p-7f;
+    f.lo *= 0x1p-7f;
+    return f;
+}
+
 }  // namespace pfs

@@ -617,8 +617,8 @@ inline DiffuseArgs diffuse_args(const float *P, const float *Q, int w, int h, fl
     d.beta = (float)(1.0 + 4.0 * (double)d.alpha);
     d.rcp_beta = 1.0f / d.beta;
     d.fast_div = d.beta >= 0x1p-20f && d.beta <= 0x1p20f;  // false for NaN
-    d.dw = fixed_div(d.fw);
-    d.dh = fixed_div(d.fh);
+    d.dw = side_div(d.fw, fixed_div);
+    d.dh = side_div(d.fh, fixed_div);
     d.db = FixedDiv{};
     if (d.beta >= 1.0f && d.beta <= 64.0f) {
         // Numerators of at least 2^-96 then keep x*lo and the quotient far

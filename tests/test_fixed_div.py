@@ -65,3 +65,44 @@ def test_proven_divisors_divide_exactly():
     assert tried >= 40 and refused < 20   # most divisors are proven
     assert ints == 131072                 # every field side up to 2^17 is
     assert outside == 0
+
+
+SIDES = r"""
+#include "pfs_fixed_div.h"
+#include <cstdio>
+#include <cstring>
+#include <initializer_list>
+static uint32_t bits(float f) { uint32_t u; std::memcpy(&u, &f, 4); return u; }
+int main() {
+  long refused = 0, bad = 0;
+  #pragma omp parallel for reduction(+:refused) schedule(dynamic, 4096)
+  for (int n = 131073; n <= 4159487; ++n) refused += !pfs::side_div((float)n, pfs::prove_fixed_div).ok;
+  for (float n : {131072.0f, 131073.0f, 200003.0f, 262144.0f, 1000001.0f, 4159486.0f, 16777213.0f, 16777216.0f}) {
+    const pfs::FixedDiv d = pfs::side_div(n, pfs::prove_fixed_div);
+    if (!d.ok) { ++bad; continue; }
+    #pragma omp parallel for reduction(+:bad)
+    for (uint32_t m = 1u << 23; m < 1u << 24; ++m) {
+      const float x = (float)m, t = x * d.lo;
+      if (bits(std::fmaf(x, d.hi, t)) != bits(x / n)) ++bad;
+    }
+  }
+  int outside = 0;
+  for (float n : {16777218.0f, 33554432.0f, INFINITY, NAN}) outside += pfs::side_div(n, pfs::prove_fixed_div).ok;
+  std::printf("%ld %ld %d\n", refused, bad, outside);
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+def test_sides_past_2_17_divide_exactly():
+    """Field sides above what prove_fixed_div takes: all are proven up to
+    4,159,486 (the next is the first that is not), and those tried divide every
+    significand exactly."""
+    with tempfile.TemporaryDirectory() as d:
+        src, exe = os.path.join(d, "side.cpp"), os.path.join(d, "side")
+        with open(src, "w") as f:
+            f.write(SIDES)
+        subprocess.run(["g++", "-O2", "-std=c++17", "-mfma", "-ffp-contract=off", "-fopenmp",
+                        "-I", CSRC, src, "-o", exe], check=True)
+        out = subprocess.run([exe], capture_output=True, text=True, check=True).stdout
+    assert out.split() == ["1", "0", "0"]

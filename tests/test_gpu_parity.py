@@ -584,6 +584,14 @@ def test_plain_step_at_2048_bitexact(orc):
     assert_bitexact(gpu_run(s, 1, combined=True), oracle_run(orc, s, 1))
 
 
+@pytest.mark.parametrize("w,h", [(131073, 5), (200003, 41), (262144, 30), (7, 150001)])
+def test_sides_past_2_17(orc, w, h):
+    """Fields longer than 2^17 cells, whose back-trace divides by a scaled side:
+    traces within the staged cells and longer ones."""
+    s = scenes.random_scene(w, h, w, h, seed=w % 97, dt=0.5, visc=0.2, iters=5, vel_scale=3.0 * w)
+    assert_bitexact(gpu_run(s, 2, combined=True), oracle_run(orc, s, 2))
+
+
 def test_stream_and_repeat_determinism(orc):
     s = scenes.random_scene(150, 90, 150, 90, seed=13, dt=0.7, visc=0.2, iters=8)
     st = torch.cuda.Stream()
