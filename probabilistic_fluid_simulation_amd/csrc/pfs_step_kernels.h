@@ -72,8 +72,7 @@ struct DiffuseArgs {
     float *pw;           // pressure-start plane (last chunk)
     float *bpl;          // divergence plane (last chunk)
     int w, h, tiles_x, ntiles;
-    float dt, fw, fh, inv_w, inv_h;
-    int pow2_w, pow2_h;
+    float dt, fw, fh;
     float alpha, beta, rcp_beta, gamma;
     int fast_div;  // division by beta: 0 IEEE, 1 five operations, 2 two (proven for it)
     FixedDiv db, dw, dh;  // beta, w and h as fixed divisors
@@ -95,7 +94,6 @@ struct PressureArgs {
     int w, h, tiles_x, ntiles;
     float dt, fw, fh, inv_w, inv_h;
     int pow2_w, pow2_h;
-    FixedDiv dw, dh;       // w and h as fixed divisors
     float dt_viw, dt_vih;  // dt / (field/image width ratio), as src/fluid.cpp:97-98
     int first;
     int tile_base;  // first tile of this scene in a batched launch
@@ -608,10 +606,6 @@ inline DiffuseArgs diffuse_args(const float *P, const float *Q, int w, int h, fl
     d.dt = dt;
     d.fw = (float)w;
     d.fh = (float)h;
-    d.inv_w = 1.0f / (float)w;
-    d.inv_h = 1.0f / (float)h;
-    d.pow2_w = (w & (w - 1)) == 0;
-    d.pow2_h = (h & (h - 1)) == 0;
     // diffuse's coefficients, src/fluid.cpp:144-145 (beta evaluated in double)
     d.alpha = visc * dt;
     d.beta = (float)(1.0 + 4.0 * (double)d.alpha);
@@ -663,8 +657,6 @@ inline PressureArgs pressure_args(float *P, float *Q, const float *image, float 
     p.inv_h = 1.0f / (float)h;
     p.pow2_w = (w & (w - 1)) == 0;
     p.pow2_h = (h & (h - 1)) == 0;
-    p.dw = fixed_div(p.fw);
-    p.dh = fixed_div(p.fh);
     // src/fluid.cpp:82-83,97-98 with the image the size of the field.
     const float viw = (float)w / (float)w, vih = (float)h / (float)h;
     p.dt_viw = dt / viw;
