@@ -214,7 +214,7 @@ def small_scene_leg() -> dict:
     run_same = all(np.asarray(g).tobytes() == np.asarray(w).tobytes()
                    for g, w in zip(got_run, want_run))
     same = all(np.asarray(g).tobytes() == np.asarray(w).tobytes() for g, w in zip(got, want))
-    return {"workload": s.name, "steps": n, "tile": fluid.get_step_tile(128, 128, s.iters, True),
+    return {"workload": s.name, "steps": n, "tile": fluid.get_step_side(128, 128, s.iters, True),
             "gpu_us_per_step": gpu_ms * 1e3, "gpu_cell_steps_per_s": s.cells / (gpu_ms * 1e-3),
             "gpu_run_us_per_step": run_ms * 1e3, "gpu_run_bit_exact": bool(run_same),
             "cpu_us_per_step": cpu_s / n * 1e6, "cpu_cell_steps_per_s": s.cells * n / cpu_s,
@@ -222,10 +222,11 @@ def small_scene_leg() -> dict:
 
 
 def tiles_leg(reps: int = 50) -> dict:
-    """The fused kernels' tile side over field sizes: pfs_autotune_step times
+    """The fused kernels' tile class over field sizes: pfs_autotune_step times
     a whole timestep (field and dye of one size, dt = 1/120, nu = 0.1) for
-    the sides 64, 32 and 16 on scratch copies, and the rule's side beside
-    the measured fastest.  The first shape is the 128x128, K = 4 scene."""
+    the classes 64, 32 and 16 on scratch copies; beside the measured fastest
+    the side that an untuned step takes ("side") and its class ("rule").  The
+    first shape is the 128x128, K = 4 scene."""
     import torch
 
     from probabilistic_fluid_simulation_amd import fluid, scenes
@@ -237,10 +238,10 @@ def tiles_leg(reps: int = 50) -> dict:
         vp, tmp = fluid.VPField.from_numpy(s.vp), fluid.VPField.from_numpy(s.tmp)
         im, itmp = fluid.VPField.from_numpy(s.image), fluid.VPField.from_numpy(s.itmp)
         fluid.clear_step_tuning()
-        rule = fluid.get_step_tile(n, n, k, dye_fused=True)
+        own = fluid.get_step_side(n, n, k, dye_fused=True)
         side, ms = fluid.autotune_step(vp, tmp, s.dt, s.visc, k, image=im, itmp=itmp, reps=reps)
         out[s.name] = {"us_per_step": {str(t): m * 1e3 for t, m in ms.items()},
-                       "fastest": side, "rule": rule}
+                       "fastest": side, "rule": fluid.tile_class(own), "side": own}
         del vp, tmp, im, itmp
     fluid.clear_step_tuning()
     torch.cuda.synchronize()

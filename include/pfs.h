@@ -179,8 +179,13 @@ int pfs_get_step_path(void);
  * the smallest such side of all.  side 0 clears a forced class. */
 int pfs_set_step_tile(int side);
 /* The class forced or measured for this shape, else the largest of 64, 32 and
- * 16 with a tile for every two CUs (16 if none); < 0 on error. */
+ * 16 with a tile for every two CUs (16 if none); < 0 on error.  A step of a shape
+ * neither forced nor measured need not be of that class: see the next. */
 int pfs_get_step_tile(int vx, int vy, int iters, int dye_fused);
+/* The side, 8 to 64, of the square tiles that a step of this shape takes now;
+ * < 0 on error.  Forcing the class it lies in (16 up to 24, 32 up to 40, else
+ * 64) gives the same side. */
+int pfs_get_step_side(int vx, int vy, int iters, int dye_fused);
 /* Times pfs_fluid_timestep (image/itmp NULL: pfs_simulate_fluid_step) on
  * scratch copies of the buffers, `reps` steps per side after one untimed
  * step, for the sides 64, 32 and 16 in that order (ms[0..2], per step, if

@@ -79,6 +79,7 @@ SIGNATURES = {
     "pfs_set_step_path": [_I],
     "pfs_set_step_tile": [_I],
     "pfs_get_step_tile": [_I, _I, _I, _I],
+    "pfs_get_step_side": [_I, _I, _I, _I],
     "pfs_autotune_step": [_P, _P, _P, _P, _F, _F, _I, _I, _V, ctypes.POINTER(ctypes.c_int),
                           ctypes.POINTER(ctypes.c_float), _I],
     "pfs_clear_step_tuning": [],

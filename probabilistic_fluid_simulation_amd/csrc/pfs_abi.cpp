@@ -674,6 +674,11 @@ int pfs_get_step_tile(int vx, int vy, int iters, int dye_fused) {
     return tile ? tile : tile_for_counts(tile_count(vx, vy, 64), tile_count(vx, vy, 32));
 }
 
+int pfs_get_step_side(int vx, int vy, int iters, int dye_fused) {
+    if (vx < 1 || vy < 1 || iters < 1) return set_error(PFS_ERR_INVALID, "bad step shape");
+    return tile_side(set_tile(vx, vy, iters, dye_fused != 0), vx, vy);
+}
+
 int pfs_autotune_step(const pfs_field *vp, const pfs_field *tmp, const pfs_field *image,
                       const pfs_field *itmp, float dt, float viscosity, int iters, int reps,
                       void *stream, int *side, float *ms, int n_ms) {

@@ -117,6 +117,8 @@ int diffuse_op(const float *a, float *last, float *before, int w, int h, float d
                int iters, float *ws, hipStream_t s);
 int pressure_op(float *a, float *last, float *before, int w, int h, float dt, int iters, float *ws,
                 hipStream_t s);
+// The square tiles' side in a step with that tile class (0: any).
+int tile_side(int tile, int w, int h);
 int threads_for(int H, int ts = 64);  // threads of the fused kernels for halo H, tile side ts
 
 // Validation helpers.

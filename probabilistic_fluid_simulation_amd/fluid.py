@@ -288,17 +288,32 @@ TILE_SIDES = (64, 32, 16)
 
 
 def set_step_tile(side: int) -> None:
-    """Force the fused step's tile side (16, 32 or 64); 0 returns to the
-    automatic choice (the autotuner's record for the shape, else the rule)."""
+    """Force the fused step's tile class (16, 32 or 64); 0 returns to the
+    automatic choice (the autotuner's record for the shape, else the step's own)."""
     _lib.call("pfs_set_step_tile", side)
 
 
 def get_step_tile(w: int, h: int, iters: int, dye_fused: bool = False) -> int:
-    """The tile side a step of this shape takes now."""
+    """The tile class forced or measured for this shape, else the largest of
+    64, 32 and 16 with a tile for every two CUs (16 if none)."""
+    return _step_query("pfs_get_step_tile", w, h, iters, dye_fused)
+
+
+def get_step_side(w: int, h: int, iters: int, dye_fused: bool = False) -> int:
+    """The side of the square tiles that a step of this shape takes now, 8 to 64."""
+    return _step_query("pfs_get_step_side", w, h, iters, dye_fused)
+
+
+def tile_class(side: int) -> int:
+    """The class (a value of set_step_tile) that a side lies in."""
+    return 16 if side <= 24 else 32 if side <= 40 else 64
+
+
+def _step_query(name: str, w: int, h: int, iters: int, dye_fused: bool) -> int:
     lib = _lib.load()
-    side = lib.pfs_get_step_tile(w, h, iters, int(bool(dye_fused)))
+    side = getattr(lib, name)(w, h, iters, int(bool(dye_fused)))
     if side < 0:
-        raise _lib.PfsError("pfs_get_step_tile", side, lib.pfs_last_error().decode(errors="replace"))
+        raise _lib.PfsError(name, side, lib.pfs_last_error().decode(errors="replace"))
     return side
 
 

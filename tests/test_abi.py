@@ -14,7 +14,7 @@ import subprocess
 import numpy as np
 import pytest
 
-from probabilistic_fluid_simulation_amd import _lib, scenes
+from probabilistic_fluid_simulation_amd import _lib, fluid, scenes
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -165,6 +165,28 @@ def test_step_tile_rule_and_forcing():
         with pytest.raises(_lib.PfsError):
             _lib.call("pfs_set_step_tile", bad)
     assert lib.pfs_get_step_tile(0, 5, 8, 0) < 0
+
+
+@pytest.mark.parametrize("w,h,side", [
+    (1, 1, 8), (128, 128, 8), (129, 128, 12), (320, 240, 20), (360, 360, 24), (512, 512, 32),
+    (640, 480, 36), (700, 700, 48), (1024, 1024, 64), (1100, 1024, 48), (3840, 2160, 64)])
+def test_step_side_reported_is_the_one_taken(w, h, side):
+    """The automatic side with 256 CUs (the default where no device answers);
+    forcing the class it lies in changes nothing, and what a step of another class
+    takes is reported too."""
+    lib = _lib.load()
+    lib.pfs_clear_step_tuning()
+    assert fluid.get_step_side(w, h, 8, True) == side
+    try:
+        fluid.set_step_tile(fluid.tile_class(side))
+        assert fluid.get_step_side(w, h, 8, True) == side
+        for c in (16, 32, 64):
+            fluid.set_step_tile(c)
+            assert fluid.tile_class(fluid.get_step_side(w, h, 8, True)) == c
+    finally:
+        fluid.set_step_tile(0)
+    with pytest.raises(_lib.PfsError):
+        fluid.get_step_side(0, 5, 8)
 
 
 def test_splitmix64_published_vector():
