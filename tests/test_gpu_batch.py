@@ -54,6 +54,32 @@ def test_batch_mixed_scenes(orc, graphs, tile):
     b.close()
 
 
+CHUNKS = {  # field w, h, dye w, h, K, channels
+    # launches of 8 + 8 + 1 and 8 + 8 + 8 + 1 sweeps in wave tiles of 2 rows a wave
+    "2-rows": [(150, 90, 150, 90, 17, 4), (301, 64, 97, 301, 17, 4), (40, 33, 40, 33, 25, 4),
+               (257, 130, 257, 130, 25, 4), (130, 67, 130, 67, 8, 4), (64, 64, 64, 64, 16, 4)],
+    # enough cells a group for 4 rows a wave
+    "4-rows": [(900, 600, 900, 600, 17, 4), (129, 77, 129, 77, 17, 4), (1000, 700, 500, 350, 25, 4),
+               (70, 300, 70, 300, 25, 4), (800, 900, 800, 900, 16, 4)],
+}
+
+
+@pytest.mark.parametrize("tile", [32, 64], ids=["t32", "t64"])
+@pytest.mark.parametrize("mix", list(CHUNKS))
+def test_batch_many_chunks(orc, mix, tile):
+    """Scenes of several launches a solve, chunks in the middle among them, whose
+    tile tables chunks of one halo share."""
+    b = Batch()
+    sc = [_scene(i, spec) for i, spec in enumerate(CHUNKS[mix])]
+    slots = [b.add(*to_dev(s), s.dt, s.visc, s.iters) for s in sc]
+    b.set_tile(tile)
+    steps = 11 if mix == "2-rows" else 3
+    b.step(steps)
+    for slot, s in zip(slots, sc):
+        _check(b, slot, s, orc, steps)
+    b.close()
+
+
 def test_batch_autotune_restores_the_scenes(orc):
     """autotune times every tile side on the live scenes, puts them back as
     they were (buffers and step counts), and forces the fastest side."""
