@@ -83,10 +83,11 @@ using PressureBatchFn = void (*)(const PressureArgs *, const int *, int);
 #define PFS_H_CASES(X) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9)
 
 DiffuseBatchFn diffuse_small_batch_for(int H, bool last) {
+    if (!last) return H == kMaxChunk ? k_diffuse_batch<kMaxChunk, false> : nullptr;
     switch (H) {
 #define PFS_CASE(h) \
     case h:         \
-        return last ? k_diffuse_batch<h, true> : k_diffuse_batch<h, false>;
+        return k_diffuse_batch<h, true>;
         PFS_H_CASES(PFS_CASE)
 #undef PFS_CASE
     }
@@ -111,10 +112,11 @@ DiffuseBatchFn diffuse_wave_batch_for(int H, bool first, bool last) {
 
 template <int TS>
 PressureBatchFn pressure_batch_for_ts(int H, bool last) {
+    if (!last) return H == kMaxChunk ? k_pressure_batch<kMaxChunk, false, TS> : nullptr;
     switch (H) {
 #define PFS_CASE(h) \
     case h:         \
-        return last ? k_pressure_batch<h, true, TS> : k_pressure_batch<h, false, TS>;
+        return k_pressure_batch<h, true, TS>;
         PFS_H_CASES(PFS_CASE)
 #undef PFS_CASE
     }

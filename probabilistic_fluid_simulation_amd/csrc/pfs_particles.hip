@@ -1315,6 +1315,7 @@ struct SortArgs {
 template <int RB, int NT>
 void sort_passes(const SortArgs &a, int passes) {
     const int nb = blocks_for(a.n, sort_tile<NT>());
+    const bool few = NT < kThreads && nb <= kFewTiles;  // past kSmallSort never
     const uint32_t *kin = a.keys;
     for (int p = 0; p < passes; ++p) {
         const int shift = RB * p;
@@ -1327,11 +1328,12 @@ void sort_passes(const SortArgs &a, int passes) {
         else
             hipLaunchKernelGGL((k_radix_hist<RB, NT, false>), dim3(nb), dim3(NT), 0, a.s, kin, a.ck,
                                nullptr, a.n, shift, a.w.hist, nb);
-        if (nb <= kFewTiles) {
-            hipLaunchKernelGGL((k_radix_scatter<RB, NT, true>), dim3(nb), dim3(NT), 0, a.s, kin, vin,
-                               a.kb[(p + 1) & 1], a.vb[(p + 1) & 1], a.n, shift, a.w.hist, a.w.tot, nb,
-                               a.x, a.y, oxs, oys);
-        } else {
+        if constexpr (NT < kThreads)
+            if (few)
+                hipLaunchKernelGGL((k_radix_scatter<RB, NT, true>), dim3(nb), dim3(NT), 0, a.s, kin, vin,
+                                   a.kb[(p + 1) & 1], a.vb[(p + 1) & 1], a.n, shift, a.w.hist, a.w.tot,
+                                   nb, a.x, a.y, oxs, oys);
+        if (!few) {
             if (nb <= sort_tile<256>())
                 hipLaunchKernelGGL(k_digit_rows<256>, dim3(1 << RB), dim3(256), 0, a.s, a.w.hist,
                                    a.w.tot, nb);
