@@ -14,7 +14,7 @@ __global__ __launch_bounds__((Geo<H, TS>::NT)) void k_diffuse(DiffuseArgs a) {
 
 template <int TS>
 DiffuseFn diffuse_for_ts(int H, bool last) {
-    if (!last) return H == kLongChunk ? k_diffuse<kLongChunk, false, TS> : k_diffuse<kMaxChunk, false, TS>;
+    if (!last) return H == kMaxChunk ? k_diffuse<kMaxChunk, false, TS> : nullptr;
     switch (H) {
 #define PFS_CASE(h) \
     case h:         \
