@@ -1226,7 +1226,8 @@ int grid_for(int n) { return blocks_for(n, 256); }
 // against four, us: 65,536 particles of 20 neighbours 14.2 / 9.9, 131,072
 // 14.9 / 12.0, 262,144 17.8 / 17.9, 1,048,576 41.3 / 60.8.
 constexpr int kSerialFrom = 1 << 18;
-// The same line for the constraint solve's passes.  4 iterations, one lane
+// The same line for the constraint solve's passes, by the count alone: sets of
+// long lists above it would still gain from four lanes.  4 iterations, one lane
 // against four, us: 65,536 particles of 7 / 37 neighbours 108 / 248 against
 // 68 / 119, 262,144 145 / 372 against 137 / 312, 393,216 171 / 498 against 183 /
 // 420, 1,048,576 360 / 1054 against 452 / 1027.

@@ -119,7 +119,11 @@ __device__ __forceinline__ void store_pair(float2 *p, float2 a, float2 b, bool t
 // read as VGPRs; and the sweep loop's values, which are loaded and stored as
 // vectors: left as parts of those vectors across the loop, the register
 // allocator of ROCm 7.2 gave one of them and a temporary the same register
-// (seen in the assembly, and in the results).
+// (seen in the assembly, and in the results).  So what a sweep loop carries or
+// reads and what was loaded as part of a vector takes a register of its own
+// before the loop, and u, v and the pressure again before they are stored as one.
+// The source does not tell which of them would fare badly without: every
+// instance of these kernels is compared bit for bit (tests/test_gpu_every_kernel.py).
 __device__ __forceinline__ float own_register(float x) {
     float y;
     asm("v_mov_b32 %0, %1" : "=v"(y) : "v"(x));
