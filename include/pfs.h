@@ -71,7 +71,7 @@ int pfs_advect_color(const pfs_field *image, pfs_field *out, const pfs_field *vp
 /* includes/fluid.hpp:58 / src/fluid.cpp:129-196.  `iters` Jacobi smoothing
  * sweeps of channels 0,1 between vp and vp_out; swaps the two structs' data
  * pointers after every sweep but the last.  From 5 sweeps on, 4-channel fields
- * aligned to 16 bytes run several sweeps a launch in a workspace of 16 bytes a
+ * aligned to 16 bytes run several sweeps a launch in a workspace of 28 bytes a
  * cell that the library keeps for the stream, at most 256 MiB on a GPU for all
  * streams; past that, otherwise, and while the stream is being captured, each
  * sweep is a launch.  Same results either way; pfs_compute_pressure likewise. */

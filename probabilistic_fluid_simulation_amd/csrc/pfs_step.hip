@@ -292,8 +292,10 @@ int fused_step(const StepArgs &s, float *ws, hipStream_t stream, hipEvent_t *ev,
 // `last` and the one before it in `before` (the two fields, in the order the
 // reference's pointer swaps leave them).  Other channels keep their values.
 // Workspace (floats, N = w*h): the iterates of u and v in [0, 2N) and [2N, 4N),
-// or the divergence in [0, N) and the iterates of p in [N, 2N) and [2N, 3N).
-size_t op_workspace_bytes(int w, int h) { return 4 * (size_t)w * h * sizeof(float); }
+// the divergence in [4N, 5N) and the iterates of p in [5N, 6N) and [6N, 7N).  (Both
+// operators in the same 4N: 640x480 at 30 sweeps, all operators in turn 65.7 us
+// against 64.1, each one's planes then lying in the XCDs' L2s for the other.)
+size_t op_workspace_bytes(int w, int h) { return 7 * (size_t)w * h * sizeof(float); }
 
 int diffuse_op(const float *a, float *last, float *before, int w, int h, float dt, float visc,
                int iters, float *ws, hipStream_t stream) {
@@ -320,9 +322,9 @@ int diffuse_op(const float *a, float *last, float *before, int w, int h, float d
 int pressure_op(float *a, float *last, float *before, int w, int h, float dt, int iters, float *ws,
                 hipStream_t stream) {
     PressureArgs p = pressure_args(a, a, nullptr, nullptr, w, h, dt, ws);
-    float *plane[2] = {ws + (size_t)w * h, ws + 2 * (size_t)w * h};
+    float *plane[2] = {ws + 5 * (size_t)w * h, ws + 6 * (size_t)w * h};
     p.gamma = pressure_gamma(dt);
-    p.bpl = p.bdst = ws;
+    p.bpl = p.bdst = ws + 4 * (size_t)w * h;
     p.field[0] = last;
     p.field[1] = before;
     const OpPlan plan = op_plan(iters, w, h);
