@@ -210,7 +210,9 @@ size_t fused_workspace_bytes(int w, int h) {
 // 128^2 8: 8.7, 12: 9.3, 16: 10.2; 320x240 16 (300 tiles): 13.8, 20: 11.5, 24:
 // 12.4; 360^2 24: 13.1, 32: 15.2.  The pressure alone: 611x397 32 (260 tiles) 12.8,
 // 36: 8.7; 800x600 48: 12.2, 56: 13.6, 64: 15.2; past a tile a CU at 64, two at 48
-// or 56: 1100x1024 48: 19.2, 56: 21.4, 64: 24.5, 1200x1024 56: 21.8, 64: 25.0.
+// or 56: 1100x1024 48: 19.2, 56: 21.4, 64: 24.5, 1200x1024 56: 21.8, 64: 25.0.  Where
+// 64 just fits, pairs of 48 depend on the sweeps: a 1024^2 step 36.6 (48) against
+// 37.9 (64) at 8, 55.2 against 56.6 at 16, but 33.0 against 31.4 at 4: left at 64.
 int tile_side(int tile, int w, int h) {
     const int cus = device_cus();
     auto smallest = [&](std::initializer_list<int> sides) {
