@@ -1033,7 +1033,8 @@ __device__ __forceinline__ void for_listed(const PbfArgs &b, const Staged *st, i
 // loops do not branch; adding +-0 leaves the sums unchanged).
 // Root and division correctly rounded without their range handling: r and an
 // approximation of 1/r from one reciprocal root by Goldschmidt's iteration and
-// a last residual step (exact for every d2 in [2^-100, 2^100), all 1.7e9 tried),
+// a last residual step (exact for every d2 in [2^-100, 2^100), all 1.7e9 tried once
+// on the GPU; the tests hold samples and the significands excluded below),
 // the division by Markstein's steps as in div_fast.  Their theorem needs 1/r
 // correctly rounded, which it is but for 5 significands of d2 in two binades,
 // all x tried for those: only r = 2 - 2^-23 (times a power of two) divides some
