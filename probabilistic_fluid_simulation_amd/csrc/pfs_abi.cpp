@@ -117,13 +117,16 @@ bool get_op_workspace(size_t bytes, hipStream_t s, Lease *out) {
     Workspace &w = find(g_op_ws, dev, s);
     std::unique_lock<std::mutex> held(w.m);
     if (w.bytes < bytes) {
-        std::lock_guard<std::mutex> lock(g_ws_mutex);
-        size_t &total = g_op_held[dev];
-        if (total - w.bytes + bytes > kOpBytes) return false;
-        total -= w.bytes;
-        const int rc = grow(w, bytes, s);
-        total += w.bytes;
+        {
+            std::lock_guard<std::mutex> lock(g_ws_mutex);
+            size_t &total = g_op_held[dev];
+            if (total - w.bytes + bytes > kOpBytes) return false;
+            total += bytes - w.bytes;
+        }
+        const int rc = grow(w, bytes, s);  // may wait for the stream: the maps stay open
         if (rc != PFS_OK) {
+            std::lock_guard<std::mutex> lock(g_ws_mutex);
+            g_op_held[dev] -= bytes - w.bytes;
             clear_error();
             return false;
         }
